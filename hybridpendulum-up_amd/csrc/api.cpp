@@ -44,7 +44,7 @@ template <class T> std::vector<T> cast_vec(const std::vector<double>& v) { retur
 
 // Transform tables from a Wigner-d table d (M,M,B,2B) and weights w (2B).
 template <class T> struct XformTables {
-    DevBuf Wf, Wi, twB, twMB, dftN, idftN, twNf, twNi, bsF, bsI, hrows;
+    DevBuf Wf, Wi, twB, agF, agI, dftN, idftN, twNf, twNi, bsF, bsI, hrows;
     XformDev<T> view{};
     void build(int B, int dim, int N, const double* d, const double* w) {
         const int M = 2 * B - 1, n2 = 2 * B;
@@ -68,17 +68,27 @@ template <class T> struct XformTables {
         std::vector<T> tb(2 * n2), dn, idn, tf, ti;
         for (int t = 0; t < n2; t++) { tb[2 * t] = (T)std::cos(kPi * t / B); tb[2 * t + 1] = (T)std::sin(kPi * t / B); }
         twB = upload(tb);
-        if (n2 <= 32) {  // [r][t] then [t][r]: frequency r - (B-1), grid angle pi t / B, zero padded to 32 x 32
-            std::vector<T> tm(2 * 2 * 32 * 32, T(0));
-            for (int r = 0; r < M; r++)
-                for (int t = 0; t < n2; t++) {
-                    const int e = (((r - (B - 1)) * t) % n2 + n2) % n2;
-                    for (int c = 0; c < 2; c++) {
-                        tm[2 * (r * 32 + t) + c] = tb[2 * e + c];
-                        tm[2 * (32 * 32 + t * 32 + r) + c] = tb[2 * e + c];
+        if (B <= 32) {  // MFMA (alpha, gamma) tables (see XformDev::agF)
+            const int sz = kAgTabR * kAgTabK;
+            std::vector<T> af(2 * sz, T(0)), ai(2 * sz, T(0));
+            for (int r = 0; r <= B; r++)
+                for (int k = 0; k <= B; k++) {
+                    // exactly reduced: cos and sin vanish exactly where they should
+                    const int e = (r * k) % n2;
+                    const double c = e % B == 0 ? (e ? -1.0 : 1.0) : 2 * e % n2 == B ? 0.0 : std::cos(kPi * e / B);
+                    const double s = e % B == 0 ? 0.0 : std::sin(kPi * e / B);
+                    if (r < B) {
+                        const double h = k == 0 || k == B ? 0.5 : 1.0;
+                        af[r * kAgTabK + k] = (T)(h * c);
+                        af[sz + r * kAgTabK + k] = (T)(h * s);
+                    }
+                    if (k < B) {
+                        ai[r * kAgTabK + k] = (T)c;
+                        ai[sz + r * kAgTabK + k] = (T)s;
                     }
                 }
-            twMB = upload(tm);
+            agF = upload(af);
+            agI = upload(ai);
         }
         const int Nn = std::max(N, 1);
         dn.resize(2 * (size_t)Nn * Nn); idn.resize(2 * (size_t)Nn * Nn); tf.resize(2 * Nn); ti.resize(2 * Nn);
@@ -124,7 +134,8 @@ template <class T> struct XformTables {
         view.B = B; view.dim = dim; view.N = Nn;
         view.nx = ipow64(Nn, dim); view.nrc = nrc_of(B);
         view.Wf = Wf.as<T>(); view.Wi = Wi.as<T>(); view.twB = twB.as<cT<T>>();
-        view.twMB = n2 <= 32 ? twMB.as<cT<T>>() : nullptr;
+        view.agF = B <= 32 ? agF.as<T>() : nullptr;
+        view.agI = B <= 32 ? agI.as<T>() : nullptr;
         view.dftN = dftN.as<cT<T>>(); view.idftN = idftN.as<cT<T>>();
         view.twNf = twNf.as<cT<T>>(); view.twNi = twNi.as<cT<T>>();
         view.bsF = Nn <= 32 ? bsF.as<cT<T>>() : nullptr;

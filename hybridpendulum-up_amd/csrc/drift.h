@@ -116,6 +116,8 @@ void launch_drift_slab(const DriftDev<T>& D, const void* Fin, const void* Z3, co
 
 // ---------------------------------------------------------- transforms --
 
+constexpr int kAgTabR = 48, kAgTabK = 36;  // rows and row stride of the MFMA (alpha, gamma) tables
+
 template <class T> struct XformDev {
     int B, dim, N;
     int64_t nx, nrc;
@@ -123,8 +125,12 @@ template <class T> struct XformDev {
     const T* Wi;        // inverse beta weights  [mn][j][l] = (2l+1) d^l_mn(beta_j), rows of wis
     int wfs, wis;       // row strides (zero-padded to whole reduction groups)
     const cT<T>* twB;   // e^{i pi t / B}, t in [0, 2B)
-    const cT<T>* twMB;  // [32][32] e^{i pi (r - (B-1)) t / B} for r < 2B-1, t < 2B, zero elsewhere, then its
-                        // transpose [t][r] (B <= 16)
+    // DFT tables of the MFMA (alpha, gamma) stages (B <= 32), each cos then sin,
+    // kAgTabR rows of kAgTabK, zero padded: forward cos/sin (pi r k / B), rows
+    // r < B (frequency), k <= B (angle, entries k = 0 and B halved); inverse
+    // rows r <= B (angle), k < B (frequency)
+    const T* agF;
+    const T* agI;
     const cT<T>* dftN;  // forward DFT matrix N x N (row-major [k][a]) e^{-2 pi i k a/N}
     const cT<T>* idftN; // inverse DFT matrix (1/N scaled) e^{+2 pi i k a/N}/N
     const cT<T>* twNf;  // e^{-2 pi i t/N}, t in [0, N)

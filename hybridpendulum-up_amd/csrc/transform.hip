@@ -569,26 +569,6 @@ __global__ void k_compact_to_full(int B, int64_t nx, const cT<T>* __restrict__ c
     }
 }
 
-// ------------------------------------- (alpha, gamma) stages for B <= 16 --
-//
-// Work items hold one row of the stage's input in registers and sweep a
-// frequency x angle twiddle table E[r][t] = e^{i pi (r - lmax) t / B}, zero
-// padded to 32 x 32, so every loop runs a fixed 32 (or 8) steps without
-// guards.  The table row and column of each step depend only on loop
-// counters and on the wave's part of the block, so the table is read through
-// the scalar cache (uniform addresses) instead of LDS.  A stage whose work
-// items fill only part of the block splits its output range into chunks of
-// 8 over wave-aligned parts.  Blocks are numbered so that consecutive omega
-// chunks of one beta_j land on the same XCD (the hardware deals blocks to the
-// 8 XCDs round-robin): a cache line shared by neighbouring chunks is then
-// fetched into one L2 only.
-
-constexpr int kAgMax = 32;  // 2B limit of the register-row kernels
-
-// table in the constant address space: uniform indices become scalar loads
-template <class T> using cTab = __attribute__((address_space(4))) const T*;
-template <class T> __device__ __forceinline__ cT<T> etw(cTab<T> e, int i) { return cmk<T>(e[2 * i], e[2 * i + 1]); }
-
 // block b of nb -> work index, a bijection with XCD k = b % 8 owning a
 // contiguous range of work indices (the last nb % 8 blocks keep their index)
 __device__ __forceinline__ int xcd_major(int b, int nb) {
@@ -603,9 +583,8 @@ __device__ __forceinline__ int xcd_major(int b, int nb) {
 // blocks an XCD runs side by side share the G lines of neighbouring x-tiles
 // and also the f lines that straddle the slices j and j + 1 of a (gamma, x) row
 // (with j slowest, every such line was fetched twice: 1.47x the f bytes).
-template <class T, int XC>
-__device__ __forceinline__ void ag_block(int nxc, int n2, int& j, int64_t& x0) {
-    constexpr int XT = XC * (int)sizeof(cT<T>) >= 128 ? 1 : 128 / (XC * (int)sizeof(cT<T>));
+template <class T> __device__ __forceinline__ void ag_block(int XC, int nxc, int n2, int& j, int64_t& x0) {
+    const int XT = XC * (int)sizeof(cT<T>) >= 128 ? 1 : 128 / (XC * (int)sizeof(cT<T>));
     const int w = xcd_major(blockIdx.x, gridDim.x);
     const int full = nxc / XT, head = full * XT * n2;
     int xt;
@@ -621,136 +600,370 @@ __device__ __forceinline__ void ag_block(int nxc, int n2, int& j, int64_t& x0) {
     x0 = (int64_t)xt * XC;
 }
 
-// tasks of a stage -> parts of the block: <= 64 -> 4, <= 128 -> 2, else 1
-__device__ __forceinline__ int stage_parts(int T) { return T <= 64 ? 4 : (T <= 128 ? 2 : 1); }
+// ------------------------------ (alpha, gamma) stages on MFMA, B <= 32 --
+//
+// Both angular DFTs of a (beta_j, omega) tile as real matrix products on the
+// even and odd parts of the data.  With f folded over a <-> -a and g <-> -g
+// into four parity planes (ee, oe, eo, oo: even/odd in alpha, then in gamma),
+// the forward 2-D DFT is, for m, n >= 0,
+//   CC = cos ee cos',  SC = sin oe cos',  CS = cos eo sin',  SS = sin oo sin'
+// (cos/sin (pi m a / B) from the left over a, the same over g from the right),
+//   G[m][+-n] = (CC -+ SS) + i (SC +- CS),
+// and the inverse is its transpose.  The folding quarters the products of the
+// direct DFT: 4 B flops per grid point, 80 at B = 20, where the FP32 matrix
+// cores need a third of the time the tile's traffic takes, so the kernels are
+// bound by their f and G (H) traffic.  A block of four waves takes one beta_j
+// and XC omega points.  A wave takes 16 columns (g, x) or (m, x) at a time, x
+// fastest, and all four planes of them, so that the fold is formed once, in
+// registers, on the way to the operands, and a column's results replace its
+// own inputs: each block holds one f tile in LDS and nothing else.
+//
+// Strides (elements) rs between rows and sx between omega points: with
+// sx = 32 / XC mod 32 (FP64: 16 / XC mod 16) and rs = 2 mod 4 (FP64: odd)
+// the operand reads of a half (FP64: quarter) wave fall in distinct banks.
+//
+// Measured at B = 20, 18^3 omega points, FP32: forward 6.38 -> 1.25 ms, inverse
+// 7.34 -> 1.18 ms against the direct DFTs in LDS these replace there; at
+// B = 10, 16^3, FP64 (direct DFTs in registers before): forward 0.378 -> 0.136,
+// inverse 0.530 -> 0.137 ms.
 
-template <class T, int XC>
-__global__ __launch_bounds__(256) void k_fwd_ag_r(XformDev<T> X, const T* __restrict__ f, const T* __restrict__ wR,
-                                                  int wstride, cT<T>* __restrict__ G, int nxc) {
-    extern __shared__ char smem_raw[];
-    const int B = X.B, n2 = 2 * B, lmax = B - 1, M = 2 * B - 1;
-    const int rp = n2 + 1;                                   // padded row of sf
-    T* sf = reinterpret_cast<T*>(smem_raw);                  // [xl][g][a]  XC*n2*rp
-    cT<T>* sH = reinterpret_cast<cT<T>*>(smem_raw);          // [m>=0][g][xl], aliases sf
-    const cTab<T> E = (cTab<T>)(const T*)X.twMB;
+// i / d for 0 <= i < 2^17 and 1 <= d <= 64, inv = 1.0f / d: (i + 0.5) / d is at
+// least 0.5 / d away from an integer, far beyond the rounding of two FP32
+// operations.  Three instructions instead of an integer division's twenty:
+// the index arithmetic of the tiles' staging was half of the kernels' time.
+__device__ __forceinline__ int div_small(int i, float inv) { return (int)(((float)i + 0.5f) * inv); }
+
+// DFT tables of lane (lr, lq): row 16 t + lr, K index 4 s + lq (zero padded)
+template <class T, int MT, int KS> struct AgTab {
+    T c[MT][KS], s[MT][KS];
+    __device__ __forceinline__ void load(const T* tab, int lr, int lq) {
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+#pragma unroll
+            for (int k = 0; k < KS; k++) {
+                const int i = (16 * t + lr) * kAgTabK + 4 * k + lq;
+                c[t][k] = tab[i];
+                s[t][k] = tab[kAgTabR * kAgTabK + i];
+            }
+    }
+};
+
+template <class T, int MT, int KS>
+__global__ __launch_bounds__(256) void k_fwd_ag_mfma(XformDev<T> X, const T* __restrict__ f, const T* __restrict__ wR,
+                                                     int wstride, cT<T>* __restrict__ G, int lx, int nxc, int rs,
+                                                     int sx, int vec) {
+    using MF = Mfma<T>;
+    using acc_t = typename MF::acc;
+    extern __shared__ __align__(16) char smem_raw[];
+    T* sf = reinterpret_cast<T*>(smem_raw);  // [xl][g][a], strides sx, rs
+    const int B = X.B, n2 = 2 * B, lmax = B - 1, M = 2 * B - 1, XC = 1 << lx;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lq = lane >> 4;
     int j;
     int64_t x0;
-    ag_block<T, XC>(nxc, n2, j, x0);
+    ag_block<T>(XC, nxc, n2, j, x0);
     const int64_t nx = X.nx;
-    const int tid = threadIdx.x;
-    const int64_t n2c = (int64_t)n2 * n2 * n2;
-    for (int i = tid; i < XC * n2 * n2; i += 256) {
-        const int xl = i / (n2 * n2), g = (i / n2) % n2, a = i % n2;
-        const int64_t x = x0 + xl;
-        const int64_t iR = a + (int64_t)n2 * (j + (int64_t)n2 * g);
-        T v = x < nx ? f[iR + n2c * x] : T(0);
-        if (wR) v *= wR[iR * wstride];  // transform of the product f(R, x) w(R)
-        sf[(xl * n2 + g) * rp + a] = v;
-    }
-    __syncthreads();
-    // alpha DFT, m >= 0: H[m][g] = sum_a f[a] e^{+i m alpha_a}; item (g, xl)
+    const int xn = (int)(nx - x0 < XC ? nx - x0 : XC);  // omega points of the block
+    const float invB = 1.0f / (float)B;
+    // f rows (x, g): n2 consecutive values each; pieces of VE values (one at a
+    // time if f is not aligned to a piece), loaded in batches
     {
-        const int TA = n2 * XC, SA = stage_parts(TA), PA = 256 / SA;
-        const int part = __builtin_amdgcn_readfirstlane(tid / PA), task = tid % PA;
-        const bool act = task < TA;
-        const int g = task / XC, xl = task % XC;
-        T row[kAgMax];
+        typedef T VecT __attribute__((ext_vector_type(2)));
+        const T* fb = f + (int64_t)n2 * j + (int64_t)n2 * n2 * n2 * x0;
+        const int tot = xn * n2 * B;  // pairs
+        constexpr int NL = 8;
+        for (int i0 = tid; i0 < tot; i0 += 256 * NL) {
+            VecT v[NL];
+            unsigned src[NL];
+            int dst[NL], iR[NL];
 #pragma unroll
-        for (int a = 0; a < kAgMax; a++) row[a] = (act && a < n2) ? sf[(xl * n2 + g) * rp + a] : T(0);
-        __syncthreads();  // sH overwrites sf
-        for (int m = part; m < B; m += SA) {
-            const cTab<T> e = E + 2 * (m + lmax) * kAgMax;
-            cT<T> acc = czero<T>();
-#pragma unroll
-            for (int a = 0; a < kAgMax; a++) {
-                const cT<T> tw = etw<T>(e, a);
-                acc.x = fma(row[a], tw.x, acc.x);
-                acc.y = fma(row[a], tw.y, acc.y);
+            for (int u = 0; u < NL; u++) {
+                const int i = i0 + 256 * u < tot ? i0 + 256 * u : i0;
+                const int row = div_small(i, invB), p = i - row * B, xl = div_small(row, 0.5f * invB), g = row - xl * n2;
+                iR[u] = 2 * p + n2 * n2 * g;
+                src[u] = (unsigned)(iR[u] + n2 * n2 * n2 * xl);
+                dst[u] = xl * sx + g * rs + 2 * p;
             }
-            if (act) sH[(m * n2 + g) * XC + xl] = acc;
+            if (vec) {
+#pragma unroll
+                for (int u = 0; u < NL; u++) v[u] = *reinterpret_cast<const VecT*>(fb + src[u]);
+            } else {
+#pragma unroll
+                for (int u = 0; u < NL; u++) {
+                    v[u].x = fb[src[u]];
+                    v[u].y = fb[src[u] + 1];
+                }
+            }
+            if (wR) {  // transform of the product f(R, x) w(R)
+                const T* wb = wR + (int64_t)n2 * j * wstride;
+#pragma unroll
+                for (int u = 0; u < NL; u++) {
+                    v[u].x *= wb[(int64_t)iR[u] * wstride];
+                    v[u].y *= wb[(int64_t)(iR[u] + 1) * wstride];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < NL; u++)
+                if (i0 + 256 * u < tot) {
+                    sf[dst[u]] = v[u].x;
+                    sf[dst[u] + 1] = v[u].y;
+                }
+        }
+    }
+    AgTab<T, MT, KS> tab;
+    tab.load(X.agF, lr, lq);
+    __syncthreads();
+    // alpha: column (g, x), g = 0..B, from its rows g and -g (equal at g = 0 and
+    // B, whose doubled fold the tables' halved K entries 0 and B undo); row g
+    // becomes [cos ee | sin oe](m), row -g [cos eo | sin oo](m)
+    const int ncA = (B + 1) << lx;
+    for (int c0 = 16 * w; c0 < ncA; c0 += 64) {
+        const int col = c0 + lr < ncA ? c0 + lr : ncA - 1;
+        const int xl = col & (XC - 1), g = col >> lx;
+        T* r0 = sf + (xl < xn ? xl : xn - 1) * sx + g * rs;
+        T* r1 = sf + (xl < xn ? xl : xn - 1) * sx + (g ? n2 - g : 0) * rs;
+        acc_t ee[MT], oe[MT], eo[MT], oo[MT];
+#pragma unroll
+        for (int t = 0; t < MT; t++) ee[t] = oe[t] = eo[t] = oo[t] = MF::zero();
+#pragma unroll
+        for (int k = 0; k < KS; k++) {
+            const int a = 4 * k + lq < B ? 4 * k + lq : B, an = a ? n2 - a : 0;
+            const T p = r0[a], q = r0[an], u = r1[a], v = r1[an];
+            const T e0 = p + q, o0 = p - q, e1 = u + v, o1 = u - v;
+            const T fee = e0 + e1, feo = e0 - e1, foe = o0 + o1, foo = o0 - o1;
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                ee[t] = MF::fma(tab.c[t][k], fee, ee[t]);
+                eo[t] = MF::fma(tab.c[t][k], feo, eo[t]);
+                oe[t] = MF::fma(tab.s[t][k], foe, oe[t]);
+                oo[t] = MF::fma(tab.s[t][k], foo, oo[t]);
+            }
+        }
+        if (c0 + lr < ncA && xl < xn) {
+            const bool two = g != 0 && g != B;
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int m = 16 * t + MF::orow(lq, v);
+                    if (m < B) {
+                        r0[m] = ee[t][v];
+                        r0[B + m] = oe[t][v];
+                        if (two) {
+                            r1[m] = eo[t][v];
+                            r1[B + m] = oo[t][v];
+                        }
+                    }
+                }
         }
     }
     __syncthreads();
-    // gamma DFT: G[m][n] = sum_g H[m][g] e^{+i n gamma_g}, G[-m][-n] = conj; item (m, xl)
-    {
-        const int TB = B * XC, SB = stage_parts(TB), PB = 256 / SB;
-        const int part = __builtin_amdgcn_readfirstlane(tid / PB), task = tid % PB;
-        const bool act = task < TB;
-        const int m = task / XC, xl = task % XC;
-        const int64_t x = x0 + xl;
-        cT<T> h[kAgMax];
+    // gamma: column (m, x) over g = 0..B (the odd planes' rows g = 0 and B meet
+    // zero table entries)
+    const int ncB = B << lx;
+    for (int c0 = 16 * w; c0 < ncB; c0 += 64) {
+        const int col = c0 + lr < ncB ? c0 + lr : ncB - 1;
+        const int xl = col & (XC - 1), m = col >> lx;
+        const T* cb = sf + (xl < xn ? xl : xn - 1) * sx + m;
+        acc_t cc[MT], sc[MT], cs[MT], ss[MT];
 #pragma unroll
-        for (int g = 0; g < kAgMax; g++) h[g] = (act && g < n2) ? sH[(m * n2 + g) * XC + xl] : czero<T>();
-        const bool st = act && x < nx;
-        cT<T>* Gx = G + g_off(B, 0, j, min<int64_t>(x, nx - 1));
-        for (int ni = part; ni < M; ni += SB) {
-            const cTab<T> e = E + 2 * ni * kAgMax;
-            cT<T> acc = czero<T>();
+        for (int t = 0; t < MT; t++) cc[t] = sc[t] = cs[t] = ss[t] = MF::zero();
 #pragma unroll
-            for (int g = 0; g < kAgMax; g++) cfma<T>(acc, h[g], etw<T>(e, g));
-            if (st) put_g_half<T>(Gx, B, m, ni, acc);
+        for (int k = 0; k < KS; k++) {
+            const int g = 4 * k + lq < B ? 4 * k + lq : B;
+            const T* p = cb + g * rs;
+            const T* q = cb + (g ? n2 - g : 0) * rs;
+            const T er = p[0], ei = p[B], hr = q[0], hi = q[B];
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                cc[t] = MF::fma(tab.c[t][k], er, cc[t]);
+                sc[t] = MF::fma(tab.c[t][k], ei, sc[t]);
+                cs[t] = MF::fma(tab.s[t][k], hr, cs[t]);
+                ss[t] = MF::fma(tab.s[t][k], hi, ss[t]);
+            }
+        }
+        if (c0 + lr < ncB && xl < xn) {
+            cT<T>* Gx = G + g_off(B, 0, j, x0 + xl);
+            const int64_t gs = (int64_t)n2 * kGX;
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int n = 16 * t + MF::orow(lq, v);
+                    if (n < B) {
+                        const int64_t row = (int64_t)M * (n + lmax) + lmax;
+                        Gx[(row + m) * gs] = cmk<T>(cc[t][v] - ss[t][v], sc[t][v] + cs[t][v]);
+                        // conj G[m][-n] at (-m, n)
+                        if (n > 0 && m > 0) Gx[(row - m) * gs] = cmk<T>(cc[t][v] + ss[t][v], cs[t][v] - sc[t][v]);
+                    }
+                }
         }
     }
 }
 
-template <class T, int XC>
-__global__ __launch_bounds__(256) void k_inv_ag_r(XformDev<T> X, const cT<T>* __restrict__ G, T* __restrict__ f,
-                                                  int nxc) {
-    extern __shared__ char smem_raw[];
-    const int B = X.B, n2 = 2 * B, M = 2 * B - 1;
-    cT<T>* sH = reinterpret_cast<cT<T>*>(smem_raw);  // [m][g][xl]
-    const cTab<T> ET = (cTab<T>)(const T*)X.twMB + 2 * kAgMax * kAgMax;  // [t][r]
+// Inverse: f = sum over m, n >= 0 of the four planes
+//   ee cos cos' + oe sin cos' + eo cos sin' + oo sin sin'
+// with, from z+- = H[+-m][n], P = z+ + z-, Q = z+ - z-: ee = 2 Re P, oe = 2 Im Q,
+// eo = 2 Im P, oo = -2 Re Q (halved on the axes, where z- is conj z+ at n = 0
+// and z+ at m = 0).  LDS slot (x, m) holds the planes over n, then (in place,
+// column (m, x)) over g = 0..B -- the odd ones over 0 < g < B -- and then (in
+// place, column (g, x)) f(+-a, +-g).
+template <class T, int MT, int KS>
+__global__ __launch_bounds__(256) void k_inv_ag_mfma(XformDev<T> X, const cT<T>* __restrict__ H, T* __restrict__ f,
+                                                     int lx, int nxc, int rs, int sx, int vec) {
+    using MF = Mfma<T>;
+    using acc_t = typename MF::acc;
+    extern __shared__ __align__(16) char smem_raw[];
+    T* sf = reinterpret_cast<T*>(smem_raw);
+    const int B = X.B, n2 = 2 * B, M = 2 * B - 1, XC = 1 << lx;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lq = lane >> 4;
     int j;
     int64_t x0;
-    ag_block<T, XC>(nxc, n2, j, x0);
+    ag_block<T>(XC, nxc, n2, j, x0);
     const int64_t nx = X.nx;
-    const int tid = threadIdx.x;
-    // H[m][g] = sum_n G[m][n] e^{-i n gamma_g}; item (m, xl) holds its G row
+    const int xn = (int)(nx - x0 < XC ? nx - x0 : XC);
+    const float invB = 1.0f / (float)B;
+    // planes from H: tasks (x of a pair, m, n, pair), the lanes along a line of H
     {
-        const int T1 = M * XC, S1 = stage_parts(T1), P1 = 256 / S1;
-        const int part = __builtin_amdgcn_readfirstlane(tid / P1), task = tid % P1;
-        const bool act = task < T1;
-        const int mi = task / XC, xl = task % XC;
-        const int64_t x = x0 + xl;
-        const bool ld = act && x < nx;
-        // clamped, branch-free loads; invalid entries are zeroed after the load
-        const cT<T>* Hx = G + h_base(B, j, min<int64_t>(x, nx - 1));
-        cT<T> gr[kAgMax];
+        const int lp = lx ? 1 : 0, tot = (B * B) << lx;
+        constexpr int NL = 4;
+        for (int i0 = tid; i0 < tot; i0 += 256 * NL) {
+            cT<T> zp[NL], zm[NL];
+            int at[NL];
+            T fac[NL];
+            bool ax[NL];
 #pragma unroll
-        for (int ni = 0; ni < kAgMax; ni++) {
-            const cT<T> v = get_h<T>(Hx, B, min(mi, M - 1), min(ni, M - 1));
-            gr[ni] = (ld && ni < M) ? v : czero<T>();
+            for (int u = 0; u < NL; u++) {
+                const int i = i0 + 256 * u < tot ? i0 + 256 * u : i0;
+                const int q = i >> lp, qn = div_small(q, invB), m = q - qn * B, qx = div_small(qn, invB), n = qn - qx * B;
+                const int xl = (i & lp) + 2 * qx;
+                at[u] = xl < xn ? xl * sx + m * rs + n : -1;
+                fac[u] = n > 0 && m > 0 ? T(2) : (n == 0 && m == 0 ? T(0.5) : T(1));
+                ax[u] = n > 0;
+                const cT<T>* Hx = H + h_base(B, j, x0 + (xl < xn ? xl : xn - 1));
+                zp[u] = Hx[2 * (m + M * n)];
+                zm[u] = Hx[2 * (n > 0 ? M * n - m : m)];
+            }
+#pragma unroll
+            for (int u = 0; u < NL; u++) {
+                if (i0 + 256 * u >= tot || at[u] < 0) continue;
+                const cT<T> a = zp[u], b = ax[u] ? zm[u] : cconj<T>(zm[u]);
+                T* d = sf + at[u];
+                d[0] = fac[u] * (a.x + b.x);
+                d[B] = fac[u] * (a.y - b.y);
+                d[2 * B] = fac[u] * (a.y + b.y);
+                d[3 * B] = fac[u] * (b.x - a.x);
+            }
         }
-        for (int g = part; g < n2; g += S1) {
-            const cTab<T> e = ET + 2 * g * kAgMax;
-            cT<T> acc = czero<T>();
+    }
+    AgTab<T, MT, KS> tab;
+    tab.load(X.agI, lr, lq);
+    __syncthreads();
+    const int ncA = B << lx;
+    for (int c0 = 16 * w; c0 < ncA; c0 += 64) {  // gamma: column (m, x), K = n
+        const int col = c0 + lr < ncA ? c0 + lr : ncA - 1;
+        const int xl = col & (XC - 1), m = col >> lx;
+        T* cb = sf + (xl < xn ? xl : xn - 1) * sx + m * rs;
+        acc_t ee[MT], oe[MT], eo[MT], oo[MT];
 #pragma unroll
-            for (int ni = 0; ni < kAgMax; ni++) cfma<T>(acc, gr[ni], cconj<T>(etw<T>(e, ni)));
-            if (act) sH[(mi * n2 + g) * XC + xl] = acc;
+        for (int t = 0; t < MT; t++) ee[t] = oe[t] = eo[t] = oo[t] = MF::zero();
+#pragma unroll
+        for (int k = 0; k < KS; k++) {
+            const int n = 4 * k + lq < B ? 4 * k + lq : B - 1;
+            const T a = cb[n], b = cb[B + n], c = cb[2 * B + n], d = cb[3 * B + n];
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                ee[t] = MF::fma(tab.c[t][k], a, ee[t]);
+                oe[t] = MF::fma(tab.c[t][k], b, oe[t]);
+                eo[t] = MF::fma(tab.s[t][k], c, eo[t]);
+                oo[t] = MF::fma(tab.s[t][k], d, oo[t]);
+            }
+        }
+        if (c0 + lr < ncA && xl < xn) {
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int g = 16 * t + MF::orow(lq, v);
+                    if (g <= B) {
+                        cb[g] = ee[t][v];
+                        cb[B + 1 + g] = oe[t][v];
+                        if (g > 0 && g < B) {
+                            cb[2 * B + 1 + g] = eo[t][v];
+                            cb[3 * B + g] = oo[t][v];
+                        }
+                    }
+                }
         }
     }
     __syncthreads();
-    // f[a][g] = Re sum_m H[m][g] e^{-i m alpha_a}; item (g, xl) holds its H column
-    {
-        const int T2 = n2 * XC, S2 = stage_parts(T2), P2 = 256 / S2;
-        const int part = __builtin_amdgcn_readfirstlane(tid / P2), task = tid % P2;
-        const bool act = task < T2;
-        const int g = task / XC, xl = task % XC;
-        const int64_t x = x0 + xl;
-        const bool st = act && x < nx;
-        cT<T> hr[kAgMax];
+    const int ncB = (B + 1) << lx;
+    for (int c0 = 16 * w; c0 < ncB; c0 += 64) {  // alpha: column (g, x), K = m
+        const int col = c0 + lr < ncB ? c0 + lr : ncB - 1;
+        const int xl = col & (XC - 1), g = col >> lx;
+        T* cb = sf + (xl < xn ? xl : xn - 1) * sx + g;
+        const bool two = g > 0 && g < B;  // the odd planes vanish at g = 0 and B
+        acc_t ee[MT], oe[MT], eo[MT], oo[MT];
 #pragma unroll
-        for (int mi = 0; mi < kAgMax; mi++) hr[mi] = (act && mi < M) ? sH[(mi * n2 + g) * XC + xl] : czero<T>();
-        T* fo = f + (int64_t)n2 * (j + (int64_t)n2 * (g + (int64_t)n2 * min<int64_t>(x, nx - 1)));
-        for (int a = part; a < n2; a += S2) {
-            const cTab<T> e = ET + 2 * a * kAgMax;
-            T acc = T(0);
+        for (int t = 0; t < MT; t++) ee[t] = oe[t] = eo[t] = oo[t] = MF::zero();
 #pragma unroll
-            for (int mi = 0; mi < kAgMax; mi++) {
-                const cT<T> tw = etw<T>(e, mi);  // Re(h conj(tw))
-                acc = fma(hr[mi].x, tw.x, fma(hr[mi].y, tw.y, acc));
+        for (int k = 0; k < KS; k++) {
+            const T* p = cb + (4 * k + lq < B ? 4 * k + lq : B - 1) * rs;
+            const T a = p[0], b = p[B + 1], c = two ? p[2 * B + 1] : T(0), d = two ? p[3 * B] : T(0);
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                ee[t] = MF::fma(tab.c[t][k], a, ee[t]);
+                oe[t] = MF::fma(tab.s[t][k], b, oe[t]);
+                eo[t] = MF::fma(tab.c[t][k], c, eo[t]);
+                oo[t] = MF::fma(tab.s[t][k], d, oo[t]);
             }
-            if (st) fo[a] = acc;
+        }
+        if (c0 + lr < ncB && xl < xn) {
+            // f(a, g) at slot a mod B, plane ee (a < B) or oe; f(a, -g) in eo or oo
+            auto put = [&](int a, T p, T q) {
+                T* d = cb + (a < B ? a : a - B) * rs;
+                d[a < B ? 0 : B + 1] = p;
+                if (two) d[a < B ? 2 * B + 1 : 3 * B] = q;
+            };
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int a = 16 * t + MF::orow(lq, v);
+                    if (a <= B) {
+                        const T e0 = ee[t][v] + eo[t][v], e1 = ee[t][v] - eo[t][v];
+                        const T o0 = oe[t][v] + oo[t][v], o1 = oe[t][v] - oo[t][v];
+                        put(a, e0 + o0, e1 + o1);
+                        if (a > 0 && a < B) put(n2 - a, e0 - o0, e1 - o1);
+                    }
+                }
+        }
+    }
+    __syncthreads();
+    // f rows (x, g): consecutive threads take consecutive pairs of a row
+    {
+        typedef T VecT __attribute__((ext_vector_type(2)));
+        T* fb = f + (int64_t)n2 * j + (int64_t)n2 * n2 * n2 * x0;
+        const int tot = xn * n2 * B;
+        for (int i = tid; i < tot; i += 256) {
+            const int row = div_small(i, invB), p = i - row * B, xl = div_small(row, 0.5f * invB), g = row - xl * n2;
+            const int gg = g <= B ? g : n2 - g;
+            const T* s = sf + xl * sx + gg;
+            T v[2];
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+                const int a = 2 * p + e;
+                v[e] = s[(a < B ? a : a - B) * rs + (g <= B ? (a < B ? 0 : B + 1) : (a < B ? 2 * B + 1 : 3 * B))];
+            }
+            T* dst = fb + (2 * p + n2 * n2 * g + n2 * n2 * n2 * xl);
+            if (vec) {
+                VecT q;
+                q.x = v[0];
+                q.y = v[1];
+                *reinterpret_cast<VecT*>(dst) = q;
+            } else {
+                dst[0] = v[0];
+                dst[1] = v[1];
+            }
         }
     }
 }
@@ -933,7 +1146,7 @@ __global__ __launch_bounds__(NT) void k_inv_ag_fft(XformDev<T> X, const cT<T>* _
     cT<T>* sH = reinterpret_cast<cT<T>*>(smem_raw);  // [m >= 0][g][xl], row stride SH
     int j;
     int64_t x0;
-    ag_block<T, XC>(nxc, n2, j, x0);
+    ag_block<T>(XC, nxc, n2, j, x0);
     const int64_t nx = X.nx;
     // the Hermitian part of G (get_h): H[-m][g] = conj H[m][g], so only
     // the rows m >= 0 are transformed over n
@@ -992,7 +1205,7 @@ __global__ __launch_bounds__(NT) void k_fwd_ag_fft(XformDev<T> X, const T* __res
     cT<T>* sH = reinterpret_cast<cT<T>*>(smem_raw);  // [m>=0][g][xl], row stride SH, aliases sf
     int j;
     int64_t x0;
-    ag_block<T, XC>(nxc, n2, j, x0);
+    ag_block<T>(XC, nxc, n2, j, x0);
     const int64_t nx = X.nx;
     const int tid = threadIdx.x;
     stage_f_tile<T, XC, NT, n2>(f, wR, wstride, j, x0, nx, sf, rp);
@@ -1117,7 +1330,7 @@ __global__ __launch_bounds__(NT) void k_fwd_ag_q60(XformDev<T> X, const T* __res
     cT<T>* sZ = reinterpret_cast<cT<T>*>(smem_raw + 64 * sizeof(cT<T>));  // [xl][g < 30][K], aliases sf
     int j;
     int64_t x0;
-    ag_block<T, XC>(nxc, n2, j, x0);
+    ag_block<T>(XC, nxc, n2, j, x0);
     const int64_t nx = X.nx;
     const int tid = threadIdx.x;
     if (tid < n2) tw[tid] = X.twB[tid];
@@ -1186,7 +1399,7 @@ __global__ __launch_bounds__(NT) void k_inv_ag_q60(XformDev<T> X, const cT<T>* _
     T* so = reinterpret_cast<T*>(smem_raw + 64 * sizeof(cT<T>));          // [xl][g][a], aliases sH
     int j;
     int64_t x0;
-    ag_block<T, XC>(nxc, n2, j, x0);
+    ag_block<T>(XC, nxc, n2, j, x0);
     const int64_t nx = X.nx;
     const int tid = threadIdx.x;
     if (tid < n2) tw[tid] = X.twB[tid];
@@ -1261,9 +1474,55 @@ static int pick_xc(size_t per_x, size_t budget, int64_t nx) {
 #endif
 constexpr int kFftInvXC = HPUP_FFT_INV_XC, kFftFwdXC = HPUP_FFT_FWD_XC, kFftNT = HPUP_FFT_NT;
 
-// omega points per block of the register-row (alpha, gamma) kernels
-constexpr int kFwdXC = 8;
-template <class T> constexpr int inv_xc() { return sizeof(T) == 8 ? 4 : 8; }
+// Launch shape of the MFMA (alpha, gamma) kernels: omega points per block (a
+// power of two, log2 lx) and the LDS strides.  As many points as a 128-byte
+// line of G holds (16 in FP32, 8 in FP64) while a tile stays within 54 KB (three
+// blocks per CU), fewer at larger bandlimits, but not under 32-byte runs of G if
+// 80 KB (two blocks) hold them; never more than the grid has.  Measured per
+// forward kernel: whole lines against half ones at B = 6, 30^3, FP64 0.45 -> 0.28
+// ms, B = 10, 26^3, FP32 0.34 -> 0.27 ms; 32-byte against 16-byte runs at B = 32,
+// 12^3, FP64 3.9 -> 3.1 ms; at B = 20 to 25, 40 KB tiles cost the inverse 15-45%
+// and 80 KB ones gain nothing.
+template <class T> struct AgShape {
+    int lx, nxc, rs, sx;
+    size_t lds;
+    // row: values a row needs, rows: rows per omega point
+    AgShape(int row, int rows, int64_t nx) {
+        constexpr int banks = sizeof(T) == 4 ? 32 : 16;
+        rs = sizeof(T) == 4 ? (row % 4 == 2 ? row : row + 2) : row | 1;
+        lx = sizeof(T) == 4 ? 4 : 3;
+        while (lx > 0 && ((int64_t)1 << (lx - 1)) >= nx) lx--;
+        for (;; lx--) {
+            const int want = banks >> lx;  // sx = banks / XC modulo the banks
+            sx = rows * rs + ((want - rows * rs) % banks + banks) % banks;
+            lds = sizeof(T) * ((size_t)sx << lx);
+            const bool wide = ((int)sizeof(cT<T>) << lx) > 32;  // the next smaller block still writes 32-byte runs
+            if (lx == 0 || lds <= (size_t)(wide ? 54 : 80) * 1024) break;
+        }
+        const int64_t n = (nx + ((int64_t)1 << lx) - 1) >> lx;
+        HPUP_REQUIRE(n * rows * 4 < (1ll << 31), HPUP_ERR_UNSUPPORTED, "omega grid too large");
+        nxc = (int)n;
+    }
+};
+
+template <class T, int MT, int KS>
+static void fwd_ag_mfma(const XformDev<T>& X, const void* f, const void* wR, int wstride, void* G, hipStream_t st) {
+    const int n2 = 2 * X.B;
+    const AgShape<T> s(n2, n2, X.nx);
+    const int vec = (reinterpret_cast<uintptr_t>(f) % (2 * sizeof(T))) == 0;  // n2 is even: rows keep the alignment
+    allow_lds((const void*)k_fwd_ag_mfma<T, MT, KS>, s.lds);
+    hipLaunchKernelGGL((k_fwd_ag_mfma<T, MT, KS>), dim3((unsigned)(s.nxc * n2)), dim3(256), s.lds, st, X, (const T*)f,
+                       (const T*)wR, wstride, (cT<T>*)G, s.lx, s.nxc, s.rs, s.sx, vec);
+}
+template <class T, int MT, int KS>
+static void inv_ag_mfma(const XformDev<T>& X, const void* H, void* f, hipStream_t st) {
+    const int n2 = 2 * X.B;
+    const AgShape<T> s(2 * n2 + 2, X.B, X.nx);  // (B slots of 4 B values, and room for the clamped reads at B = 1)
+    const int vec = (reinterpret_cast<uintptr_t>(f) % (2 * sizeof(T))) == 0;
+    allow_lds((const void*)k_inv_ag_mfma<T, MT, KS>, s.lds);
+    hipLaunchKernelGGL((k_inv_ag_mfma<T, MT, KS>), dim3((unsigned)(s.nxc * n2)), dim3(256), s.lds, st, X,
+                       (const cT<T>*)H, (T*)f, s.lx, s.nxc, s.rs, s.sx, vec);
+}
 
 template <class T, int B, int XC, int NT>
 static void fwd_ag_fft(const XformDev<T>& X, const void* f, const void* wR, int wstride, void* G, hipStream_t st) {
@@ -1342,15 +1601,19 @@ void launch_fwd_ag(const XformDev<T>& X, const void* f, const void* wR, int wstr
             fwd_ag_q60<T, kQ60FwdXC32, (120 * kQ60FwdXC32 + 63) / 64 * 64>(X, f, wR, wstride, G, st);
         return;
     }
-    if (n2 <= kAgMax) {
-        constexpr int XC = kFwdXC;
-        const int nxc = (int)((X.nx + XC - 1) / XC);
-        HPUP_REQUIRE((int64_t)nxc * n2 < (1ll << 31), HPUP_ERR_UNSUPPORTED, "omega grid too large");
-        const size_t sh = std::max(sizeof(T) * XC * n2 * (n2 + 1), sizeof(cT<T>) * X.B * n2 * XC);
-        allow_lds((const void*)k_fwd_ag_r<T, XC>, sh);
-        hipLaunchKernelGGL((k_fwd_ag_r<T, XC>), dim3((unsigned)(nxc * n2)), dim3(256), sh, st, X, (const T*)f,
-                           (const T*)wR, wstride, (cT<T>*)G, nxc);
-        return;
+    if (X.B <= 32) {  // K = B + 1 angles in steps of 4, rows m, n < B in tiles of 16
+        switch (X.B / 4) {
+        case 0: return fwd_ag_mfma<T, 1, 1>(X, f, wR, wstride, G, st);
+        case 1: return fwd_ag_mfma<T, 1, 2>(X, f, wR, wstride, G, st);
+        case 2: return fwd_ag_mfma<T, 1, 3>(X, f, wR, wstride, G, st);
+        case 3: return fwd_ag_mfma<T, 1, 4>(X, f, wR, wstride, G, st);
+        case 4: return X.B == 16 ? fwd_ag_mfma<T, 1, 5>(X, f, wR, wstride, G, st)
+                                 : fwd_ag_mfma<T, 2, 5>(X, f, wR, wstride, G, st);
+        case 5: return fwd_ag_mfma<T, 2, 6>(X, f, wR, wstride, G, st);
+        case 6: return fwd_ag_mfma<T, 2, 7>(X, f, wR, wstride, G, st);
+        case 7: return fwd_ag_mfma<T, 2, 8>(X, f, wR, wstride, G, st);
+        default: return fwd_ag_mfma<T, 2, 9>(X, f, wR, wstride, G, st);
+        }
     }
     const size_t per_x = sizeof(T) * n2 * n2 + sizeof(cT<T>) * n2 * X.B;
     const int XC = pick_xc(per_x, kLdsTile - sizeof(cT<T>) * n2, X.nx);
@@ -1419,17 +1682,19 @@ void launch_inv_ag(const XformDev<T>& X, const void* G, void* f, hipStream_t st)
         else inv_ag_q60<T, kQ60InvXC32, (240 * kQ60InvXC32 + 63) / 64 * 64>(X, G, f, st);
         return;
     }
-    if (n2 <= kAgMax) {
-        constexpr int XC = inv_xc<T>();
-        const int nxc = (int)((X.nx + XC - 1) / XC);
-        HPUP_REQUIRE((int64_t)nxc * n2 < (1ll << 31), HPUP_ERR_UNSUPPORTED, "omega grid too large");
-        const size_t sh = sizeof(cT<T>) * M * n2 * XC;
-        allow_lds((const void*)k_inv_ag_r<T, XC>, sh);
-        hipLaunchKernelGGL((k_inv_ag_r<T, XC>), dim3((unsigned)(nxc * n2)), dim3(256), sh, st, X, (const cT<T>*)G,
-                           (T*)f, nxc);
-        return;
+    if (X.B <= 32) {  // K = B frequencies in steps of 4, rows a, g <= B in tiles of 16
+        switch ((X.B + 3) / 4) {
+        case 1: return inv_ag_mfma<T, 1, 1>(X, G, f, st);
+        case 2: return inv_ag_mfma<T, 1, 2>(X, G, f, st);
+        case 3: return inv_ag_mfma<T, 1, 3>(X, G, f, st);
+        case 4: return X.B < 16 ? inv_ag_mfma<T, 1, 4>(X, G, f, st) : inv_ag_mfma<T, 2, 4>(X, G, f, st);
+        case 5: return inv_ag_mfma<T, 2, 5>(X, G, f, st);
+        case 6: return inv_ag_mfma<T, 2, 6>(X, G, f, st);
+        case 7: return inv_ag_mfma<T, 2, 7>(X, G, f, st);
+        default: return X.B < 32 ? inv_ag_mfma<T, 2, 8>(X, G, f, st) : inv_ag_mfma<T, 3, 8>(X, G, f, st);
+        }
     }
-    // gamma chunks of 16 for 2B > 32
+    // gamma chunks of 16 for B > 32
     constexpr int GC = 16;
     const int ngc = (n2 + GC - 1) / GC;
     const size_t per_x = sizeof(cT<T>) * ((size_t)M * n2);
