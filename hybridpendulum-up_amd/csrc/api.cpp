@@ -42,9 +42,28 @@ static const double kPi = 3.14159265358979323846;
 
 template <class T> std::vector<T> cast_vec(const std::vector<double>& v) { return std::vector<T>(v.begin(), v.end()); }
 
+// Tables of the parity-folded DFTs of length 2H: cos then sin (pi r k / H) for
+// r < rows, k < cols, in kAgTabR rows of kAgTabK, zero padded; halve: the
+// entries k = 0 and k = H halved (the folded data hold those points twice).
+// Exactly reduced, so cos and sin vanish exactly where they should.
+template <class T> static std::vector<T> half_dft_table(int H, int rows, int cols, bool halve) {
+    const int sz = kAgTabR * kAgTabK;
+    std::vector<T> t(2 * sz, T(0));
+    for (int r = 0; r < rows; r++)
+        for (int k = 0; k < cols; k++) {
+            const int e = (r * k) % (2 * H);
+            const double h = halve && (k == 0 || k == H) ? 0.5 : 1.0;
+            const double c = e == 0 ? 1.0 : e == H ? -1.0 : 2 * e == H || 2 * e == 3 * H ? 0.0 : std::cos(kPi * e / H);
+            const double s = e == 0 || e == H ? 0.0 : std::sin(kPi * e / H);
+            t[r * kAgTabK + k] = (T)(h * c);
+            t[sz + r * kAgTabK + k] = (T)(h * s);
+        }
+    return t;
+}
+
 // Transform tables from a Wigner-d table d (M,M,B,2B) and weights w (2B).
 template <class T> struct XformTables {
-    DevBuf Wf, Wi, twB, agF, agI, dftN, idftN, twNf, twNi, bsF, bsI, hrows;
+    DevBuf Wf, Wi, twB, agF, agI, dftN, idftN, omT, bsF, bsI, hrows;
     XformDev<T> view{};
     void build(int B, int dim, int N, const double* d, const double* w) {
         const int M = 2 * B - 1, n2 = 2 * B;
@@ -65,33 +84,15 @@ template <class T> struct XformTables {
         view.wis = wis;
         Wf = upload(cast_vec<T>(wf));
         Wi = upload(cast_vec<T>(wi));
-        std::vector<T> tb(2 * n2), dn, idn, tf, ti;
+        std::vector<T> tb(2 * n2), dn, idn;
         for (int t = 0; t < n2; t++) { tb[2 * t] = (T)std::cos(kPi * t / B); tb[2 * t + 1] = (T)std::sin(kPi * t / B); }
         twB = upload(tb);
         if (B <= 32) {  // MFMA (alpha, gamma) tables (see XformDev::agF)
-            const int sz = kAgTabR * kAgTabK;
-            std::vector<T> af(2 * sz, T(0)), ai(2 * sz, T(0));
-            for (int r = 0; r <= B; r++)
-                for (int k = 0; k <= B; k++) {
-                    // exactly reduced: cos and sin vanish exactly where they should
-                    const int e = (r * k) % n2;
-                    const double c = e % B == 0 ? (e ? -1.0 : 1.0) : 2 * e % n2 == B ? 0.0 : std::cos(kPi * e / B);
-                    const double s = e % B == 0 ? 0.0 : std::sin(kPi * e / B);
-                    if (r < B) {
-                        const double h = k == 0 || k == B ? 0.5 : 1.0;
-                        af[r * kAgTabK + k] = (T)(h * c);
-                        af[sz + r * kAgTabK + k] = (T)(h * s);
-                    }
-                    if (k < B) {
-                        ai[r * kAgTabK + k] = (T)c;
-                        ai[sz + r * kAgTabK + k] = (T)s;
-                    }
-                }
-            agF = upload(af);
-            agI = upload(ai);
+            agF = upload(half_dft_table<T>(B, B, B + 1, true));
+            agI = upload(half_dft_table<T>(B, B + 1, B, false));
         }
         const int Nn = std::max(N, 1);
-        dn.resize(2 * (size_t)Nn * Nn); idn.resize(2 * (size_t)Nn * Nn); tf.resize(2 * Nn); ti.resize(2 * Nn);
+        dn.resize(2 * (size_t)Nn * Nn); idn.resize(2 * (size_t)Nn * Nn);
         for (int k = 0; k < Nn; k++) {
             for (int a = 0; a < Nn; a++) {
                 const double ang = 2.0 * kPi * (double)((int64_t)k * a % Nn) / Nn;
@@ -100,11 +101,9 @@ template <class T> struct XformTables {
                 idn[2 * ((size_t)k * Nn + a)] = (T)(std::cos(ang) / Nn);
                 idn[2 * ((size_t)k * Nn + a) + 1] = (T)(std::sin(ang) / Nn);
             }
-            const double ang = 2.0 * kPi * k / Nn;
-            tf[2 * k] = (T)std::cos(ang); tf[2 * k + 1] = (T)-std::sin(ang);
-            ti[2 * k] = (T)std::cos(ang); ti[2 * k + 1] = (T)std::sin(ang);
         }
-        dftN = upload(dn); idftN = upload(idn); twNf = upload(tf); twNi = upload(ti);
+        dftN = upload(dn); idftN = upload(idn);
+        if (dim >= 2 && Nn <= 64 && Nn % 2 == 0) omT = upload(half_dft_table<T>(Nn / 2, Nn / 2 + 1, Nn / 2 + 1, true));
         if (Nn <= 32) {  // chirp-Toeplitz tables: c_d = e^{+i pi d^2/N} (d in [-32, 32)), p_k = e^{-i pi k^2/N}
             std::vector<T> bf(2 * 96, T(0)), bi(2 * 96, T(0));
             auto ang = [&](int64_t q) { return kPi * (double)(((q % (2 * Nn)) + 2 * Nn) % (2 * Nn)) / Nn; };
@@ -137,7 +136,7 @@ template <class T> struct XformTables {
         view.agF = B <= 32 ? agF.as<T>() : nullptr;
         view.agI = B <= 32 ? agI.as<T>() : nullptr;
         view.dftN = dftN.as<cT<T>>(); view.idftN = idftN.as<cT<T>>();
-        view.twNf = twNf.as<cT<T>>(); view.twNi = twNi.as<cT<T>>();
+        view.omT = omT.as<T>();
         view.bsF = Nn <= 32 ? bsF.as<cT<T>>() : nullptr;
         view.bsI = Nn <= 32 ? bsI.as<cT<T>>() : nullptr;
     }
@@ -366,7 +365,7 @@ template <class T> struct PlanT : PlanBase {
             launch_omega_half<T>(xf.view, F, F, false, st);
         } else {
             launch_beta_fwd<T>(xf.view, G.p, F, st);
-            launch_omega_dft<T>(xf.view, F, nullptr, false, st);
+            launch_omega_dft<T>(xf.view, F, F, false, st);
         }
         HPUP_HIP(hipGetLastError());
     }
@@ -378,16 +377,14 @@ template <class T> struct PlanT : PlanBase {
             launch_omega_half<T>(xf.view, F, tmp.p, true, st);
             launch_beta_inv<T>(xf.view, tmp.p, G.p, st, false);
         } else {
-            launch_omega_dft_to<T>(xf.view, F, tmp.p, true, st);
+            launch_omega_dft<T>(xf.view, F, tmp.p, true, st);
             launch_beta_inv<T>(xf.view, tmp.p, G.p, st);
         }
         launch_inv_ag<T>(xf.view, G.p, f, st);
         HPUP_HIP(hipGetLastError());
     }
-    // omega DFTs of the transforms on half of the rows (chirp MFMA kernels)
-    bool half_omega() const {
-        return (model.dim == 2 || model.dim == 3) && model.N <= 32 && model.B <= 32 && xf.view.bsF && xf.view.hrows;
-    }
+    // omega DFTs of the transforms on half of the rows
+    bool half_omega() const { return model.B <= 32 && omega_half_ok(xf.view); }
     // MFMA kernels cover omega grids up to 32 points per axis, and up to 64 for
     // the reduced model (dim 2); larger grids use the LDS-tiled FMA kernels
     // (three passes).

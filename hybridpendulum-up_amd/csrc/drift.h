@@ -90,16 +90,6 @@ template <class T>
 void launch_axis3_mfma(const DriftDev<T>& D, const void* in, void* out, bool bf16x3, hipStream_t st,
                        bool scaled = false);
 
-// Omega DFTs as chirp-Toeplitz MFMA products (N <= 32).  bs: 96 entries, the
-// Toeplitz kernel c_d at [d + 32] for d in [-32, 32) and then the chirp p_k
-// (zero for k >= N); see k_slab_dft_mfma.
-template <class T>
-void launch_slab_dft_mfma(const void* in, void* out, int64_t nslab, int N, const void* bs, T scale,
-                          hipStream_t st);
-template <class T>
-void launch_axis_dft_mfma(const void* in, void* out, int N, int64_t inner, int64_t nlines, const void* bs, T scale,
-                          hipStream_t st);
-
 template <class T>
 void launch_rotmix(const DriftDev<T>& D, const void* F, void* W, void* V1, void* V2, hipStream_t st);
 // out[r][x] += scale sum_t coef[r][t] in[src[r][t]][x] over rows of nx points (src -1 padded, TS per row)
@@ -133,10 +123,10 @@ template <class T> struct XformDev {
     const T* agI;
     const cT<T>* dftN;  // forward DFT matrix N x N (row-major [k][a]) e^{-2 pi i k a/N}
     const cT<T>* idftN; // inverse DFT matrix (1/N scaled) e^{+2 pi i k a/N}/N
-    const cT<T>* twNf;  // e^{-2 pi i t/N}, t in [0, N)
-    const cT<T>* twNi;  // e^{+2 pi i t/N}
-    const cT<T>* bsF;   // chirp-Toeplitz tables of the forward / inverse omega DFT (N <= 32),
-    const cT<T>* bsI;   // 96 entries each (launch_slab_dft_mfma)
+    const T* omT;       // (k1, k2) DFT: cos then sin (2 pi k a / N), rows k <= N / 2, a <= N / 2 (entries a = 0 and
+                        // N / 2 halved), in kAgTabR rows of kAgTabK, zero padded
+    const cT<T>* bsF;   // chirp-Toeplitz tables of the forward / inverse k3 DFT (N <= 32),
+    const cT<T>* bsI;   // 96 entries each (k_axis_dft_mfma)
     // the rows (l, m, n) with n > 0, or n = 0 and m >= 0: pairs (row, row of
     // (l, -m, -n) | bit 30 when (-1)^(m-n) = -1), nhalf of them
     const int32_t* hrows;
@@ -167,18 +157,20 @@ template <class T>
 void launch_beta_inv(const XformDev<T>& X, const void* F, void* G, hipStream_t st, bool sym = true);
 template <class T>
 void launch_inv_ag(const XformDev<T>& X, const void* G, void* f, hipStream_t st);
-// in-place omega DFT of the compact rows (forward sign -1, inverse +1 with 1/nx)
+// omega DFT of the compact rows from in to out (out = in allowed), forward
+// sign -1, inverse +1 with 1/nx
 template <class T>
-void launch_omega_dft(const XformDev<T>& X, void* F, void* tmp, bool inverse, hipStream_t st);
-// the same from in to out (out = in allowed)
-template <class T>
-void launch_omega_dft_to(const XformDev<T>& X, const void* in, void* out, bool inverse, hipStream_t st);
-// Omega DFTs of the coefficients of a real grid on the half rows only (N <= 32).
+void launch_omega_dft(const XformDev<T>& X, const void* in, void* out, bool inverse, hipStream_t st);
+// Omega DFTs of the coefficients of a real grid on the half rows only
+// (omega_half_ok).
 // Forward (in place): the input holds the mirror relation F_{-m,-n} = (-1)^(m-n)
 // conj F_mn on its half rows' partners implicitly (only the half rows are read)
 // and every row is written.  Inverse (out of place): out's half rows get the
 // inverse DFT of the Hermitian part (F_mn(k) + (-1)^(m-n) conj F_{-m,-n}(-k)) / 2;
 // the other rows of out are not written.
+template <class T> bool omega_half_ok(const XformDev<T>& X) {
+    return ((X.dim == 2 && X.N <= 64) || (X.dim == 3 && X.N <= 32 && X.bsF)) && X.omT && X.hrows;
+}
 template <class T>
 void launch_omega_half(const XformDev<T>& X, const void* in, void* out, bool inverse, hipStream_t st);
 

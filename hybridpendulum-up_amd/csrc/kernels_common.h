@@ -42,6 +42,12 @@ template <class T> __device__ __forceinline__ void cfma(cT<T>& acc, cT<T> a, cT<
 // i * s * a  (multiplication by the imaginary scalar i s)
 template <class T> __device__ __forceinline__ cT<T> cimul(cT<T> a, T s) { return cmk<T>(-a.y * s, a.x * s); }
 
+// i / d for 0 <= i < 2^17 and 1 <= d <= 4096 with i / d < 2^12, inv = 1.0f / d: (i + 0.5) / d
+// is at least 0.5 / d away from an integer, beyond the rounding of two FP32
+// operations (2^-22 i / d).  Three instructions instead of an integer division's twenty:
+// the index arithmetic of a tile's staging took as long as its products.
+__device__ __forceinline__ int div_small(int i, float inv) { return (int)(((float)i + 0.5f) * inv); }
+
 // m-major compact rotation index (same formula as the host's ridx_B)
 __device__ __forceinline__ int64_t d_sumsq(int64_t n) { return n * (n + 1) * (2 * n + 1) / 6; }
 __device__ __forceinline__ int64_t d_moff(int B, int m) {

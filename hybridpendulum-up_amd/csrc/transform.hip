@@ -482,45 +482,6 @@ __global__ __launch_bounds__(256) void k_inv_ag(XformDev<T> X, const cT<T>* __re
     }
 }
 
-// ---------------------------------------------------------- omega DFT -----
-
-// In-place 2-D DFT over (k1, k2) of every N x N slab, twiddle-indexed.
-template <class T>
-__global__ __launch_bounds__(1024) void k_slab_dft(cT<T>* __restrict__ F, const cT<T>* __restrict__ twN, int N, T scale) {
-    extern __shared__ char smem_raw[];
-    const int NN = N * N;
-    cT<T>* sA = reinterpret_cast<cT<T>*>(smem_raw);
-    cT<T>* sB = sA + NN;
-    cT<T>* tw = sB + NN;
-    const int64_t base = (int64_t)blockIdx.x * NN;
-    for (int e = threadIdx.x; e < NN; e += blockDim.x) sA[e] = F[base + e];
-    for (int e = threadIdx.x; e < N; e += blockDim.x) tw[e] = twN[e];
-    __syncthreads();
-    for (int e = threadIdx.x; e < NN; e += blockDim.x) {
-        const int k1 = e % N, k2 = e / N;
-        cT<T> acc = czero<T>();
-        int t = 0;
-        for (int a = 0; a < N; a++) {
-            cfma<T>(acc, tw[t], sA[k2 * N + a]);
-            t += k1;
-            if (t >= N) t -= N;
-        }
-        sB[e] = acc;
-    }
-    __syncthreads();
-    for (int e = threadIdx.x; e < NN; e += blockDim.x) {
-        const int k1 = e % N, k2 = e / N;
-        cT<T> acc = czero<T>();
-        int t = 0;
-        for (int a = 0; a < N; a++) {
-            cfma<T>(acc, tw[t], sB[a * N + k1]);
-            t += k2;
-            if (t >= N) t -= N;
-        }
-        F[base + e] = cscale<T>(acc, scale);
-    }
-}
-
 // ---------------------------------------------------------- layouts -------
 
 template <class T>
@@ -626,12 +587,6 @@ template <class T> __device__ __forceinline__ void ag_block(int XC, int nxc, int
 // 7.34 -> 1.18 ms against the direct DFTs in LDS these replace there; at
 // B = 10, 16^3, FP64 (direct DFTs in registers before): forward 0.378 -> 0.136,
 // inverse 0.530 -> 0.137 ms.
-
-// i / d for 0 <= i < 2^17 and 1 <= d <= 64, inv = 1.0f / d: (i + 0.5) / d is at
-// least 0.5 / d away from an integer, far beyond the rounding of two FP32
-// operations.  Three instructions instead of an integer division's twenty:
-// the index arithmetic of the tiles' staging was half of the kernels' time.
-__device__ __forceinline__ int div_small(int i, float inv) { return (int)(((float)i + 0.5f) * inv); }
 
 // DFT tables of lane (lr, lq): row 16 t + lr, K index 4 s + lq (zero padded)
 template <class T, int MT, int KS> struct AgTab {
@@ -1706,55 +1661,6 @@ void launch_inv_ag(const XformDev<T>& X, const void* G, void* f, hipStream_t st)
     hipLaunchKernelGGL((k_inv_ag<T, GC>), grid, dim3(256), sh, st, X, (const cT<T>*)G, (T*)f, XC);
 }
 
-// out-of-place omega DFT: on the chirp path the first pass reads in and
-// writes out (the k3 pass of a 3-D grid, then the (k1, k2) pass in place on
-// out: DFTs along different axes commute); otherwise a copy and the in-place
-// transform
-template <class T>
-void launch_omega_dft_to(const XformDev<T>& X, const void* in, void* out, bool inverse, hipStream_t st) {
-    const int N = X.N, NN = N * N;
-    if ((X.dim == 2 || X.dim == 3) && N <= 32 && X.bsF && in != out) {
-        const cT<T>* bs = inverse ? X.bsI : X.bsF;
-        const T s2 = inverse ? T(1) / T(NN) : T(1);
-        if (X.dim == 3) {
-            launch_axis_dft_mfma<T>(in, out, N, (int64_t)NN, X.nrc, bs, inverse ? T(1) / T(N) : T(1), st);
-            launch_slab_dft_mfma<T>(out, out, X.nrc * N, N, bs, s2, st);
-        } else {
-            launch_slab_dft_mfma<T>(in, out, X.nrc, N, bs, s2, st);
-        }
-        return;
-    }
-    if (in != out)
-        HPUP_HIP(hipMemcpyAsync(out, in, sizeof(cT<T>) * (size_t)(X.nrc * X.nx), hipMemcpyDeviceToDevice, st));
-    launch_omega_dft<T>(X, out, nullptr, inverse, st);
-}
-
-template <class T>
-void launch_omega_dft(const XformDev<T>& X, void* F, void* tmp, bool inverse, hipStream_t st) {
-    (void)tmp;
-    if (X.dim == 0) return;
-    const int N = X.N, NN = N * N;
-    HPUP_REQUIRE(NN <= 4096, HPUP_ERR_UNSUPPORTED, "omega grid larger than 64 per axis");
-    if (N <= 32 && X.bsF) {  // chirp-Toeplitz products on MFMA
-        const cT<T>* bs = inverse ? X.bsI : X.bsF;
-        const int64_t nslab = X.nrc * (X.dim == 3 ? N : 1);
-        launch_slab_dft_mfma<T>(F, F, nslab, N, bs, inverse ? T(1) / T(NN) : T(1), st);
-        if (X.dim == 3) launch_axis_dft_mfma<T>(F, F, N, (int64_t)NN, X.nrc, bs, inverse ? T(1) / T(N) : T(1), st);
-        return;
-    }
-    const cT<T>* Mat = inverse ? X.idftN : X.dftN;
-    // twiddles: row 1 of the matrix (unscaled)
-    const T sc2 = inverse ? T(1) / T(NN) : T(1);
-    const int64_t nslab = X.nrc * (X.dim == 3 ? N : 1);
-    const int nt = NN <= 256 ? 256 : 1024;
-    const size_t sh = sizeof(cT<T>) * (2 * (size_t)NN + N);
-    allow_lds((const void*)k_slab_dft<T>, sh);
-    hipLaunchKernelGGL(k_slab_dft<T>, dim3((unsigned)nslab), dim3(nt), sh, st, (cT<T>*)F, inverse ? X.twNi : X.twNf,
-                       N, sc2);
-    if (X.dim == 3)
-        launch_axis_outer<T>(F, F, Mat, N, (int64_t)NN, X.nrc, T(1), st);
-}
-
 template <class T>
 void launch_full_to_compact(int B, int64_t nx, const void* full, void* compact, hipStream_t st) {
     const int64_t nrc = nrc_of(B);
@@ -1777,8 +1683,6 @@ void launch_compact_to_full(int B, int64_t nx, const void* compact, void* full, 
     template void launch_beta_fwd<T>(const XformDev<T>&, const void*, void*, hipStream_t, bool);           \
     template void launch_beta_inv<T>(const XformDev<T>&, const void*, void*, hipStream_t, bool);           \
     template void launch_inv_ag<T>(const XformDev<T>&, const void*, void*, hipStream_t);             \
-    template void launch_omega_dft<T>(const XformDev<T>&, void*, void*, bool, hipStream_t);          \
-    template void launch_omega_dft_to<T>(const XformDev<T>&, const void*, void*, bool, hipStream_t); \
     template void launch_full_to_compact<T>(int, int64_t, const void*, void*, hipStream_t);          \
     template void launch_compact_to_full<T>(int, int64_t, const void*, void*, hipStream_t);
 HPUP_INST(double)
