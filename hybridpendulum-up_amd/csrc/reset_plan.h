@@ -16,6 +16,7 @@ struct ResetConsts {
     double x0, hx, ihx;     // 3-D: grid origin, spacing and its reciprocal
     double xlo, xhi;        // 2-D: getOmega's box of valid pull-backs
     double Lg, dx2;         // 2-D: getIndRule's box length and cell area
+    double ulo, uhi;        // 2-D: the box in grid units
     double kfac;            // (1 + eps) / eps
     double J;               // jump-term Jacobian factor (1/eps or 1)
     double ew[3];           // wall normal

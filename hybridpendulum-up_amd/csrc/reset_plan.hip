@@ -398,6 +398,156 @@ __global__ __launch_bounds__(256) void k_sum_partials(const double* __restrict__
 // Groups are numbered XCD-major: the groups that run at once on one XCD are
 // neighbours and share the cache lines of their rows in that XCD's L2.
 
+// The pull-back in body coordinates and grid units: with the unit tangent
+// s = R^T t and y = Omega / h (integers i - N/2), R^T R = 1 gives
+//   Omega- / h = y - ((1 + eps)/eps) (s . y) s,   omega . t = h (s . y),
+// a dozen FP64 operations where the chain omega = R Omega, omega-, R^T omega-
+// takes sixty; the contact sign is that of sigma (s . y).  Both forms agree
+// to rounding, so the masks differ at most where s . y (dim 2: or the distance
+// to an edge of the box) is at rounding level: those points, told by a margin
+// of 1e-12 N grid units, take the masks of the chain itself (exact_masks), in
+// its order of operations.  Measured on the rows kernel: B = 30, 20^3, FP32 4.81
+// -> 3.64 ms, B = 30, 60^2, FP64 2.02 -> 1.50 ms.  Of the 3.64 ms, staging takes 1.4,
+// stores 1.3 and the arithmetic the rest, in turn (one workgroup per CU holds a
+// group); loading the next group into registers meanwhile made it 5.1 ms (spills).
+struct RowFast {
+    double s[3], sigma, lam;
+};
+__device__ __forceinline__ RowFast row_fast(const RowGeo& G) {
+    RowFast r;
+#pragma unroll
+    for (int a = 0; a < 3; a++) r.s[a] = G.R[3 * a] * G.t[0] + G.R[3 * a + 1] * G.t[1] + G.R[3 * a + 2] * G.t[2];
+    r.sigma = G.sigma;
+    r.lam = G.lam;
+    return r;
+}
+
+// the masks of the law's own chain of operations (jump_at's)
+template <int DIM>
+__device__ __forceinline__ int exact_masks(const double* sg, int stride, int k, const ResetConsts& c, int i0, int i1,
+                                        int i2) {
+    const RowGeo G = row_geo(sg, stride, k, c);
+    Jump<DIM> J;
+    jump_at<DIM>(G, c, i0, i1, i2, 0.0, J);
+    return (J.out_on ? 1 : 0) | (J.in_on ? 2 : 0);
+}
+
+template <int DIM> struct Pull {
+    bool out_on, in_on;
+    int c[DIM];     // cell (dim 3: -1 .. N - 1, dim 2: 0 .. N - 2)
+    double f[DIM];  // position in the cell
+    double dot;     // s . y
+    bool face;      // on a cell face to rounding: the interpolant is continuous there, its derivative is not
+};
+template <int DIM>
+__device__ __forceinline__ void pull_at(const RowFast& r, const double* sg, int stride, int k, const ResetConsts& c,
+                                        int i0, int i1, int i2, Pull<DIM>& p) {
+    const int N = c.N, h = N / 2;
+    const double tol = 1e-12 * N;
+    const int id[3] = {i0, i1, i2};
+    double dot = r.s[0] * (double)(i0 - h) + r.s[1] * (double)(i1 - h);
+    if (DIM == 3) dot += r.s[2] * (double)(i2 - h);
+    const double v = r.sigma * dot, q = c.kfac * dot;
+    bool near = fabs(dot) < tol;
+    p.out_on = DIM == 2 ? v >= 0.0 : v > 0.0;
+    p.in_on = DIM == 2 ? v <= 0.0 : v < 0.0;
+    p.face = false;
+    const double lo = DIM == 2 ? c.ulo : -1.0, hi = DIM == 2 ? c.uhi : (double)N;
+#pragma unroll
+    for (int a = 0; a < DIM; a++) {
+        const double u = (double)id[a] - q * r.s[a];
+        if (DIM == 2) near = near || fabs(u - lo) < tol || fabs(u - hi) < tol;
+        p.in_on = p.in_on && u >= lo && u <= hi;
+        p.face = p.face || fabs(u - rint(u)) < tol;
+        // beyond the support only masked points remain
+        const double cf = fmin(fmax(floor(u), DIM == 2 ? 0.0 : -1.0), DIM == 2 ? (double)(N - 2) : (double)(N - 1));
+        p.c[a] = (int)cf;
+        p.f[a] = u - cf;
+    }
+    p.dot = dot;
+    if (near) {
+        // (an opaque row index keeps the row's 19 geometry values from being
+        // loaded ahead of the caller's loop and held in registers)
+        int kk = k;
+        asm volatile("" : "+v"(kk));
+        const int m = exact_masks<DIM>(sg, stride, kk, c, i0, i1, i2);
+        p.out_on = m & 1;
+        p.in_on = m & 2;
+    }
+}
+
+// Corner weights and clamped indices along one axis: dim 3 extends the grid by
+// zero (corners beyond it weigh nothing)
+struct AxisW {
+    double w0, w1;
+    int j0, j1;
+};
+template <int DIM> __device__ __forceinline__ AxisW axis_w(const Pull<DIM>& p, int a, int N) {
+    AxisW x;
+    const int c = p.c[a];
+    if constexpr (DIM == 2) {
+        x = {1.0 - p.f[a], p.f[a], c, c + 1};
+    } else {
+        x.w0 = c >= 0 ? 1.0 - p.f[a] : 0.0;
+        x.w1 = c + 1 < N ? p.f[a] : 0.0;
+        x.j0 = c >= 0 ? c : 0;
+        x.j1 = c + 1 < N ? c + 1 : N - 1;
+    }
+    return x;
+}
+
+// the interpolated value of an LDS row
+template <class T, int DIM>
+__device__ __forceinline__ double interp_row(const T* row, const Pull<DIM>& p, int N) {
+    const AxisW x = axis_w<DIM>(p, 0, N), y = axis_w<DIM>(p, 1, N);
+    auto line = [&](const T* l) { return x.w0 * (double)l[x.j0] + x.w1 * (double)l[x.j1]; };
+    auto plane = [&](const T* l) { return y.w0 * line(l + N * y.j0) + y.w1 * line(l + N * y.j1); };
+    if constexpr (DIM == 2) {
+        return plane(row);
+    } else {
+        const AxisW z = axis_w<DIM>(p, 2, N);
+        return z.w0 * plane(row + N * N * z.j0) + z.w1 * plane(row + N * N * z.j1);
+    }
+}
+// the same and its derivative when the position moves by d (grid units) per unit
+template <class T, int DIM>
+__device__ __forceinline__ double interp_row_d(const T* row, const Pull<DIM>& p, int N, const double* d, double& dv) {
+    AxisW x[DIM];
+    double e0[DIM], e1[DIM];
+#pragma unroll
+    for (int a = 0; a < DIM; a++) {
+        x[a] = axis_w<DIM>(p, a, N);
+        e0[a] = DIM == 2 || p.c[a] >= 0 ? -d[a] : 0.0;
+        e1[a] = DIM == 2 || p.c[a] + 1 < N ? d[a] : 0.0;
+    }
+    auto line = [&](const T* l, double& dl) {
+        const double a = (double)l[x[0].j0], b = (double)l[x[0].j1];
+        dl = e0[0] * a + e1[0] * b;
+        return x[0].w0 * a + x[0].w1 * b;
+    };
+    auto plane = [&](const T* l, double& dp) {
+        double d0, d1;
+        const double a = line(l + N * x[1].j0, d0), b = line(l + N * x[1].j1, d1);
+        dp = x[1].w0 * d0 + x[1].w1 * d1 + e0[1] * a + e1[1] * b;
+        return x[1].w0 * a + x[1].w1 * b;
+    };
+    if constexpr (DIM == 2) {
+        return plane(row, dv);
+    } else {
+        double d0, d1;
+        const double a = plane(row + N * N * x[2].j0, d0), b = plane(row + N * N * x[2].j1, d1);
+        dv = x[2].w0 * d0 + x[2].w1 * d1 + e0[2] * a + e1[2] * b;
+        return x[2].w0 * a + x[2].w1 * b;
+    }
+}
+
+// LDS row stride (elements): the 64 lanes of a wave hold 64 / RG consecutive
+// points of RG rows, so rows 64 / RG apart modulo the 64 fill distinct banks
+__host__ __device__ __forceinline__ int row_stride(int nx, int RG) {
+    const int want = RG > 1 ? 64 / RG : 0;
+    return nx + ((want - nx) % 64 + 64) % 64;
+}
+
 __device__ __forceinline__ int xcd_major_r(int b, int nb) {
     const int per = nb >> 3;
     if (b >= per << 3) return b;
@@ -420,29 +570,36 @@ struct RowLanes {
     }
 };
 
-// Rows of the group into LDS: a thread's loads are issued in batches of 8
-// before their LDS stores, so the staging costs one memory round trip per
-// batch instead of one per element.
+// Rows of the group into LDS: a thread's loads are issued in batches before
+// their LDS stores, so the staging costs one memory round trip per batch of 8
+// instead of one per element.  Larger batches are slower (B = 30, 60^2, FP64: 1.50
+// ms with 8, 1.52 with 16, 1.69 with 32): every point of a group lies on a page of
+// its own, and more loads in flight turn over the translation caches faster.
 template <class T>
 __device__ __forceinline__ void stage_rows(const T* __restrict__ src, const int32_t* __restrict__ indR, int k0, int nr,
-                                           int RG, int64_t nR, int nx, T* rows) {
+                                           int RG, int64_t nR, int nx, int ns, T* rows) {
     constexpr int BT = 8;
     const int r = (int)threadIdx.x & (RG - 1), S = (int)blockDim.x / RG;
     if (r >= nr) return;
-    const T* s = src + indR[k0 + r];
-    T* row = rows + (int64_t)r * nx;
-    for (int x0 = (int)threadIdx.x / RG; x0 < nx; x0 += BT * S) {
+    int x0 = (int)threadIdx.x / RG;
+    const int64_t step = nR * S;
+    const T* s = src + indR[k0 + r] + nR * x0;
+    T* row = rows + r * ns;
+    for (; x0 + (BT - 1) * S < nx; x0 += BT * S) {
         T v[BT];
 #pragma unroll
-        for (int u = 0; u < BT; u++) {
-            const int x = x0 + u * S;
-            v[u] = s[nR * (x < nx ? x : x0)];
-        }
+        for (int u = 0; u < BT; u++, s += step) v[u] = *s;
 #pragma unroll
-        for (int u = 0; u < BT; u++) {
-            const int x = x0 + u * S;
-            if (x < nx) row[x] = v[u];
-        }
+        for (int u = 0; u < BT; u++) row[x0 + u * S] = v[u];
+    }
+    if (x0 < nx) {  // the last, partial batch: clamped to its first point
+        T v[BT];
+        const T* s0 = s;
+#pragma unroll
+        for (int u = 0; u < BT; u++, s += step) v[u] = *(x0 + u * S < nx ? s : s0);
+#pragma unroll
+        for (int u = 0; u < BT; u++)
+            if (x0 + u * S < nx) row[x0 + u * S] = v[u];
     }
 }
 
@@ -457,29 +614,26 @@ __global__ __launch_bounds__(1024) void k_reset_rows(const T* f_in, T* f_out, co
                                                      int RG, ResetConsts c, double scale, int accumulate) {
     extern __shared__ double smem_rr[];
     double* sg = smem_rr;                       // G_N x RG
-    T* rows = (T*)(smem_rr + G_N * RG);          // RG x nx
+    T* rows = (T*)(smem_rr + G_N * RG);          // RG rows at stride ns
+    const int ns = row_stride(nx, RG);
     const int k0 = xcd_major_r(blockIdx.x, gridDim.x) * RG;
     const int nr = min(RG, numR - k0);
     stage_geo(geo, numR, k0, nr, sg);
-    stage_rows<T>(f_in, indR, k0, nr, RG, nR, nx, rows);
+    stage_rows<T>(f_in, indR, k0, nr, RG, nR, nx, ns, rows);
     __syncthreads();
     RowLanes L(RG, c.N);
     if (L.r >= nr) return;
-    const RowGeo G = row_geo(sg, nr, L.r, c);
-    const T* row = rows + (int64_t)L.r * nx;
-    T* out = f_out + indR[k0 + L.r];
-    for (int x = L.x0; x < nx; x += L.S, L.p.advance(L.d, c.N)) {
-        Jump<DIM> J;
-        jump_at<DIM>(G, c, L.p.i0, L.p.i1, L.p.i2, 0.0, J);
-        double d = J.out_on ? -(double)row[x] * G.lam : 0.0;
-        if (J.in_on) {
-            double v = 0.0;
-#pragma unroll
-            for (int q = 0; q < Jump<DIM>::NQ; q++) v += (double)row[J.q[q]] * J.w[q];
-            d = DIM == 2 ? v * G.lam + d : d + c.J * G.lam * v;
-        }
-        const double base = accumulate ? (double)row[x] : 0.0;
-        out[nR * x] = (T)(base + scale * d);
+    const RowFast G = row_fast(row_geo(sg, nr, L.r, c));
+    const T* row = rows + L.r * ns;
+    T* out = f_out + indR[k0 + L.r] + nR * L.x0;
+    const int64_t step = nR * L.S;
+    for (int x = L.x0; x < nx; x += L.S, L.p.advance(L.d, c.N), out += step) {
+        Pull<DIM> P;
+        pull_at<DIM>(G, sg, nr, L.r, c, L.p.i0, L.p.i1, L.p.i2, P);
+        const double fx = (double)row[x];
+        double d = P.out_on ? -fx * G.lam : 0.0;
+        if (P.in_on) d += c.J * G.lam * interp_row<T, DIM>(row, P, c.N);
+        *out = (T)((accumulate ? fx : 0.0) + scale * d);
     }
 }
 
@@ -492,36 +646,47 @@ __global__ __launch_bounds__(1024) void k_reset_adj_rows(const T* g_in, T* g_out
     extern __shared__ double smem_ra[];
     double* sg = smem_ra;
     T* rows = (T*)(smem_ra + G_N * RG);
-    T* acc = rows + (int64_t)RG * nx;
+    const int ns = row_stride(nx, RG);
+    T* acc = rows + RG * ns;
     const int k0 = xcd_major_r(blockIdx.x, gridDim.x) * RG;
     const int nr = min(RG, numR - k0);
     stage_geo(geo, numR, k0, nr, sg);
-    stage_rows<T>(g_in, indR, k0, nr, RG, nR, nx, rows);
-    for (int e = threadIdx.x; e < nr * nx; e += blockDim.x) acc[e] = T(0);
+    stage_rows<T>(g_in, indR, k0, nr, RG, nR, nx, ns, rows);
+    for (int e = threadIdx.x; e < nr * ns; e += blockDim.x) acc[e] = T(0);
     __syncthreads();
     RowLanes L(RG, c.N);
     const bool act = L.r < nr;
     if (act) {
-        const RowGeo G = row_geo(sg, nr, L.r, c);
-        const T* row = rows + (int64_t)L.r * nx;
-        T* ar = acc + (int64_t)L.r * nx;
+        const RowFast G = row_fast(row_geo(sg, nr, L.r, c));
+        const T* row = rows + L.r * ns;
+        T* ar = acc + L.r * ns;
         for (int x = L.x0; x < nx; x += L.S, L.p.advance(L.d, c.N)) {
-            Jump<DIM> J;
-            jump_at<DIM>(G, c, L.p.i0, L.p.i1, L.p.i2, 0.0, J);
+            Pull<DIM> P;
+            pull_at<DIM>(G, sg, nr, L.r, c, L.p.i0, L.p.i1, L.p.i2, P);
             const double gv = (double)row[x];
-            if (J.out_on) atomicAdd(ar + x, (T)(-G.lam * gv));
-            if (J.in_on) {
+            if (P.out_on) atomicAdd(ar + x, (T)(-G.lam * gv));
+            if (P.in_on) {
+                AxisW w[DIM];
+#pragma unroll
+                for (int a = 0; a < DIM; a++) w[a] = axis_w<DIM>(P, a, c.N);
                 const double a = c.J * G.lam * gv;
 #pragma unroll
-                for (int q = 0; q < Jump<DIM>::NQ; q++)
-                    if (J.w[q] != 0.0) atomicAdd(ar + J.q[q], (T)(a * J.w[q]));
+                for (int q = 0; q < (1 << DIM); q++) {
+                    double v = (q & 1 ? w[0].w1 : w[0].w0) * (q & 2 ? w[1].w1 : w[1].w0);
+                    int j = (q & 1 ? w[0].j1 : w[0].j0) + c.N * (q & 2 ? w[1].j1 : w[1].j0);
+                    if constexpr (DIM == 3) {
+                        v *= q & 4 ? w[2].w1 : w[2].w0;
+                        j += c.N * c.N * (q & 4 ? w[2].j1 : w[2].j0);
+                    }
+                    if (v != 0.0) atomicAdd(ar + j, (T)(a * v));
+                }
             }
         }
     }
     __syncthreads();
     if (!act) return;
-    const T* row = rows + (int64_t)L.r * nx;
-    const T* ar = acc + (int64_t)L.r * nx;
+    const T* row = rows + L.r * ns;
+    const T* ar = acc + L.r * ns;
     T* out = g_out + indR[k0 + L.r];
     for (int x = L.x0; x < nx; x += L.S) out[nR * x] = (T)((double)row[x] + scale * (double)ar[x]);
 }
@@ -542,13 +707,14 @@ __global__ __launch_bounds__(1024) void k_reset_deps_rows(const T* __restrict__ 
     const int k0 = grp * RG;
     const int nr = min(RG, numR - k0);
     stage_geo(geo, numR, k0, nr, sg);
-    stage_rows<T>(f, indR, k0, nr, RG, nR, nx, rows);
+    const int ns = row_stride(nx, RG);
+    stage_rows<T>(f, indR, k0, nr, RG, nR, nx, ns, rows);
     __syncthreads();
     RowLanes L(RG, c.N);
     double v = 0.0;
     if (L.r < nr) {
-        const RowGeo G = row_geo(sg, nr, L.r, c);
-        const T* row = rows + (int64_t)L.r * nx;
+        const RowFast G = row_fast(row_geo(sg, nr, L.r, c));
+        const T* row = rows + L.r * ns;
         const T* gr = g + indR[k0 + L.r];
         constexpr int BT = 4;  // g values of a batch of points loaded together
         for (int xb = L.x0; xb < nx; xb += BT * L.S) {
@@ -561,16 +727,28 @@ __global__ __launch_bounds__(1024) void k_reset_deps_rows(const T* __restrict__ 
 #pragma unroll
             for (int u = 0; u < BT; u++) {
                 if (xb + u * L.S >= nx) break;
-                Jump<DIM> J;
-                jump_at<DIM>(G, c, L.p.i0, L.p.i1, L.p.i2, -dk, J);
-                if (J.in_on) {
-                    double I = 0.0, dI = 0.0;
+                Pull<DIM> P;
+                pull_at<DIM>(G, sg, nr, L.r, c, L.p.i0, L.p.i1, L.p.i2, P);
+                if (P.face || fabs(P.dot) < 1e-12 * c.N) {  // the cell the law's own chain finds
+                    int kk = L.r;
+                    asm volatile("" : "+v"(kk));
+                    Jump<DIM> J;
+                    jump_at<DIM>(row_geo(sg, nr, kk, c), c, L.p.i0, L.p.i1, L.p.i2, -dk, J);
+                    if (J.in_on) {
+                        double I = 0.0, dI = 0.0;
 #pragma unroll
-                    for (int q = 0; q < Jump<DIM>::NQ; q++) {
-                        const double fq = (double)row[J.q[q]];
-                        I += J.w[q] * fq;
-                        dI += J.dw[q] * fq;
+                        for (int q = 0; q < Jump<DIM>::NQ; q++) {
+                            const double fq = (double)row[J.q[q]];
+                            I += J.w[q] * fq;
+                            dI += J.dw[q] * fq;
+                        }
+                        v += (double)gv[u] * G.lam * (dJ * I + c.J * dI);
                     }
+                } else if (P.in_on) {
+                    // d(Omega- / h)/d eps = -d((1 + eps)/eps)/d eps (s . y) s
+                    const double e = -dk * P.dot, d[3] = {e * G.s[0], e * G.s[1], e * G.s[2]};
+                    double dI;
+                    const double I = interp_row_d<T, DIM>(row, P, c.N, d, dI);
                     v += (double)gv[u] * G.lam * (dJ * I + c.J * dI);
                 }
                 L.p.advance(L.d, c.N);
@@ -626,6 +804,8 @@ void ResetGeom::build(int B, int dim_, int N_, double L, const hpup_reset_params
         c.dx2 = dx * dx;
         c.kfac = (1.0 + p.epsilon) / p.epsilon;
         c.J = 1.0;
+        c.ulo = (c.xlo - c.xg[0]) * c.ihx;
+        c.uhi = (c.xhi - c.xg[0]) * c.ihx;
     } else {
         c.kfac = (1.0 + p.epsilon) / p.epsilon;
         c.J = p.jacobian ? 1.0 / p.epsilon : 1.0;
@@ -686,7 +866,7 @@ void ResetGeom::build(int B, int dim_, int N_, double L, const hpup_reset_params
 // rows per group of the row-group kernels: as many as fit `per` bytes of LDS
 // per omega point into 128 KiB, at most 8; 0 if not even one row fits
 static int rows_per_group(int64_t nx, size_t per) {
-    const int64_t budget = 128 * 1024 - G_N * 8 * 8;
+    const int64_t budget = 128 * 1024 - G_N * 8 * 8;  // (the row padding comes on top, at most 64 values a row)
     const int64_t rg = std::min<int64_t>(budget / (nx * (int64_t)per), 8);
     return rg >= 8 ? 8 : rg >= 4 ? 4 : rg >= 2 ? 2 : (int)rg;  // a power of two (the kernels' lane split), or 0
 }
@@ -707,16 +887,14 @@ bool ResetGeom::rows_pass(const void* fin, void* fout, double scale, bool accumu
     if (RG < 1) return false;
     if (numR == 0) return true;
     const int ng = (numR + RG - 1) / RG;
-    const size_t sh = sizeof(double) * G_N * RG + sizeof(T) * (size_t)RG * nx;
-    if (dim == 2) {
-        allow_lds((const void*)k_reset_rows<T, 2>, sh);
-        hipLaunchKernelGGL((k_reset_rows<T, 2>), dim3(ng), dim3(1024), sh, st, (const T*)fin, (T*)fout,
-                           geo.as<double>(), indR.as<int32_t>(), numR, nR, (int)nx, RG, consts, scale, accumulate ? 1 : 0);
-    } else {
-        allow_lds((const void*)k_reset_rows<T, 3>, sh);
-        hipLaunchKernelGGL((k_reset_rows<T, 3>), dim3(ng), dim3(1024), sh, st, (const T*)fin, (T*)fout,
-                           geo.as<double>(), indR.as<int32_t>(), numR, nR, (int)nx, RG, consts, scale, accumulate ? 1 : 0);
-    }
+    const size_t sh = sizeof(double) * G_N * RG + sizeof(T) * (size_t)RG * row_stride((int)nx, RG);
+    auto go = [&](auto kern) {
+        allow_lds((const void*)kern, sh);
+        hipLaunchKernelGGL(kern, dim3(ng), dim3(1024), sh, st, (const T*)fin, (T*)fout, geo.as<double>(),
+                           indR.as<int32_t>(), numR, nR, (int)nx, RG, consts, scale, accumulate ? 1 : 0);
+    };
+    if (dim == 2) go(k_reset_rows<T, 2>);
+    else go(k_reset_rows<T, 3>);
     HPUP_HIP(hipGetLastError());
     return true;
 }
@@ -727,7 +905,7 @@ bool ResetGeom::adjoint_rows(const void* g, void* out, double scale, hipStream_t
     if (RG < 1) return false;
     if (numR == 0) return true;
     const int ng = (numR + RG - 1) / RG;
-    const size_t sh = sizeof(double) * G_N * RG + 2 * sizeof(T) * (size_t)RG * nx;
+    const size_t sh = sizeof(double) * G_N * RG + 2 * sizeof(T) * (size_t)RG * row_stride((int)nx, RG);
     if (dim == 2) {
         allow_lds((const void*)k_reset_adj_rows<T, 2>, sh);
         hipLaunchKernelGGL((k_reset_adj_rows<T, 2>), dim3(ng), dim3(1024), sh, st, (const T*)g, (T*)out,
@@ -786,7 +964,7 @@ void ResetGeom::eps_grad(const void* f, const void* g, double* part, double scal
     const int RG = rows_per_group(nx, sizeof(T));
     if (RG >= 1) {  // LDS row groups
         const int ng = (numR + RG - 1) / RG;
-        const size_t sh = sizeof(double) * G_N * RG + sizeof(T) * (size_t)RG * nx;
+        const size_t sh = sizeof(double) * G_N * RG + sizeof(T) * (size_t)RG * row_stride((int)nx, RG);
         if (dim == 2) {
             allow_lds((const void*)k_reset_deps_rows<T, 2>, sh);
             hipLaunchKernelGGL((k_reset_deps_rows<T, 2>), dim3(ng), dim3(1024), sh, st, (const T*)f, (const T*)g,
