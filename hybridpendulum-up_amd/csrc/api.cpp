@@ -63,7 +63,7 @@ template <class T> static std::vector<T> half_dft_table(int H, int rows, int col
 
 // Transform tables from a Wigner-d table d (M,M,B,2B) and weights w (2B).
 template <class T> struct XformTables {
-    DevBuf Wf, Wi, twB, agF, agI, dftN, idftN, omT, bsF, bsI, hrows;
+    DevBuf Wf, Wi, twB, agF, agI, twMB, twNf, twNi, dftN, idftN, omT, bsF, bsI, hrows;
     XformDev<T> view{};
     void build(int B, int dim, int N, const double* d, const double* w) {
         const int M = 2 * B - 1, n2 = 2 * B;
@@ -92,6 +92,30 @@ template <class T> struct XformTables {
             agI = upload(half_dft_table<T>(B, B + 1, B, false));
         }
         const int Nn = std::max(N, 1);
+        if (sizeof(T) == 4 && dim >= 2) {  // tables of the FP32 forms (see XformDev::keep)
+            if (n2 <= 32) {  // [r][t] then [t][r]: frequency r - (B-1), grid angle pi t / B, zero padded to 32 x 32
+                std::vector<T> tm(2 * 2 * 32 * 32, T(0));
+                for (int r = 0; r < M; r++)
+                    for (int t = 0; t < n2; t++) {
+                        const int e = (((r - (B - 1)) * t) % n2 + n2) % n2;
+                        for (int c = 0; c < 2; c++) {
+                            tm[2 * (r * 32 + t) + c] = tb[2 * e + c];
+                            tm[2 * (32 * 32 + t * 32 + r) + c] = tb[2 * e + c];
+                        }
+                    }
+                twMB = upload(tm);
+            }
+            if (dim == 2 && Nn > 32) {
+                std::vector<T> tf(2 * Nn), ti(2 * Nn);
+                for (int k = 0; k < Nn; k++) {
+                    const double ang = 2.0 * kPi * k / Nn;
+                    tf[2 * k] = (T)std::cos(ang); tf[2 * k + 1] = (T)-std::sin(ang);
+                    ti[2 * k] = (T)std::cos(ang); ti[2 * k + 1] = (T)std::sin(ang);
+                }
+                twNf = upload(tf);
+                twNi = upload(ti);
+            }
+        }
         dn.resize(2 * (size_t)Nn * Nn); idn.resize(2 * (size_t)Nn * Nn);
         for (int k = 0; k < Nn; k++) {
             for (int a = 0; a < Nn; a++) {
@@ -135,6 +159,8 @@ template <class T> struct XformTables {
         view.Wf = Wf.as<T>(); view.Wi = Wi.as<T>(); view.twB = twB.as<cT<T>>();
         view.agF = B <= 32 ? agF.as<T>() : nullptr;
         view.agI = B <= 32 ? agI.as<T>() : nullptr;
+        view.twMB = twMB.as<cT<T>>();
+        view.twNf = twNf.as<cT<T>>(); view.twNi = twNi.as<cT<T>>();
         view.dftN = dftN.as<cT<T>>(); view.idftN = idftN.as<cT<T>>();
         view.omT = omT.as<T>();
         view.bsF = Nn <= 32 ? bsF.as<cT<T>>() : nullptr;
@@ -354,37 +380,49 @@ template <class T> struct PlanT : PlanBase {
     }
     size_t cbytes() const { return sizeof(cT<T>) * (size_t)ncoef; }
 
+    // FP32 grids whose rounding 64-bit figures stand in (XformDev::keep): the
+    // reduced model's hybrid steps, whose densities get_stat reads, and 3-D grids
+    // of up to 16 points per axis, those of the restitution gradient
+    bool keep_fp32(bool hybrid) const {
+        return sizeof(T) == 4 && ((model.dim == 2 && hybrid) || (model.dim == 3 && model.N <= 16));
+    }
+    XformDev<T> xform(bool hybrid) const {
+        XformDev<T> X = xf.view;
+        X.keep = keep_fp32(hybrid) ? 1 : 0;
+        return X;
+    }
     void forward(const void* f, void* F, hipStream_t st) override { forward_weighted(f, nullptr, 0, F, st); }
     // forward transform of the grid product f(R, x) wR[R * wstride]
-    void forward_weighted(const void* f, const T* wR, int wstride, void* F, hipStream_t st) {
-        const int M = 2 * model.B - 1;
+    void forward_weighted(const void* f, const T* wR, int wstride, void* F, hipStream_t st, bool hybrid = false) {
+        const XformDev<T> X = xform(hybrid);
         ensure(G, sizeof(cT<T>) * (size_t)g_elems(model.B, nx));
-        launch_fwd_ag<T>(xf.view, f, wR, wstride, G.p, st);
-        if (half_omega()) {  // the omega DFTs on half of the rows write the other half
-            launch_beta_fwd<T>(xf.view, G.p, F, st, false);
-            launch_omega_half<T>(xf.view, F, F, false, st);
+        launch_fwd_ag<T>(X, f, wR, wstride, G.p, st);
+        if (half_omega(X)) {  // the omega DFTs on half of the rows write the other half
+            launch_beta_fwd<T>(X, G.p, F, st, false);
+            launch_omega_half<T>(X, F, F, false, st);
         } else {
-            launch_beta_fwd<T>(xf.view, G.p, F, st);
-            launch_omega_dft<T>(xf.view, F, F, false, st);
+            launch_beta_fwd<T>(X, G.p, F, st);
+            launch_omega_dft<T>(X, F, F, false, st);
         }
         HPUP_HIP(hipGetLastError());
     }
-    void backward(const void* F, void* f, hipStream_t st) override {
-        const int M = 2 * model.B - 1;
+    void backward(const void* F, void* f, hipStream_t st) override { backward_as(F, f, st, false); }
+    void backward_as(const void* F, void* f, hipStream_t st, bool hybrid) {
+        const XformDev<T> X = xform(hybrid);
         ensure(G, sizeof(cT<T>) * (size_t)g_elems(model.B, nx));
         ensure(tmp, cbytes());
-        if (half_omega()) {  // the Hermitian part on half of the rows
-            launch_omega_half<T>(xf.view, F, tmp.p, true, st);
-            launch_beta_inv<T>(xf.view, tmp.p, G.p, st, false);
+        if (half_omega(X)) {  // the Hermitian part on half of the rows
+            launch_omega_half<T>(X, F, tmp.p, true, st);
+            launch_beta_inv<T>(X, tmp.p, G.p, st, false);
         } else {
-            launch_omega_dft<T>(xf.view, F, tmp.p, true, st);
-            launch_beta_inv<T>(xf.view, tmp.p, G.p, st);
+            launch_omega_dft<T>(X, F, tmp.p, true, st);
+            launch_beta_inv<T>(X, tmp.p, G.p, st);
         }
-        launch_inv_ag<T>(xf.view, G.p, f, st);
+        launch_inv_ag<T>(X, G.p, f, st);
         HPUP_HIP(hipGetLastError());
     }
     // omega DFTs of the transforms on half of the rows
-    bool half_omega() const { return model.B <= 32 && omega_half_ok(xf.view); }
+    bool half_omega(const XformDev<T>& X) const { return model.B <= 32 && omega_half_ok(X); }
     // MFMA kernels cover omega grids up to 32 points per axis, and up to 64 for
     // the reduced model (dim 2); larger grids use the LDS-tiled FMA kernels
     // (three passes).
@@ -781,9 +819,9 @@ template <class T> struct PlanT : PlanBase {
         HPUP_REQUIRE(F && f && nsteps >= 0, HPUP_ERR_ARG, "bad argument");
         for (int it = 0; it < nsteps; it++) {
             step(F, 1, st);
-            backward(F, f, st);
+            backward_as(F, f, st, true);
             reset_grid(f, f, model.dt, 0, st);
-            forward(f, F, st);
+            forward_weighted(f, nullptr, 0, F, st, true);
         }
     }
     void marginals(const void* f, const double* xg, std::vector<double>& hR, std::vector<double>& hG,

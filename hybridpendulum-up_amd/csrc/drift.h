@@ -121,6 +121,14 @@ template <class T> struct XformDev {
     // rows r <= B (angle), k < B (frequency)
     const T* agF;
     const T* agI;
+    // FP32 only: the grid's 64-bit figures (statistics, gradients) are taken from
+    // it, and its transforms keep the direct (alpha, gamma) stages and (k1, k2)
+    // DFTs, in whose rounding those figures stand, with these tables
+    int keep;
+    const cT<T>* twMB;  // [32][32] e^{i pi (r - (B-1)) t / B} for r < 2B-1, t < 2B, zero elsewhere, then its
+                        // transpose [t][r] (B <= 16)
+    const cT<T>* twNf;  // e^{-2 pi i t/N}, t in [0, N) (dim 2, N > 32)
+    const cT<T>* twNi;  // e^{+2 pi i t/N}
     const cT<T>* dftN;  // forward DFT matrix N x N (row-major [k][a]) e^{-2 pi i k a/N}
     const cT<T>* idftN; // inverse DFT matrix (1/N scaled) e^{+2 pi i k a/N}/N
     const T* omT;       // (k1, k2) DFT: cos then sin (2 pi k a / N), rows k <= N / 2, a <= N / 2 (entries a = 0 and
@@ -169,7 +177,7 @@ void launch_omega_dft(const XformDev<T>& X, const void* in, void* out, bool inve
 // inverse DFT of the Hermitian part (F_mn(k) + (-1)^(m-n) conj F_{-m,-n}(-k)) / 2;
 // the other rows of out are not written.
 template <class T> bool omega_half_ok(const XformDev<T>& X) {
-    return ((X.dim == 2 && X.N <= 64) || (X.dim == 3 && X.N <= 32 && X.bsF)) && X.omT && X.hrows;
+    return ((X.dim == 2 && X.N <= (X.keep ? 32 : 64)) || (X.dim == 3 && X.N <= 32 && X.bsF)) && X.omT && X.hrows;
 }
 template <class T>
 void launch_omega_half(const XformDev<T>& X, const void* in, void* out, bool inverse, hipStream_t st);

@@ -1,6 +1,7 @@
 // Omega DFTs of the transforms (the unnormalized DFT over the omega axes and
 // its inverse with 1/N per axis), on the rows of the compact coefficients:
-// k_slab_dft over (k1, k2) of each slab, k_axis_dft_mfma over k3.
+// k_slab_dft over (k1, k2) of each slab, k_axis_dft_mfma over k3.  FP32 grids with
+// XformDev::keep: k_slab_dft_chirp (N <= 32), k_slab_dft_fma (dim 2, N > 32).
 #include <algorithm>
 
 #include "drift.h"
@@ -21,6 +22,7 @@ namespace hpup {
 // on those rows only.
 enum OmegaRows {
     kRowsAll = 0,     // every row
+    kRowsHalf = 1,    // the half rows
     kRowsMirror = 2,  // the half rows, output written to the mirror rows too
     kRowsSym = 3      // the half rows, input taken as the Hermitian part
 };
@@ -441,6 +443,184 @@ __global__ __launch_bounds__(256) void k_axis_dft_mfma(const cT<T>* in, cT<T>* o
         }
 }
 
+// ------------------------------------- (k1, k2), FP32 with XformDev::keep --
+//
+// The (k1, k2) DFTs in the summation orders that FP32 grids behind 64-bit figures
+// keep (see the (alpha, gamma) stages of the same name in transform.hip):
+// Toeplitz products for N <= 32, direct sums beyond.  k_slab_dft takes 0.7 (N =
+// 30) and 0.15 (N = 60) of their time.
+constexpr int kPad = 34;
+
+// C X^T products of a 32 x 32 tile with three real products instead of four (Gauss):
+// P1 = Re C Re X, P2 = Im C Im X, P3 = (Re C + Im C)(Re X + Im X), and
+// C X = P1 - P2 + i (P3 - P1 - P2)
+template <class T> struct ToepGauss {
+    using MF = Mfma<T>;
+    using acc_t = typename MF::acc;
+    const ToepTab<T>* c;
+    int k2t, k1t, lr, lq, ks;  // ks: K = 4 steps that reach the data
+    // along k1: reduction over k = 4 u + lq
+    __device__ __forceinline__ void t1(const T* pr, const T* pi, cT<T>* out) const {
+        acc_t p1 = MF::zero(), p2 = MF::zero(), p3 = MF::zero();
+        const int row = (16 * k2t + lr) * kPad, b = 16 * k1t + lr + 32 - lq;
+#pragma unroll 4
+        for (int u = 0; u < ks; u++) {
+            const T xr = pr[row + 4 * u + lq], xi = pi[row + 4 * u + lq];
+            const cT<T> f = c->re_in[b - 4 * u];
+            p1 = MF::fma(xr, f.x, p1);
+            p2 = MF::fma(xi, f.y, p2);
+            p3 = MF::fma(xr + xi, f.x + f.y, p3);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) out[v] = cmk<T>(p1[v] - p2[v], p3[v] - p1[v] - p2[v]);
+    }
+    // along k2: reduction over k = ks lq + u
+    __device__ __forceinline__ void t2(const T* pr, const T* pi, cT<T>* out) const {
+        acc_t p1 = MF::zero(), p2 = MF::zero(), p3 = MF::zero();
+        const int col = 16 * k1t + lr, r0 = ks * lq, b = 16 * k2t + lr + 32 - ks * lq;
+#pragma unroll 4
+        for (int u = 0; u < ks; u++) {
+            const T xr = pr[(r0 + u) * kPad + col], xi = pi[(r0 + u) * kPad + col];
+            const cT<T> f = c->re_in[b - u];
+            p1 = MF::fma(f.x, xr, p1);
+            p2 = MF::fma(f.y, xi, p2);
+            p3 = MF::fma(f.x + f.y, xr + xi, p3);
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) out[v] = cmk<T>(p1[v] - p2[v], p3[v] - p1[v] - p2[v]);
+    }
+};
+
+// 2-D DFT over (k1, k2) of N x N slabs of in, times `scale`, into out (in
+// place when they are equal: a slab is read whole before it is written, and
+// the mirror rows a kRowsMirror pass writes are read by no other slab).  Slab
+// sl is row sl / nz at k3 = sl % nz (rows from the half list).
+template <class T, int MODE>
+__global__ __launch_bounds__(256) void k_slab_dft_chirp(const cT<T>* in, cT<T>* out, const cT<T>* __restrict__ bs,
+                                                       int N, T scale, int nslab, int nz, const int32_t* __restrict__ hr) {
+    __shared__ T pa_re[32 * kPad], pa_im[32 * kPad], pb_re[32 * kPad], pb_im[32 * kPad];
+    __shared__ ToepTab<T> tab;
+    __shared__ cT<T> pk[32];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int k2t = w >> 1, k1t = w & 1, lr = lane & 15, lq = lane >> 4;
+    tab.fill(bs, tid);
+    if (tid < 32) pk[tid] = bs[64 + tid];
+    __syncthreads();
+    // reductions trimmed to the N data points (plane A is zero beyond N along
+    // k1; plane B's rows k2 >= N are zero through p_k2 = 0)
+    ToepGauss<T> gm{&tab, k2t, k1t, lr, lq, (N + 3) / 4};
+    const int NN = N * N;
+    const int k1 = 16 * k1t + lr;
+    const cT<T> p1 = pk[k1];
+    // slab sl: its base, and for the mirror modes the mirror slab's (at -k3)
+    auto slab = [&](int sl, int64_t& b, int64_t& bm, bool& neg, bool& self) {
+        const int i = sl / nz, k3 = sl - i * nz;
+        const HalfRow h = half_row(hr, i);
+        b = ((int64_t)h.r * nz + k3) * NN;
+        bm = ((int64_t)h.rm * nz + (k3 == 0 ? 0 : nz - k3)) * NN;
+        neg = h.neg;
+        self = h.rm == h.r;
+    };
+    // the slab's four elements per thread (clamped in-range loads; with the
+    // mirror slab's element at (-k2, -k1) for kRowsSym); the next slab's are
+    // loaded while this one is transformed
+    cT<T> x[4], y[4];
+    auto load = [&](int sl) {
+        int64_t b, bm;
+        bool ng, sf;
+        slab(sl, b, bm, ng, sf);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int idx = tid + 256 * i, a2 = idx >> 5, a1 = idx & 31;
+            const bool ok = a2 < N && a1 < N;
+            x[i] = in[b + (ok ? a2 * N + a1 : 0)];
+            if (MODE == kRowsSym) {
+                const int m2 = a2 == 0 ? 0 : N - a2, m1 = a1 == 0 ? 0 : N - a1;
+                y[i] = in[bm + (ok ? m2 * N + m1 : 0)];
+            }
+        }
+    };
+    if ((int)blockIdx.x < nslab) load(blockIdx.x);
+    for (int sl = blockIdx.x; sl < nslab; sl += gridDim.x) {
+        int64_t b, bm;
+        bool neg, self;
+        slab(sl, b, bm, neg, self);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {  // pre-chirp along k1, zero outside the slab
+            const int idx = tid + 256 * i, a2 = idx >> 5, a1 = idx & 31;
+            cT<T> u = x[i];
+            if (MODE == kRowsSym) {
+                const cT<T> c = sconj<T>(y[i], neg);
+                u = cmk<T>(T(0.5) * (u.x + c.x), T(0.5) * (u.y + c.y));
+            }
+            const cT<T> v = a2 < N && a1 < N ? cmul<T>(u, pk[a1]) : czero<T>();
+            pa_re[a2 * kPad + a1] = v.x;
+            pa_im[a2 * kPad + a1] = v.y;
+        }
+        __syncthreads();  // plane A complete; plane B of the previous slab consumed
+        // another slab: no overlap with this slab's output, also in place
+        if (sl + (int)gridDim.x < nslab) load(sl + gridDim.x);
+        cT<T> R[4];
+        gm.t1(pa_re, pa_im, R);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {  // along k1 done; pre-chirp along k2 (p = 0 in the padding)
+            const int k2 = 16 * k2t + Mfma<T>::orow(lq, v);
+            const cT<T> yv = cmul<T>(cmul<T>(R[v], p1), pk[k2]);
+            pb_re[k2 * kPad + k1] = yv.x;
+            pb_im[k2 * kPad + k1] = yv.y;
+        }
+        __syncthreads();  // plane B complete; plane A consumed
+        gm.t2(pb_re, pb_im, R);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            const int k2 = 16 * k2t + Mfma<T>::orow(lq, v);
+            if (k1 < N && k2 < N) {
+                const cT<T> z = cscale<T>(cmul<T>(R[v], pk[k2]), scale);
+                out[b + k2 * N + k1] = z;
+                if (MODE == kRowsMirror && !self)
+                    out[bm + (k2 == 0 ? 0 : N - k2) * N + (k1 == 0 ? 0 : N - k1)] = sconj<T>(z, neg);
+            }
+        }
+    }
+}
+
+// In-place 2-D DFT over (k1, k2) of every N x N slab, twiddle-indexed.
+template <class T>
+__global__ __launch_bounds__(1024) void k_slab_dft_fma(cT<T>* __restrict__ F, const cT<T>* __restrict__ twN, int N, T scale) {
+    extern __shared__ char smem_raw[];
+    const int NN = N * N;
+    cT<T>* sA = reinterpret_cast<cT<T>*>(smem_raw);
+    cT<T>* sB = sA + NN;
+    cT<T>* tw = sB + NN;
+    const int64_t base = (int64_t)blockIdx.x * NN;
+    for (int e = threadIdx.x; e < NN; e += blockDim.x) sA[e] = F[base + e];
+    for (int e = threadIdx.x; e < N; e += blockDim.x) tw[e] = twN[e];
+    __syncthreads();
+    for (int e = threadIdx.x; e < NN; e += blockDim.x) {
+        const int k1 = e % N, k2 = e / N;
+        cT<T> acc = czero<T>();
+        int t = 0;
+        for (int a = 0; a < N; a++) {
+            cfma<T>(acc, tw[t], sA[k2 * N + a]);
+            t += k1;
+            if (t >= N) t -= N;
+        }
+        sB[e] = acc;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < NN; e += blockDim.x) {
+        const int k1 = e % N, k2 = e / N;
+        cT<T> acc = czero<T>();
+        int t = 0;
+        for (int a = 0; a < N; a++) {
+            cfma<T>(acc, tw[t], sB[a * N + k1]);
+            t += k2;
+            if (t >= N) t -= N;
+        }
+        F[base + e] = cscale<T>(acc, scale);
+    }
+}
+
 // ---------------------------------------------------------- launchers ---
 
 // (k1, k2) DFT of nslab slabs.  XC slabs per block: as many as fill the four
@@ -502,6 +682,15 @@ static void axis_half(const XformDev<T>& X, const void* in, void* out, const cT<
                        inner, scale, X.hrows);
 }
 
+template <class T, int MODE>
+static void slab_keep(const XformDev<T>& X, const void* in, void* out, bool inverse, T scale, hipStream_t st) {
+    const int N = X.N, nz = X.dim == 3 ? N : 1;
+    const int64_t nslab = X.nhalf * nz;
+    HPUP_REQUIRE(nslab < ((int64_t)1 << 31), HPUP_ERR_UNSUPPORTED, "slab DFT: too many slabs");
+    const unsigned grid = (unsigned)std::min<int64_t>(nslab, 4096);
+    hipLaunchKernelGGL((k_slab_dft_chirp<T, MODE>), dim3(grid), dim3(256), 0, st, (const cT<T>*)in, (cT<T>*)out,
+                       inverse ? X.bsI : X.bsF, N, scale, (int)nslab, nz, X.hrows);
+}
 
 template <class T>
 void launch_omega_half(const XformDev<T>& X, const void* in, void* out, bool inverse, hipStream_t st) {
@@ -513,11 +702,25 @@ void launch_omega_half(const XformDev<T>& X, const void* in, void* out, bool inv
     const int64_t nslab = X.nhalf * nz;
     if (!inverse) {
         HPUP_REQUIRE(in == out, HPUP_ERR_ARG, "forward half-row omega DFT runs in place");
+        if constexpr (sizeof(T) == 4) {
+            if (X.keep) {
+                if (X.dim == 2) return slab_keep<T, kRowsMirror>(X, in, out, false, s2, st);
+                slab_keep<T, kRowsHalf>(X, in, out, false, s2, st);
+                return axis_half<T, kRowsMirror>(X, out, out, bs, s3, st);
+            }
+        }
         slab_dft<T>(X, in, out, nslab, nz, false, s2, X.hrows, false, X.dim == 2, st);
         if (X.dim == 3) axis_half<T, kRowsMirror>(X, out, out, bs, s3, st);
         return;
     }
     HPUP_REQUIRE(in != out, HPUP_ERR_ARG, "inverse half-row omega DFT runs out of place");
+    if constexpr (sizeof(T) == 4) {
+        if (X.keep) {
+            if (X.dim == 2) return slab_keep<T, kRowsSym>(X, in, out, true, s2, st);
+            axis_half<T, kRowsSym>(X, in, out, bs, s3, st);
+            return slab_keep<T, kRowsHalf>(X, out, out, true, s2, st);
+        }
+    }
     if (X.dim == 3) {
         axis_half<T, kRowsSym>(X, in, out, bs, s3, st);
         slab_dft<T>(X, out, out, nslab, nz, true, s2, X.hrows, false, false, st);
@@ -539,6 +742,19 @@ void launch_omega_dft(const XformDev<T>& X, const void* in, void* out, bool inve
         return;
     }
     const T s2 = inverse ? T(1) / T(N * N) : T(1);
+    if constexpr (sizeof(T) == 4) {
+        if (X.keep && X.dim == 2 && N > 32) {
+            const int NN = N * N;
+            HPUP_REQUIRE(NN <= 4096, HPUP_ERR_UNSUPPORTED, "omega grid larger than 64 per axis");
+            if (in != out)
+                HPUP_HIP(hipMemcpyAsync(out, in, sizeof(cT<T>) * (size_t)(X.nrc * X.nx), hipMemcpyDeviceToDevice, st));
+            const size_t sh = sizeof(cT<T>) * (2 * (size_t)NN + N);
+            allow_lds((const void*)k_slab_dft_fma<T>, sh);
+            hipLaunchKernelGGL(k_slab_dft_fma<T>, dim3((unsigned)X.nrc), dim3(1024), sh, st, (cT<T>*)out,
+                               inverse ? X.twNi : X.twNf, N, s2);
+            return;
+        }
+    }
     if (X.dim == 3 && N <= 32) {
         axis_all<T>(X, in, out, inverse, st);
         slab_dft<T>(X, out, out, X.nrc * N, N, inverse, s2, nullptr, false, false, st);

@@ -1415,6 +1415,162 @@ __global__ __launch_bounds__(NT) void k_inv_ag_q60(XformDev<T> X, const cT<T>* _
     store_f_rows<T, XC, NT, n2>(so, f, j, x0, nx);
 }
 
+// ------------------------- (alpha, gamma) stages, FP32 grids with XformDev::keep
+//
+// Direct DFTs for B <= 16 in one fixed summation order.  The MFMA stages above are
+// faster (B = 10: 1.9x) and no less accurate, but round FP32 differently, and
+// 64-bit figures that a program takes from an FP32 grid (get_stat's moments after
+// a hybrid step, the restitution gradient) would move by 1e-7 with them: those
+// grids stay on these kernels.
+//
+// Work items hold one row of the stage's input in registers and sweep a
+// frequency x angle twiddle table E[r][t] = e^{i pi (r - lmax) t / B}, zero
+// padded to 32 x 32, so every loop runs a fixed 32 steps without guards.  The
+// table row and column of each step depend only on loop counters and on the
+// wave's part of the block, so the table is read through the scalar cache
+// (uniform addresses) instead of LDS.  A stage whose work items fill only part
+// of the block splits its output range over wave-aligned parts.
+
+constexpr int kAgMax = 32;  // 2B limit
+
+// table in the constant address space: uniform indices become scalar loads
+template <class T> using cTab = __attribute__((address_space(4))) const T*;
+template <class T> __device__ __forceinline__ cT<T> etw(cTab<T> e, int i) { return cmk<T>(e[2 * i], e[2 * i + 1]); }
+
+// tasks of a stage -> parts of the block: <= 64 -> 4, <= 128 -> 2, else 1
+__device__ __forceinline__ int stage_parts(int T) { return T <= 64 ? 4 : (T <= 128 ? 2 : 1); }
+
+template <class T, int XC>
+__global__ __launch_bounds__(256) void k_fwd_ag_r(XformDev<T> X, const T* __restrict__ f, const T* __restrict__ wR,
+                                                  int wstride, cT<T>* __restrict__ G, int nxc) {
+    extern __shared__ char smem_raw[];
+    const int B = X.B, n2 = 2 * B, lmax = B - 1, M = 2 * B - 1;
+    const int rp = n2 + 1;                                   // padded row of sf
+    T* sf = reinterpret_cast<T*>(smem_raw);                  // [xl][g][a]  XC*n2*rp
+    cT<T>* sH = reinterpret_cast<cT<T>*>(smem_raw);          // [m>=0][g][xl], aliases sf
+    const cTab<T> E = (cTab<T>)(const T*)X.twMB;
+    int j;
+    int64_t x0;
+    ag_block<T>(XC, nxc, n2, j, x0);
+    const int64_t nx = X.nx;
+    const int tid = threadIdx.x;
+    const int64_t n2c = (int64_t)n2 * n2 * n2;
+    for (int i = tid; i < XC * n2 * n2; i += 256) {
+        const int xl = i / (n2 * n2), g = (i / n2) % n2, a = i % n2;
+        const int64_t x = x0 + xl;
+        const int64_t iR = a + (int64_t)n2 * (j + (int64_t)n2 * g);
+        T v = x < nx ? f[iR + n2c * x] : T(0);
+        if (wR) v *= wR[iR * wstride];  // transform of the product f(R, x) w(R)
+        sf[(xl * n2 + g) * rp + a] = v;
+    }
+    __syncthreads();
+    // alpha DFT, m >= 0: H[m][g] = sum_a f[a] e^{+i m alpha_a}; item (g, xl)
+    {
+        const int TA = n2 * XC, SA = stage_parts(TA), PA = 256 / SA;
+        const int part = __builtin_amdgcn_readfirstlane(tid / PA), task = tid % PA;
+        const bool act = task < TA;
+        const int g = task / XC, xl = task % XC;
+        T row[kAgMax];
+#pragma unroll
+        for (int a = 0; a < kAgMax; a++) row[a] = (act && a < n2) ? sf[(xl * n2 + g) * rp + a] : T(0);
+        __syncthreads();  // sH overwrites sf
+        for (int m = part; m < B; m += SA) {
+            const cTab<T> e = E + 2 * (m + lmax) * kAgMax;
+            cT<T> acc = czero<T>();
+#pragma unroll
+            for (int a = 0; a < kAgMax; a++) {
+                const cT<T> tw = etw<T>(e, a);
+                acc.x = fma(row[a], tw.x, acc.x);
+                acc.y = fma(row[a], tw.y, acc.y);
+            }
+            if (act) sH[(m * n2 + g) * XC + xl] = acc;
+        }
+    }
+    __syncthreads();
+    // gamma DFT: G[m][n] = sum_g H[m][g] e^{+i n gamma_g}, G[-m][-n] = conj; item (m, xl)
+    {
+        const int TB = B * XC, SB = stage_parts(TB), PB = 256 / SB;
+        const int part = __builtin_amdgcn_readfirstlane(tid / PB), task = tid % PB;
+        const bool act = task < TB;
+        const int m = task / XC, xl = task % XC;
+        const int64_t x = x0 + xl;
+        cT<T> h[kAgMax];
+#pragma unroll
+        for (int g = 0; g < kAgMax; g++) h[g] = (act && g < n2) ? sH[(m * n2 + g) * XC + xl] : czero<T>();
+        const bool st = act && x < nx;
+        cT<T>* Gx = G + g_off(B, 0, j, min<int64_t>(x, nx - 1));
+        for (int ni = part; ni < M; ni += SB) {
+            const cTab<T> e = E + 2 * ni * kAgMax;
+            cT<T> acc = czero<T>();
+#pragma unroll
+            for (int g = 0; g < kAgMax; g++) cfma<T>(acc, h[g], etw<T>(e, g));
+            if (st) put_g_half<T>(Gx, B, m, ni, acc);
+        }
+    }
+}
+
+template <class T, int XC>
+__global__ __launch_bounds__(256) void k_inv_ag_r(XformDev<T> X, const cT<T>* __restrict__ G, T* __restrict__ f,
+                                                  int nxc) {
+    extern __shared__ char smem_raw[];
+    const int B = X.B, n2 = 2 * B, M = 2 * B - 1;
+    cT<T>* sH = reinterpret_cast<cT<T>*>(smem_raw);  // [m][g][xl]
+    const cTab<T> ET = (cTab<T>)(const T*)X.twMB + 2 * kAgMax * kAgMax;  // [t][r]
+    int j;
+    int64_t x0;
+    ag_block<T>(XC, nxc, n2, j, x0);
+    const int64_t nx = X.nx;
+    const int tid = threadIdx.x;
+    // H[m][g] = sum_n G[m][n] e^{-i n gamma_g}; item (m, xl) holds its G row
+    {
+        const int T1 = M * XC, S1 = stage_parts(T1), P1 = 256 / S1;
+        const int part = __builtin_amdgcn_readfirstlane(tid / P1), task = tid % P1;
+        const bool act = task < T1;
+        const int mi = task / XC, xl = task % XC;
+        const int64_t x = x0 + xl;
+        const bool ld = act && x < nx;
+        // clamped, branch-free loads; invalid entries are zeroed after the load
+        const cT<T>* Hx = G + h_base(B, j, min<int64_t>(x, nx - 1));
+        cT<T> gr[kAgMax];
+#pragma unroll
+        for (int ni = 0; ni < kAgMax; ni++) {
+            const cT<T> v = get_h<T>(Hx, B, min(mi, M - 1), min(ni, M - 1));
+            gr[ni] = (ld && ni < M) ? v : czero<T>();
+        }
+        for (int g = part; g < n2; g += S1) {
+            const cTab<T> e = ET + 2 * g * kAgMax;
+            cT<T> acc = czero<T>();
+#pragma unroll
+            for (int ni = 0; ni < kAgMax; ni++) cfma<T>(acc, gr[ni], cconj<T>(etw<T>(e, ni)));
+            if (act) sH[(mi * n2 + g) * XC + xl] = acc;
+        }
+    }
+    __syncthreads();
+    // f[a][g] = Re sum_m H[m][g] e^{-i m alpha_a}; item (g, xl) holds its H column
+    {
+        const int T2 = n2 * XC, S2 = stage_parts(T2), P2 = 256 / S2;
+        const int part = __builtin_amdgcn_readfirstlane(tid / P2), task = tid % P2;
+        const bool act = task < T2;
+        const int g = task / XC, xl = task % XC;
+        const int64_t x = x0 + xl;
+        const bool st = act && x < nx;
+        cT<T> hr[kAgMax];
+#pragma unroll
+        for (int mi = 0; mi < kAgMax; mi++) hr[mi] = (act && mi < M) ? sH[(mi * n2 + g) * XC + xl] : czero<T>();
+        T* fo = f + (int64_t)n2 * (j + (int64_t)n2 * (g + (int64_t)n2 * min<int64_t>(x, nx - 1)));
+        for (int a = part; a < n2; a += S2) {
+            const cTab<T> e = ET + 2 * a * kAgMax;
+            T acc = T(0);
+#pragma unroll
+            for (int mi = 0; mi < kAgMax; mi++) {
+                const cT<T> tw = etw<T>(e, mi);  // Re(h conj(tw))
+                acc = fma(hr[mi].x, tw.x, fma(hr[mi].y, tw.y, acc));
+            }
+            if (st) fo[a] = acc;
+        }
+    }
+}
+
 // ---------------------------------------------------------- launchers -----
 
 static int pick_xc(size_t per_x, size_t budget, int64_t nx) {
@@ -1564,7 +1720,19 @@ void launch_fwd_ag(const XformDev<T>& X, const void* f, const void* wR, int wstr
             fwd_ag_q60<T, kQ60FwdXC32, (120 * kQ60FwdXC32 + 63) / 64 * 64>(X, f, wR, wstride, G, st);
         return;
     }
-    if (X.B <= 32) {  // K = B + 1 angles in steps of 4, rows m, n < B in tiles of 16
+    if constexpr (sizeof(T) == 4) {
+        if (X.keep && n2 <= kAgMax) {
+            constexpr int XC = 8;
+            const int nxc = (int)((X.nx + XC - 1) / XC);
+            HPUP_REQUIRE((int64_t)nxc * n2 < (1ll << 31), HPUP_ERR_UNSUPPORTED, "omega grid too large");
+            const size_t sh = std::max(sizeof(T) * XC * n2 * (n2 + 1), sizeof(cT<T>) * X.B * n2 * XC);
+            allow_lds((const void*)k_fwd_ag_r<T, XC>, sh);
+            hipLaunchKernelGGL((k_fwd_ag_r<T, XC>), dim3((unsigned)(nxc * n2)), dim3(256), sh, st, X, (const T*)f,
+                               (const T*)wR, wstride, (cT<T>*)G, nxc);
+            return;
+        }
+    }
+    if (X.B <= 32 && !X.keep) {  // K = B + 1 angles in steps of 4, rows m, n < B in tiles of 16
         switch (X.B / 4) {
         case 0: return fwd_ag_mfma<T, 1, 1>(X, f, wR, wstride, G, st);
         case 1: return fwd_ag_mfma<T, 1, 2>(X, f, wR, wstride, G, st);
@@ -1645,7 +1813,19 @@ void launch_inv_ag(const XformDev<T>& X, const void* G, void* f, hipStream_t st)
         else inv_ag_q60<T, kQ60InvXC32, (240 * kQ60InvXC32 + 63) / 64 * 64>(X, G, f, st);
         return;
     }
-    if (X.B <= 32) {  // K = B frequencies in steps of 4, rows a, g <= B in tiles of 16
+    if constexpr (sizeof(T) == 4) {
+        if (X.keep && n2 <= kAgMax) {
+            constexpr int XC = 8;
+            const int nxc = (int)((X.nx + XC - 1) / XC);
+            HPUP_REQUIRE((int64_t)nxc * n2 < (1ll << 31), HPUP_ERR_UNSUPPORTED, "omega grid too large");
+            const size_t sh = sizeof(cT<T>) * M * n2 * XC;
+            allow_lds((const void*)k_inv_ag_r<T, XC>, sh);
+            hipLaunchKernelGGL((k_inv_ag_r<T, XC>), dim3((unsigned)(nxc * n2)), dim3(256), sh, st, X, (const cT<T>*)G,
+                               (T*)f, nxc);
+            return;
+        }
+    }
+    if (X.B <= 32 && !X.keep) {  // K = B frequencies in steps of 4, rows a, g <= B in tiles of 16
         switch ((X.B + 3) / 4) {
         case 1: return inv_ag_mfma<T, 1, 1>(X, G, f, st);
         case 2: return inv_ag_mfma<T, 1, 2>(X, G, f, st);
