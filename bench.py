@@ -43,10 +43,11 @@ def kernel_flops(name, B, N):
     acts on a (r, k3) slab of N^2 points; kappa_p = c0 + i (real circulant) for
     the coordinate ramps of this workload, so one application is two real
     N^3-MAC products (4 N^3 FLOPs) plus an axis sum.  The fused kernel applies
-    four per slab (T1 F, T2 F, T1 V1, T2 V2), the axis-3 kernel one; nRc =
+    four per slab (T1 F, T2 F, T1 V1, T2 V2), the axis-3 kernel one; the folded
+    kernel applies the four to parity planes, half the products of each; nRc =
     B(2B-1)(2B+1)/3 rotation rows, N slabs each."""
     nrc = B * (2 * B - 1) * (2 * B + 1) // 3
-    per = {"k_drift_fused": 4, "k_axis3_mfma": 1}.get(name, 0)
+    per = {"k_drift_fused": 4, "k_drift_fold": 2, "k_axis3_mfma": 1}.get(name, 0)
     return per * 4.0 * N ** 3 * nrc * N
 
 ERR_STEPS = 200  # the workload's step count, at which the precision gate is taken

@@ -169,7 +169,7 @@ template <class T> struct XformTables {
 };
 
 template <class T> struct DriftTables {
-    DevBuf cg_src, cg_coef, u_src, u_coef, e3, kap, kc, kd, M3, mix_src, mix_coef;
+    DevBuf cg_src, cg_coef, u_src, u_coef, e3, kap, kc, kd, M3, mix_src, mix_coef, mix_order;
     DriftDev<T> view{};
     MixDev<T> mix{};
     bool smix = false;
@@ -242,6 +242,16 @@ template <class T> struct DriftTables {
         }
         mix_src = upload(src);
         mix_coef = upload(cast_vec<T>(coef));
+        // m, then n, then l: the rows that share sources (l +- 1, n +- 1 at the
+        // same m) lie within 2 (B - max(|m|, |n|)) of each other
+        std::vector<int32_t> order;
+        order.reserve(nrc);
+        for (int m = -(s.B - 1); m < s.B; m++)
+            for (int n = -(s.B - 1); n < s.B; n++)
+                for (int l = std::max(std::abs(m), std::abs(n)); l < s.B; l++)
+                    order.push_back((int32_t)ridx_B(s.B, l, m, n));
+        mix_order = upload(order);
+        mix.order = mix_order.as<int32_t>();
         mix.TS = TS;
         mix.src = mix_src.as<int32_t>();
         mix.coef = mix_coef.as<cT<T>>();
@@ -286,6 +296,7 @@ template <class T> struct DriftTables {
         for (int i = 0; i < 9; i++) v.G[i] = (T)s.G[i];
         for (int i = 0; i < 3; i++) { v.b[i] = (T)s.b[i]; v.gyro[i] = (T)s.gyro[i]; v.c0[i] = (T)s.c0[i]; }
         v.ramp = s.ramp ? 1 : 0;
+        v.odd = s.odd ? 1 : 0;
         v.smix = smix ? 1 : 0;
         v.adj = s.adj ? 1 : 0;
         v.has_gyro = s.has_gyro ? 1 : 0;

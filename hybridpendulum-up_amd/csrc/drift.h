@@ -14,6 +14,12 @@ size_t lds_limit();
 // Raises a kernel's dynamic-LDS cap when one launch needs more than 64 KB.
 void allow_lds(const void* kernel, size_t bytes);
 
+// Workgroups of a persistent kernel: enough to fill every CU at the kernel's
+// occupancy, never more than there is work, a multiple of 8 (whole workgroups
+// per XCD) from 8 on.  The resident count is looked up once per (kernel, device,
+// LDS size).
+unsigned persistent_blocks(const void* kernel, int64_t nwork, int threads, size_t lds);
+
 template <class T> struct DriftDev {
     int B, dim, N;
     int64_t nx, nrc;
@@ -35,6 +41,7 @@ template <class T> struct DriftDev {
     const cT<T>* grav[3];
     // every kap_p = c0[p] + i (real circulant): the real-circulant path
     int ramp;
+    int odd;  // ... and the real circulants are odd
     T c0[3];
     // structured mixing coefficients: -i CG_1 real, -i CG_2 imaginary,
     // CG_3 zero, u_1 imaginary, u_2 real (the pendulum models)
@@ -76,12 +83,20 @@ template <class T> struct MixDev {
     int TS;
     const int32_t* src;   // nrc*TS, -1 padded
     const cT<T>* coef;    // nrc*TS*(dim+2)
+    const int32_t* order; // the nrc rows in the order the folded kernel walks them
 };
 
 // bf16x3: circulants as 3xBF16 split products (FP32 storage only)
 template <class T>
 void launch_drift_fused(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0,
                         void* Fout, void* ACC, const StageCoef<T>& sc, bool bf16x3, hipStream_t st);
+// the parity-folded kernel, taken where drift_fold_ok (odd real circulants,
+// structured mixing, forward operator; the size rule is at its definition), with
+// no grid gravity and no stage sums
+template <class T> bool drift_fold_ok(const DriftDev<T>& D);
+template <class T>
+void launch_drift_fold(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0,
+                       void* Fout, const StageCoef<T>& sc, hipStream_t st);
 // name of the kernel launch_drift_fused runs for D (grav: density-form gravity)
 template <class T> const char* drift_fused_name(const DriftDev<T>& D, bool grav, bool bf16x3);
 // out = T3 in; scaled: out = T3 [(e3[r] - i b3 kc(k3)) in] (the 3-D adjoint's

@@ -1,0 +1,489 @@
+// Parity-folded drift kernel for omega grids up to 30 points per axis (the
+// forward operator of the pendulum models: real circulants, structured mixing).
+//
+// k_drift_fold evaluates the derivative of the (r, k3) slabs it visits with the
+// integrator epilogue, as k_drift_fused does (see drift_mfma.hip for the terms):
+//   dF = T1 V1 + T2 V2 + b1 c1 T1 F + b2 c2 T2 F + W,
+//   V1 = -U1 F - a2 c2 Z3 - a3 c3 T2 F,  V2 = -U2 F - a1 c1 Z3,
+//   W  = -sum_p c_p CG_p F + D F + (e3 + b3 c3) Z3,   c_p = i kc_p,
+// with T_p = c0 1 1^T + i K_p, K_p real and antisymmetric (kappa_p(-d) = -kappa_p(d)).
+// A thread owns the four elements (+-i1, +-i2), i1, i2 = 0..H = N/2, so the
+// sums and differences over each axis' sign (even and odd parts) are formed in
+// its registers.  On those parts K_p maps even to odd and back, and so does a
+// multiplication by kc_p: every product is a real (H + 1) x (H + 1) matrix on one
+// parity plane, a quarter of the full circulant, and N = 30 fills the 16 x 16
+// matrix instruction exactly.  With x' = (x(+) +- x(-)) / 2 per axis and planes
+// holding 4 x' (plain sums):
+//   (K x)'_e[k] = sum_a (kappa[k-a] - kappa[k+a]) x'_o[a]                  0 < a < H
+//   (K x)'_o[k] = sum_a (kappa[k-a] + kappa[k+a]) x'_e[a]  (kappa[k-a] at a = 0, H)
+//   (1 1^T x)'_e[k] = sum_a 2 x'_e[a]                       (x'_e at a = 0, H)
+//   (kc x)'_e = kc x'_o, (kc x)'_o = kc x'_e.
+// Wave w = p1 + 2 p2 produces plane (p1, p2) of everything but W from the LDS
+// planes of F, V1 and V2.  The matrices' operands stay in its registers, every
+// LDS address is a register plus an immediate, and an axis sum is folded over a
+// lane's own points before one matrix instruction adds it: the unfolded kernels
+// spend most of their vector instructions on table reads, axis sums, lane
+// permutes and addresses.
+//
+// What bounds it: no single unit (B = 15, N = 30, FP32: matrix pipe 24 %, vector
+// units 32 %, tag lookups 60 %, HBM 75 % of a copy's rate).  The six gathered
+// source rows cost 0.28 of 1.37 ms, the streams alone 0.83 ms.  Against
+// k_drift_fused / k_drift_fused_c (ms per launch, average of a step's four):
+//   B = 15, N = 30: FP32 1.63 -> 1.37, FP64 3.00 -> 2.48;  B = 30, N = 20, FP32: 5.54 -> 4.04.
+// Tried and not kept: the slab in its natural order with 16-byte loads and the
+// folding in LDS (FP64 N = 30: 2.80, FP32 N = 20: 4.63), mixing tables prefetched
+// through LDS (FP32 1.57), three waves per SIMD in FP64 (spills, 3.08).
+#include "drift.h"
+#include "kernels_common.h"
+#include "mfma.h"
+
+namespace hpup {
+
+template <class T> using kc_ptr = __attribute__((address_space(4))) const T*;
+template <class T> __device__ __forceinline__ kc_ptr<T> as_const(const T* p) { return (kc_ptr<T>)p; }
+
+template <class P> __device__ __forceinline__ P* at_b(P* p, unsigned ob) {
+    using C = typename std::conditional<std::is_const<P>::value, const char, char>::type;
+    return reinterpret_cast<P*>(reinterpret_cast<C*>(p) + ob);
+}
+// data touched once per launch: FP64 streams it (FP32 measures the same either way)
+template <class T> __device__ __forceinline__ cT<T> ld_once(const cT<T>* p) {
+    if constexpr (sizeof(T) == 8) return ld_stream<T>(p);
+    else return *p;
+}
+template <class T> __device__ __forceinline__ void st_once(cT<T>* p, cT<T> v) {
+    if constexpr (sizeof(T) == 8) st_stream<T>(p, v);
+    else *p = v;
+}
+
+// (x0, x1, x2, x3) at signs (+,+), (-,+), (+,-), (-,-) <-> planes ee, oe, eo, oo
+// (even/odd in axis 1, then 2): the same sums both ways
+template <class T> __device__ __forceinline__ void parity4(const cT<T>* x, cT<T>* y) {
+    const cT<T> s0 = cadd<T>(x[0], x[1]), d0 = csub<T>(x[0], x[1]);
+    const cT<T> s1 = cadd<T>(x[2], x[3]), d1 = csub<T>(x[2], x[3]);
+    y[0] = cadd<T>(s0, s1);
+    y[1] = cadd<T>(d0, d1);
+    y[2] = csub<T>(s0, s1);
+    y[3] = csub<T>(d0, d1);
+}
+
+// waves per SIMD: FP32 fits 128 registers, FP64 needs more than three allow
+template <class T> constexpr int fold_waves() { return sizeof(T) == 4 ? 4 : 2; }
+
+// XS: slabs (consecutive k3 of one row, which share the mixing sources and
+// coefficients) a workgroup visits together; KS: K = 4
+// steps over the H + 1 points of an axis
+template <class T, int DIM, int KS, int XS>
+__global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T> D, MixDev<T> MX, const cT<T>* Fin,
+                                                                     const cT<T>* __restrict__ Z3, const cT<T>* F0,
+                                                                     cT<T>* Fout, StageCoef<T> sc,
+                                                                     int ngroup) {
+    using MF = Mfma<T>;
+    using acc_t = typename MF::acc;
+    constexpr int NC = DIM + 2;
+    // FP64: the next slab's own elements are loaded before this one's products
+    // (N = 30: 2.55 -> 2.48 ms; FP32, four waves per SIMD instead of two, gains
+    // nothing at N = 30 and loses 14 % at N = 20, which spills)
+    constexpr bool AHEAD = sizeof(T) == 8;
+    constexpr int MB = 2;  // source rows whose loads are issued together
+    extern __shared__ __align__(16) char smem_fold[];
+    const int N = D.N, NN = N * N, H = N / 2, H1 = H + 1;
+    constexpr int HP = 4 * KS, RS = HP + 1, PL = HP * RS;  // a plane: H1 x H1 points in HP x RS, zero beyond
+    const int nz = DIM == 3 ? N : 1;
+    cT<T>* pF = reinterpret_cast<cT<T>*>(smem_fold);  // [XS][4][HP][RS]; the result planes in the end
+    cT<T>* pV1 = pF + XS * 4 * PL;
+    cT<T>* pV2 = pV1 + XS * 4 * PL;
+    __shared__ T skc[32], skd[32];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lq = lane >> 4;
+    for (int i = tid; i < 3 * XS * 4 * PL; i += 256) pF[i] = czero<T>();
+    if (tid < N) {
+        skc[tid] = D.kc[tid];
+        skd[tid] = D.kd[tid];
+    }
+
+    // ---- this wave's matrices (plane (p1, p2)), entry [out lr][in 4 s + lq]
+    const int p1 = w & 1, p2 = w >> 1;
+    T m1[KS], m2[KS], d1[KS], d2[KS], ws[KS], rr1, rr2;
+    {
+        auto mats = [&](const cT<T>* kap, int p, T c0, T b, T* m, T* d, T& rr) {
+            auto K = [&](int j) { return kap[((j % N) + N) % N].y; };
+            const T kco = lr <= H ? D.kc[lr] : T(0);
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                const int a = 4 * s + lq;
+                const bool in = a <= H, self = a == 0 || a == H, oself = lr == 0 || lr == H;
+                T oe = T(0), eo = T(0);  // even -> odd, odd -> even
+                if (in && lr <= H) {
+                    const T km = K(lr - a), kp = K(lr + a);
+                    oe = oself ? T(0) : self ? km : km + kp;
+                    eo = self ? T(0) : km - kp;
+                }
+                oe *= T(0.25);
+                eo *= T(0.25);
+                m[s] = p ? oe : eo;               // K into this plane's parity
+                d[s] = -b * kco * (p ? eo : oe);  // b c (i K): K to the other parity and kc back
+                ws[s] = !in ? T(0) : self ? T(0.25) : T(0.5);  // the axis sum's weights
+            }
+            rr = lr <= H ? c0 * (p ? b * kco : T(1)) : T(0);
+        };
+        mats(D.kap, p1, D.c0[0], D.b[0], m1, d1, rr1);
+        mats(D.kap + N, p2, D.c0[1], D.b[1], m2, d2, rr2);
+    }
+
+    // ---- this thread's elements
+    const int HH = H1 * H1, q = tid / HH;
+    const bool act = q < XS;
+    const int xs = act ? q : 0, e = act ? tid - q * HH : 0, i2 = e / H1, i1 = e - i2 * H1;
+    const int pos = xs * 4 * PL + i2 * RS + i1;  // in plane (0, 0)
+    const bool self1 = i1 == 0 || i1 == H, self2 = i2 == 0 || i2 == H;
+    unsigned ob[4];
+    {
+        const int n1 = i1 ? N - i1 : 0, n2 = i2 ? N - i2 : 0;
+        ob[0] = (unsigned)(xs * NN + i2 * N + i1) * (unsigned)sizeof(cT<T>);
+        ob[1] = (unsigned)(xs * NN + i2 * N + n1) * (unsigned)sizeof(cT<T>);
+        ob[2] = (unsigned)(xs * NN + n2 * N + i1) * (unsigned)sizeof(cT<T>);
+        ob[3] = (unsigned)(xs * NN + n2 * N + n1) * (unsigned)sizeof(cT<T>);
+    }
+    const T kc1 = D.kc[i1], kc2 = D.kc[i2];  // of the (+, +) element; zero where an axis is its own mirror
+    // D(k) = sum_i G_ii kd(k_i) - sum_{i != j} G_ij kc(k_i) kc(k_j)
+    const T dde = D.G[0] * D.kd[i1] + D.G[DIM + 1] * D.kd[i2], ddo = -(D.G[1] + D.G[DIM]) * kc1 * kc2;
+    const T g22 = DIM == 3 ? D.G[8] : T(0), g02 = DIM == 3 ? (D.G[2] + D.G[6]) * kc1 : T(0),
+            g12 = DIM == 3 ? (D.G[5] + D.G[7]) * kc2 : T(0);
+    const bool gyro = DIM == 3 && D.has_gyro;
+    __syncthreads();
+
+    // LDS reads of the products: T1 takes data rows i2 = lr over a = 4 s + lq,
+    // T2 data columns i1 = lr (lr beyond the plane is clamped: not stored).  Each
+    // plane's base is a register, the steps are immediate offsets.
+    const int lrc = lr < HP ? lr : HP - 1;
+    const int orw = lrc * RS + lq, ocl = lq * RS + lrc;
+    const cT<T>* bw = pF + w * PL;
+    const cT<T>* b1 = pF + (w ^ 1) * PL;
+    const cT<T>* b2 = pF + (w ^ 2) * PL;
+    constexpr int OV1 = XS * 4 * PL, OV2 = 2 * OV1;
+
+    const int nrc = (int)D.nrc, TS = MX.TS;
+    const int nxcd = gridDim.x >= 8 ? 8 : 1;
+    const int per = (int)gridDim.x / nxcd;
+    const int xcd = (int)blockIdx.x % nxcd;
+    const int hi = (int)((int64_t)ngroup * (xcd + 1) / nxcd);
+    int sl = (int)((int64_t)ngroup * xcd / nxcd) + (int)blockIdx.x / nxcd;  // group sl: row sl % nrc, k3 group sl / nrc
+    const int dr = per % nrc, dk = per / nrc;
+    int rp = sl % nrc, kg = sl / nrc;
+    const kc_ptr<int32_t> ord = as_const<int32_t>(MX.order);
+    int rnext = sl < hi ? ord[rp] : 0;
+    cT<T> fo[4], Zv[4];
+    auto load_own = [&](int row, int k3g) {
+        const int64_t bn = ((int64_t)row * nz + (DIM == 3 ? min(k3g * XS, N - XS) : 0)) * NN;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            fo[j] = *at_b(Fin + bn, ob[j]);
+            Zv[j] = DIM == 3 ? ld_once<T>(at_b(Z3 + bn, ob[j])) : czero<T>();
+        }
+    };
+    if (AHEAD && sl < hi) load_own(rnext, kg);
+    while (sl < hi) {
+        const int r = rnext;
+        // the group's first k3; a last group that would pass N starts earlier and
+        // leaves the slabs it shares with the previous group to that one
+        const int k30 = DIM == 3 ? min(kg * XS, N - XS) : 0;
+        const bool own = act && k30 + xs >= kg * XS;
+        const int64_t base = ((int64_t)r * nz + k30) * NN;
+        int rn = rp + dr, kn = kg + dk;
+        if (rn >= nrc) {
+            rn -= nrc;
+            kn++;
+        }
+        rnext = ord[rn];
+        const cT<T>* Fb = Fin + base;
+        const T kc3 = DIM == 3 ? skc[k30 + xs] : T(0), kd3 = DIM == 3 ? skd[k30 + xs] : T(0);
+        if (!AHEAD) load_own(r, kg);
+        // ---- mixing, as in k_drift_fused: W += (g0 kc1 + i g1 kc2) F_s, V1 += i u1 F_s, V2 += u2 F_s
+        const kc_ptr<int32_t> srcT = as_const<int32_t>(MX.src) + (int64_t)r * TS;
+        const kc_ptr<T> coefT = as_const<T>((const T*)MX.coef) + 2 * (int64_t)r * TS * NC;
+        cT<T> W[4], V1[4], V2[4];
+        {
+            const T de = DIM == 3 ? dde + g22 * kd3 : dde, a1 = g02 * kc3, a2 = g12 * kc3;
+            cT<T> pl[4];
+            parity4<T>(fo, pl);
+            if (act) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) pF[pos + j * PL] = pl[j];
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                T dd = (j == 0 || j == 3) ? de + ddo : de - ddo;
+                if (DIM == 3) dd -= (j & 1 ? -a1 : a1) + (j & 2 ? -a2 : a2);
+                W[j] = cscale<T>(fo[j], dd);
+                V1[j] = V2[j] = czero<T>();
+            }
+        }
+        for (int t0 = 0; t0 < TS; t0 += MB) {
+            int src[MB];
+            cT<T> fv[MB][4];
+#pragma unroll
+            for (int u = 0; u < MB; u++) src[u] = t0 + u < TS ? srcT[t0 + u] : -1;
+#pragma unroll
+            for (int u = 0; u < MB; u++) {
+                const cT<T>* Fs = Fin + ((int64_t)(src[u] < 0 ? 0 : (src[u] & 0xffffff)) * nz + k30) * NN;
+#pragma unroll
+                for (int j = 0; j < 4; j++) fv[u][j] = *at_b(Fs, ob[j]);
+            }
+#pragma unroll
+            for (int u = 0; u < MB; u++) {
+                if (src[u] < 0) continue;
+                const int fl = src[u] >> 24;
+                const int64_t cb = (int64_t)(t0 + u) * NC;
+                if (fl & 1) {
+                    const T a = coefT[2 * cb] * kc1, b = coefT[2 * (cb + 1) + 1] * kc2;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const T aj = j & 1 ? -a : a, bj = j & 2 ? -b : b;
+                        W[j].x = fma(aj, fv[u][j].x, fma(-bj, fv[u][j].y, W[j].x));
+                        W[j].y = fma(aj, fv[u][j].y, fma(bj, fv[u][j].x, W[j].y));
+                    }
+                }
+                if (fl & 2) {
+                    const T ui = coefT[2 * (cb + DIM) + 1];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        V1[j].x = fma(-ui, fv[u][j].y, V1[j].x);
+                        V1[j].y = fma(ui, fv[u][j].x, V1[j].y);
+                    }
+                }
+                if (fl & 4) {
+                    const T ur = coefT[2 * (cb + DIM + 1)];
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        V2[j].x = fma(ur, fv[u][j].x, V2[j].x);
+                        V2[j].y = fma(ur, fv[u][j].y, V2[j].y);
+                    }
+                }
+            }
+        }
+        if (DIM == 3) {
+            const kc_ptr<T> e3p = as_const<T>((const T*)D.e3) + 2 * (int64_t)r;
+            const T e3r = e3p[0], e3i = e3p[1] + D.b[2] * kc3;
+            const T z1 = gyro ? kc2 * D.gyro[1] : T(0), z2 = gyro ? kc1 * D.gyro[0] : T(0);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const T s1 = j & 2 ? -z1 : z1, s2 = j & 1 ? -z2 : z2;
+                V1[j].x = fma(s1, Zv[j].y, V1[j].x);
+                V1[j].y = fma(-s1, Zv[j].x, V1[j].y);
+                V2[j].x = fma(s2, Zv[j].y, V2[j].x);
+                V2[j].y = fma(-s2, Zv[j].x, V2[j].y);
+                W[j].x = fma(e3r, Zv[j].x, fma(-e3i, Zv[j].y, W[j].x));
+                W[j].y = fma(e3r, Zv[j].y, fma(e3i, Zv[j].x, W[j].y));
+            }
+        }
+        {
+            cT<T> pl[4];
+            parity4<T>(V1, pl);
+            if (act) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) pV1[pos + j * PL] = pl[j];
+            }
+            parity4<T>(V2, pl);
+            if (act) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) pV2[pos + j * PL] = pl[j];
+            }
+        }
+        cT<T> f0v[4];
+        if (sc.read_f0) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) f0v[j] = ld_once<T>(at_b(F0 + base, ob[j]));
+        }
+        if (AHEAD && sl + per < hi) load_own(rnext, kn);
+        __syncthreads();  // 1: the planes are complete
+
+        // ---- everything but T1 V1
+        acc_t cr[XS], ci[XS];
+#pragma unroll
+        for (int x = 0; x < XS; x++) {
+            const cT<T>* frow = bw + orw + x * 4 * PL;                     // own plane
+            const cT<T>* fcol = bw + ocl + x * 4 * PL;
+            const cT<T>* f1row = b1 + orw + x * 4 * PL;                    // other parity in axis 1
+            const cT<T>* f2col = b2 + ocl + x * 4 * PL;                    // other parity in axis 2
+            const cT<T>* y2col = p2 ? f2col : fcol + OV2;                  // p2 odd: b2 c2 (c0 1 1^T F); even: c0 1 1^T V2
+            acc_t ar = MF::zero(), ai = MF::zero(), gr = MF::zero(), gi = MF::zero();
+            cT<T> s1 = czero<T>(), s2 = czero<T>(), s3 = czero<T>();  // axis sums of this lane's a
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                const cT<T> x1 = frow[4 * s], x2 = fcol[4 * s * RS];
+                ar = MF::fma(x1.x, d1[s], ar);
+                ai = MF::fma(x1.y, d1[s], ai);
+                ar = MF::fma(d2[s], x2.x, ar);
+                ai = MF::fma(d2[s], x2.y, ai);
+                const cT<T> v = f2col[OV2 + 4 * s * RS];
+                ar = MF::fma(m2[s], -v.y, ar);
+                ai = MF::fma(m2[s], v.x, ai);
+                const cT<T> y2 = y2col[4 * s * RS];
+                s2.x = fma(ws[s], y2.x, s2.x);
+                s2.y = fma(ws[s], y2.y, s2.y);
+                if (p1) {
+                    const cT<T> y1 = f1row[4 * s];
+                    s1.x = fma(ws[s], y1.x, s1.x);
+                    s1.y = fma(ws[s], y1.y, s1.y);
+                }
+                if (gyro) {  // T2 F
+                    const cT<T> z = f2col[4 * s * RS];
+                    gr = MF::fma(m2[s], -z.y, gr);
+                    gi = MF::fma(m2[s], z.x, gi);
+                    s3.x = fma(ws[s], x2.x, s3.x);
+                    s3.y = fma(ws[s], x2.y, s3.y);
+                }
+            }
+            // p2 odd: times i (b2 kc2 c0 sum F); even: c0 sum V2
+            ar = MF::fma(rr2, p2 ? -s2.y : s2.x, ar);
+            ai = MF::fma(rr2, p2 ? s2.x : s2.y, ai);
+            if (p1) {
+                ar = MF::fma(-s1.y, rr1, ar);
+                ai = MF::fma(s1.x, rr1, ai);
+            }
+            if (gyro && !p2) {
+                gr = MF::fma(rr2, s3.x, gr);
+                gi = MF::fma(rr2, s3.y, gi);
+            }
+            cr[x] = ar;
+            ci[x] = ai;
+            if (gyro) {  // V1 -= i a3 kc3 T2 F (planes hold four times the parts)
+                const T s = T(4) * skc[k30 + x] * D.gyro[2];
+                cT<T>* v1 = pV1 + (x * 4 + w) * PL;
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int o2 = MF::orow(lq, v);
+                    if (o2 < H1 && lr < H1) {
+                        cT<T> u = v1[o2 * RS + lr];
+                        u.x = fma(s, gi[v], u.x);
+                        u.y = fma(-s, gr[v], u.y);
+                        v1[o2 * RS + lr] = u;
+                    }
+                }
+            }
+        }
+        __syncthreads();  // 2: V1 complete; F and V2 consumed
+#pragma unroll
+        for (int x = 0; x < XS; x++) {
+            acc_t ar = cr[x], ai = ci[x];
+            cT<T> s1 = czero<T>();
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                const cT<T> v = b1[OV1 + orw + x * 4 * PL + 4 * s];
+                ar = MF::fma(-v.y, m1[s], ar);
+                ai = MF::fma(v.x, m1[s], ai);
+                if (!p1) {  // c0 1 1^T V1
+                    const cT<T> y = bw[OV1 + orw + x * 4 * PL + 4 * s];
+                    s1.x = fma(ws[s], y.x, s1.x);
+                    s1.y = fma(ws[s], y.y, s1.y);
+                }
+            }
+            if (!p1) {
+                ar = MF::fma(s1.x, rr1, ar);
+                ai = MF::fma(s1.y, rr1, ai);
+            }
+            cT<T>* t = pF + (x * 4 + w) * PL;
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int o2 = MF::orow(lq, v);
+                if (o2 < H1 && lr < H1) t[o2 * RS + lr] = cmk<T>(ar[v], ai[v]);
+            }
+        }
+        __syncthreads();  // 3: the result planes are complete
+
+        // ---- dF = unfolded planes + W, epilogue (as k_drift_fused)
+        cT<T> y[4], qv[4];
+        {
+            cT<T> pl[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) pl[j] = pF[pos + j * PL];
+            parity4<T>(pl, y);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) qv[j] = cadd<T>(y[j], W[j]);
+        const bool st[4] = {own, own && !self1, own && !self2, own && !self1 && !self2};
+        if (sc.deriv_only) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (st[j]) st_once<T>(at_b(Fout + base, ob[j]), cscale<T>(qv[j], sc.dt));
+        } else {
+            if (!sc.read_f0) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) f0v[j] = *at_b(Fb, ob[j]);  // the slab itself, read again (an L2 hit)
+            }
+            const T h = sc.dt * sc.cd;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {  // every load is consumed before the first store
+                f0v[j].x = fma(h, qv[j].x, f0v[j].x);
+                f0v[j].y = fma(h, qv[j].y, f0v[j].y);
+                asm volatile("" : "+v"(f0v[j].x), "+v"(f0v[j].y));
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (st[j]) st_once<T>(at_b(Fout + base, ob[j]), f0v[j]);
+        }
+        sl += per;
+        kg = kn;
+        rp = rn;
+    }
+}
+
+// ---------------------------------------------------------- launcher -----
+
+// Sizes.  FP64: 3-D 1.07-1.54x (B = 8), 2-D 1.1-1.4x (B = 20) faster than the kernels
+// that serve the others, but for N = 16, which fills k_drift_fused_c's tile while its
+// planes of nine points do not fill a K step here (3-D 0.82x, 2-D 1.04x).  FP32: 3-D
+// from N = 18 on, 1.10-1.39x.  Smaller 3-D grids and the reduced model keep the other
+// kernels' rounding, in which the 64-bit gradients of an FP32 sweep stand (they
+// would move by 1e-8; N <= 14 would gain 1.04-1.32x, 2-D 0.76-1.38x).
+template <class T> bool drift_fold_ok(const DriftDev<T>& D) {
+    if (!D.ramp || !D.odd || !D.smix || D.adj || D.N % 2 || D.N > 30) return false;
+    if (sizeof(T) == 4) return D.dim == 3 && D.N >= 18;
+    return D.N >= 4 && D.N != 16;
+}
+
+template <class T, int DIM, int KS, int XS>
+static void fold_t(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0, void* Fout,
+                   const StageCoef<T>& sc, hipStream_t st) {
+    const size_t sh = sizeof(cT<T>) * 3 * XS * 4 * (size_t)(4 * KS * (4 * KS + 1));
+    const int nkg = DIM == 3 ? (D.N + XS - 1) / XS : 1;
+    const int64_t ng = D.nrc * nkg;
+    auto kern = k_drift_fold<T, DIM, KS, XS>;
+    allow_lds((const void*)kern, sh);
+    const unsigned grid = persistent_blocks((const void*)kern, ng, 256, sh);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(256), sh, st, D, MX, (const cT<T>*)Fin, (const cT<T>*)Z3, (const cT<T>*)F0,
+                       (cT<T>*)Fout, sc, (int)ng);
+}
+
+template <class T>
+void launch_drift_fold(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0,
+                       void* Fout, const StageCoef<T>& sc, hipStream_t st) {
+    HPUP_REQUIRE(drift_fold_ok<T>(D) && !sc.read_acc && !sc.write_acc,
+                 HPUP_ERR_UNSUPPORTED, "folded drift: odd real circulants, structured mixing, no stage sums");
+    if constexpr (sizeof(T) == 8) {
+        const int KS = (D.N / 2 + 1 + 3) / 4;
+        if (D.dim == 2) {
+            switch (KS) {
+            case 1: return fold_t<T, 2, 1, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
+            case 2: return fold_t<T, 2, 2, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
+            case 3: return fold_t<T, 2, 3, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
+            default: return fold_t<T, 2, 4, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
+            }
+        }
+        if (KS == 1) return fold_t<T, 3, 1, 4>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 4, 6
+        if (KS == 2) return fold_t<T, 3, 2, 4>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 8 .. 14
+    }
+    // slabs per workgroup: as many quarter planes as 256 threads hold
+    if (D.N <= 20) return fold_t<T, 3, 3, 2>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 18, 20
+    if (D.N == 22) return fold_t<T, 3, 3, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
+    return fold_t<T, 3, 4, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 24 .. 30
+}
+
+template bool drift_fold_ok<float>(const DriftDev<float>&);
+template bool drift_fold_ok<double>(const DriftDev<double>&);
+template void launch_drift_fold<float>(const DriftDev<float>&, const MixDev<float>&, const void*, const void*, const void*,
+                                       void*, const StageCoef<float>&, hipStream_t);
+template void launch_drift_fold<double>(const DriftDev<double>&, const MixDev<double>&, const void*, const void*,
+                                        const void*, void*, const StageCoef<double>&, hipStream_t);
+
+}  // namespace hpup

@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <tuple>
 #include <type_traits>
 
 #include "drift.h"
@@ -1496,18 +1497,15 @@ __global__ __launch_bounds__(256) void k_axis3_bf16x3(DriftDev<float> D, const f
 
 // ---------------------------------------------------------- launchers ---
 
-// Workgroups of a persistent fused kernel: enough to fill every CU at the
-// kernel's occupancy, never more than there are slabs.  The resident count is
-// looked up once per (kernel, device).
-template <class K> static unsigned persistent_grid(K kernel, int64_t nslab, int threads = 256, size_t lds = 0) {
+unsigned persistent_blocks(const void* kernel, int64_t nwork, int threads, size_t lds) {
     static std::mutex mu;
-    static std::map<std::pair<const void*, int>, int> resident;
+    static std::map<std::tuple<const void*, int, size_t>, int> resident;
     int dev = 0;
     HPUP_HIP(hipGetDevice(&dev));
     int cached = 0;
     {
         std::lock_guard<std::mutex> lk(mu);
-        auto it = resident.find({(const void*)kernel, dev});
+        auto it = resident.find({kernel, dev, lds});
         if (it != resident.end()) cached = it->second;
     }
     if (!cached) {
@@ -1516,11 +1514,14 @@ template <class K> static unsigned persistent_grid(K kernel, int64_t nslab, int 
         HPUP_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, lds));
         cached = std::max(1, ncu * std::max(per_cu, 1));
         std::lock_guard<std::mutex> lk(mu);
-        resident[{(const void*)kernel, dev}] = cached;
+        resident[{kernel, dev, lds}] = cached;
     }
-    int64_t g = std::min<int64_t>(nslab, cached);
+    int64_t g = std::min<int64_t>(nwork, cached);
     if (g >= 8) g -= g % 8;  // whole workgroups per XCD
     return (unsigned)g;
+}
+template <class K> static unsigned persistent_grid(K kernel, int64_t nslab, int threads = 256, size_t lds = 0) {
+    return persistent_blocks((const void*)kernel, nslab, threads, lds);
 }
 
 // the compact-layout kernel serves omega grids up to kCompactMaxN points per
@@ -1647,6 +1648,10 @@ void launch_drift_fused(const DriftDev<T>& D, const MixDev<T>& MX, const void* F
         else launch_fused_t<T, GemmF<T, true>, 2, false, true>(D, MX, Fin, Z3, F0, Fout, ACC, sc, nslab, st);
         return;
     }
+    if (!grav && drift_fold_ok<T>(D)) {
+        launch_drift_fold<T>(D, MX, Fin, Z3, F0, Fout, sc, st);
+        return;
+    }
     if (D.ramp && D.smix && !grav && D.N <= kCompactMaxN) {
         if (D.dim == 3) launch_compact<T, 3>(D, MX, Fin, Z3, F0, Fout, ACC, sc, nslab, st);
         else launch_compact<T, 2>(D, MX, Fin, Z3, F0, Fout, ACC, sc, nslab, st);
@@ -1671,6 +1676,7 @@ void launch_drift_fused(const DriftDev<T>& D, const MixDev<T>& MX, const void* F
 
 template <class T> const char* drift_fused_name(const DriftDev<T>& D, bool grav, bool bf16x3) {
     if (D.N > 32) return "k_drift_fused64";
+    if (!bf16x3 && !grav && drift_fold_ok<T>(D)) return "k_drift_fold";
     if (!bf16x3 && !D.adj && D.ramp && D.smix && !grav && D.N <= kCompactMaxN) return "k_drift_fused_c";
     return "k_drift_fused";
 }

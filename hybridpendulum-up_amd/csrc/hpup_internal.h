@@ -164,6 +164,8 @@ struct DriftSpec {
     // along axis p) + i (Im kappa_p circulant) F: one real circulant instead of
     // a complex one.
     bool ramp = false;
+    // ramp, and Im kappa_p is odd on every axis (x real): the parity-folded kernel
+    bool odd = false;
     double c0[3] = {0, 0, 0};
     // Clebsch-Gordan gravity terms per compact output r: up to TG terms (src, coef[dim] complex)
     int TG = 0;

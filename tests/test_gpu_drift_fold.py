@@ -1,0 +1,113 @@
+"""The parity-folded drift kernel (odd real circulants on even and odd parts)
+against the oracle at the edges of its range: the smallest and largest grids of
+each tile depth (6 | 10, 14 | 18, 22 | 24, 30), slab groups that do not divide
+the k3 axis (10 = 4 + 4 + 2, 14 = 3 x 4 + 2), grids that keep another kernel
+(16; FP32 2-D and small 3-D grids), full diffusion matrices, inertias with
+and without gyroscopic terms, several slabs per workgroup, and a coordinate whose
+real circulant is not odd, which the folding must not take.
+
+Tolerances: relative L2 1e-10 (FP64) and 2e-5 (FP32), as the other drift kernels'
+tests: a derivative is sums of at most 6 N + 30 products, so FP32 rounding stays
+below 210 * 6e-8 = 1.3e-5."""
+import numpy as np
+import pytest
+
+import hpup
+import oracle as O
+from helpers import density, omega_grid, operators, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+G2 = np.array([[0.1, 0.03], [0.02, 0.15]])
+G3 = np.array([[0.1, 0.02, 0.01], [0.03, 0.2, -0.02], [0.015, 0.025, 0.05]])
+BT = (0.2, 0.3, 0.25)
+JT = {"gyro": np.diag([1.0, 0.93539, 0.24935]), "iso": np.eye(3)}
+
+
+def _full(B, dim, N, L, seed):
+    f = density(B, dim, N, L, (8, 4, 2), seed=seed, Sigma=np.eye(dim) * 1.2)
+    _, _, _, w = O.grid(B)
+    return O.fft_forward(B, f, O.wigner_table(B), w, dim, N)
+
+
+CASES = [(2, N, "") for N in (4, 6, 12, 14, 16, 18, 22, 24, 30)] + \
+        [(3, N, "gyro") for N in (4, 6, 8, 10, 14, 16, 18, 20, 22, 24, 30)] + [(3, 10, "iso"), (3, 24, "iso")]
+
+
+@pytest.mark.parametrize("dim,N,inertia", CASES)
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-10), ("fp32", 2e-5)])
+def test_derivative_and_step(dim, N, inertia, precision, tol):
+    """dF (the derivative-only epilogue) and two midpoint steps (both update
+    epilogues) at B = 2 and 3."""
+    import torch
+    print("case fold", dim, N, inertia, precision, flush=True)
+    B, L, dt = (2 if dim == 3 and N > 14 else 3), 8.0, 0.004
+    Jt = JT[inertia] if dim == 3 else None
+    G, b = (G3 if dim == 3 else G2), np.array(BT[:dim])
+    Ffull = _full(B, dim, N, L, 10 * N + dim)
+    X, OJO, MR, u, cells = operators(B, dim, N, L, Jt)
+    kw = {} if Jt is None else {"Jt": Jt}
+    p = hpup.Plan(B, dim, N, L, b=BT if dim == 3 else (BT[0], BT[1], 0.0), G=G, dt=dt, method="midpoint",
+                  precision=precision, **kw)
+    F = p.upload_full(Ffull)
+    dF = p.derivative(F)
+    torch.cuda.synchronize()
+
+    def dense(y):
+        return O.derivative(B, dim, N, y, X, OJO, MR, b, G, L, u, cells)
+
+    def structured(y, h, method):
+        return O.integrate_structured(B, dim, N, y, X, Jt, MR, b, G, h, L, u, cells, method)
+
+    big = dim == 3 and N > 14  # the dense oracle takes minutes there
+    ref = (structured(Ffull, 1.0, "euler") - Ffull) if big else dense(Ffull)
+    e = rel_l2(p.download_full(dF), ref)
+    print("  derivative rel err %.2e" % e, flush=True)
+    assert e < tol
+    p.step(F, 2)
+    torch.cuda.synchronize()
+    y = Ffull
+    for _ in range(2):
+        y = structured(y, dt, "midpoint") if big else y + dt * dense(y + dt / 2 * dense(y))
+    e = rel_l2(p.download_full(F), y)
+    print("  two steps rel err %.2e" % e, flush=True)
+    assert e < tol
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-10), ("fp32", 2e-5)])
+def test_many_rows(precision, tol):
+    """B = 12 (2300 rows): every workgroup walks several rows, which the walk's
+    order permutes."""
+    import torch
+    print("case fold rows", precision, flush=True)
+    B, N, L, dt = 12, 18, 8.0, 0.004
+    Ffull = _full(B, 2, N, L, 7)
+    X, _, MR, u, cells = operators(B, 2, N, L)
+    ref = O.integrate_structured(B, 2, N, Ffull, X, None, MR, np.array(BT[:2]), G2, dt, L, u, cells, "RK4")
+    p = hpup.Plan(B, 2, N, L, b=(BT[0], BT[1], 0.0), G=G2, dt=dt, method="RK4", precision=precision)
+    F = p.upload_full(Ffull)
+    p.step(F, 1)
+    torch.cuda.synchronize()
+    e = rel_l2(p.download_full(F), ref)
+    print("  rel err %.2e" % e, flush=True)
+    assert e < tol
+
+
+@pytest.mark.parametrize("N", [14, 30])
+def test_circulant_not_odd(N):
+    """x + 0.3 i cos(2 pi x / L): the circulant's real part stays constant but
+    its imaginary part is not odd."""
+    print("case fold not odd", N, flush=True)
+    B, L, dt = 3, 8.0, 0.01
+    Ffull = _full(B, 2, N, L, 40 + N)
+    X, _, MR, u, cells = operators(B, 2, N, L)
+    x = omega_grid(2, N, L)
+    Xg = np.zeros_like(X)
+    for p in range(2):
+        Xg[..., p] = np.fft.fftn(x[p] + 0.3j * np.cos(2 * np.pi * x[p] / L))
+    b = np.array(BT[:2])
+    ref = O.integrate(B, 2, N, Ffull, Xg, None, MR, b, G2, dt, L, u, cells, "RK2")
+    out = hpup.pendulum_propagate_reduced(Ffull, Xg, MR, b, G2, dt, L, u, cells, "RK2")
+    e = rel_l2(out, ref)
+    print("  rel err %.2e" % e, flush=True)
+    assert e < 1e-10
