@@ -392,20 +392,17 @@ template <class T> struct PlanT : PlanBase {
     size_t cbytes() const { return sizeof(cT<T>) * (size_t)ncoef; }
 
     // FP32 grids whose rounding 64-bit figures stand in (XformDev::keep): the
-    // reduced model's hybrid steps, whose densities get_stat reads, and 3-D grids
+    // reduced model's with a reset, whose densities get_stat reads, and 3-D grids
     // of up to 16 points per axis, those of the restitution gradient
-    bool keep_fp32(bool hybrid) const {
-        return sizeof(T) == 4 && ((model.dim == 2 && hybrid) || (model.dim == 3 && model.N <= 16));
-    }
-    XformDev<T> xform(bool hybrid) const {
+    XformDev<T> xform() const {
         XformDev<T> X = xf.view;
-        X.keep = keep_fp32(hybrid) ? 1 : 0;
+        X.keep = sizeof(T) == 4 && (model.dim == 2 ? (bool)reset : model.dim == 3 && model.N <= 16);
         return X;
     }
     void forward(const void* f, void* F, hipStream_t st) override { forward_weighted(f, nullptr, 0, F, st); }
     // forward transform of the grid product f(R, x) wR[R * wstride]
-    void forward_weighted(const void* f, const T* wR, int wstride, void* F, hipStream_t st, bool hybrid = false) {
-        const XformDev<T> X = xform(hybrid);
+    void forward_weighted(const void* f, const T* wR, int wstride, void* F, hipStream_t st) {
+        const XformDev<T> X = xform();
         ensure(G, sizeof(cT<T>) * (size_t)g_elems(model.B, nx));
         launch_fwd_ag<T>(X, f, wR, wstride, G.p, st);
         if (half_omega(X)) {  // the omega DFTs on half of the rows write the other half
@@ -417,9 +414,8 @@ template <class T> struct PlanT : PlanBase {
         }
         HPUP_HIP(hipGetLastError());
     }
-    void backward(const void* F, void* f, hipStream_t st) override { backward_as(F, f, st, false); }
-    void backward_as(const void* F, void* f, hipStream_t st, bool hybrid) {
-        const XformDev<T> X = xform(hybrid);
+    void backward(const void* F, void* f, hipStream_t st) override {
+        const XformDev<T> X = xform();
         ensure(G, sizeof(cT<T>) * (size_t)g_elems(model.B, nx));
         ensure(tmp, cbytes());
         if (half_omega(X)) {  // the Hermitian part on half of the rows
@@ -830,9 +826,9 @@ template <class T> struct PlanT : PlanBase {
         HPUP_REQUIRE(F && f && nsteps >= 0, HPUP_ERR_ARG, "bad argument");
         for (int it = 0; it < nsteps; it++) {
             step(F, 1, st);
-            backward_as(F, f, st, true);
+            backward(F, f, st);
             reset_grid(f, f, model.dt, 0, st);
-            forward_weighted(f, nullptr, 0, F, st, true);
+            forward(f, F, st);
         }
     }
     void marginals(const void* f, const double* xg, std::vector<double>& hR, std::vector<double>& hG,

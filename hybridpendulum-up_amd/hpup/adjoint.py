@@ -23,8 +23,9 @@ factor of the diffusion term.  Each reverse stage is one fused kernel
 the forward stage values come from the same fused stage kernel
 (Plan.step_stages).  The forward states are kept at checkpoints every
 `checkpoint` steps; on the way back each segment is recomputed from its
-checkpoint once, keeping every stage value, and each step's reverse stages
-run in one call (Plan.adjoint_step).
+checkpoint once, keeping every stage value (the last segment keeps them on the
+way forward), and each step's reverse stages run in one call
+(Plan.adjoint_step).
 """
 import numpy as np
 
@@ -59,34 +60,38 @@ class Gradient:
         import torch
         K = int(nsteps)
         cp = max(1, int(checkpoint or K or 1))
-        checkpoints = [F0.clone()]
-        F = F0.clone()
-        for k in range(K):
-            self.fwd.step(F, 1)
-            if (k + 1) % cp == 0 and k + 1 < K:
-                checkpoints.append(F.clone())
-        FK = F
-        lam = dJ(FK).clone()
-        acc = torch.zeros(5, dtype=torch.float64, device=FK.device)
         ns = len(HORNER[self.method])
-        for seg in range(len(checkpoints) - 1, -1, -1):
-            k0 = seg * cp
-            k1 = min(K, k0 + cp)
-            # the segment's steps from its checkpoint, keeping every stage value
-            # (the last step's result is the next checkpoint, not recomputed)
-            stored = []
-            F = checkpoints[seg]
-            for k in range(k0, k1):
+        nseg = max(1, -(-K // cp))
+        checkpoints = [F0.clone()]
+        for seg in range(1, nseg):
+            checkpoints.append(self.fwd.step(checkpoints[-1].clone(), cp))
+
+        def segment(seg, last):
+            """The segment's steps from its checkpoint: (F_k, stage values) of
+            each, and the state after them (only formed for the last segment)."""
+            stored, F = [], checkpoints[seg]
+            n = min(K, (seg + 1) * cp) - seg * cp
+            for k in range(n):
                 ys = [torch.empty_like(F) for _ in range(ns - 1)]
-                nxt = torch.empty_like(F) if k < k1 - 1 else None
+                nxt = torch.empty_like(F) if last or k < n - 1 else None
                 self.fwd.step_stages(F, ys, nxt)
                 stored.append((F, ys))
                 F = nxt
-            for k in range(k1 - 1, k0 - 1, -1):
-                Fk, ys = stored[k - k0]
+            return stored, F
+
+        # the last segment is swept first: its stage values are taken on the way
+        # forward instead of a second time (the step forms the same ones).  10 RK4
+        # steps, checkpoint 5, B = 15, N = 30, FP32: 6.30 -> 5.42 ms
+        stored, FK = segment(nseg - 1, True)
+        lam = dJ(FK).clone()
+        acc = torch.zeros(5, dtype=torch.float64, device=FK.device)
+        for seg in range(nseg - 1, -1, -1):
+            if stored is None:
+                stored, _ = segment(seg, False)
+            while stored:
+                Fk, ys = stored.pop()
                 lam = self.adj.adjoint_step(Fk, ys, lam, acc)
-                stored[k - k0] = None
-            del stored
+            stored = None
         acc = acc.cpu().numpy()
         G = np.array([[acc[2], acc[4]], [acc[4], acc[3]]])  # G_10 and G_01 enter A as their sum
         return FK, lam, {"b": acc[:2].copy(), "G": G}
@@ -202,8 +207,10 @@ class HybridGradient:
         self.adj = Plan(B, dim, N, operator=1, **kw)
         self.ta = TransformAdjoint(self.fwd)
 
-    def _grid_before_reset(self, F):
-        Fp = self.fwd.step(F.clone(), 1)
+    def _grid_before_reset(self, F, Fp=None):
+        """The grid before the reset of the step from F (Fp: F after its
+        continuous step; F itself for a step in place)."""
+        Fp = self.fwd.step(F.clone() if Fp is None else Fp, 1)
         return self.fwd.backward(Fp)
 
     def run(self, F0, nsteps, dJ, checkpoint=None):
@@ -216,9 +223,16 @@ class HybridGradient:
         checkpoints = [F0.clone()]
         F = F0.clone()
         f = self.fwd.empty_grid()
+        fk = None
         for k in range(K):
+            if k == K - 1:
+                # the last step is swept first: its grid before the reset is kept
+                # (B = 10, N = 16, FP64, two steps, checkpoint 1: 12.42 -> 10.94 ms)
+                fk = self._grid_before_reset(F, F)
+                self.fwd.forward(self.fwd.reset(fk, f, self.dt), F)
+                break
             self.fwd.hybrid_step(F, f, 1)
-            if (k + 1) % cp == 0 and k + 1 < K:
+            if (k + 1) % cp == 0:
                 checkpoints.append(F.clone())
         FK = F
         lam = dJ(FK).clone()
@@ -232,10 +246,11 @@ class HybridGradient:
                 self.fwd.hybrid_step(nxt, f, 1)
                 states.append(nxt)
             for k in range(k1 - 1, k0 - 1, -1):
-                fk = self._grid_before_reset(states[k - k0])
+                if fk is None:
+                    fk = self._grid_before_reset(states[k - k0])
                 gbar = self.ta.forward_adjoint(lam)
                 self.fwd.reset_eps_grad(fk, gbar, acc, self.dt)
-                del fk
+                fk = None
                 fbar = self.fwd.reset_adjoint(gbar, gbar, self.dt)
                 lam = self.adj.step(self.ta.backward_adjoint(fbar).contiguous(), 1)
             del states

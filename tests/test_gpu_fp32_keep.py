@@ -1,8 +1,8 @@
-"""FP32 grids behind 64-bit figures (the reduced model's hybrid steps, 3-D grids of
-up to 16 points per axis) keep the direct (alpha, gamma) stages and the Toeplitz
+"""FP32 grids behind 64-bit figures (the reduced model with a reset, 3-D grids of up to
+16 points per axis) keep the direct (alpha, gamma) stages and the Toeplitz
 or direct (k1, k2) DFTs: against the FP64 plan at the edges of those kernels (B =
 16 | 17, the FFT bandlimit 15; N = 32 | 34, 64; the smallest grids), and the same
-plan's transforms outside a hybrid step, which take the MFMA forms.
+plan's transforms before it has a reset, which take the MFMA forms in 2-D.
 
 Tolerance: relative L2 2e-5, the other FP32 tests' (a transform is about 2 N + 6 B
 products deep, rounding below 300 * 6e-8 = 1.8e-5)."""
