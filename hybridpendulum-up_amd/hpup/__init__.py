@@ -221,7 +221,7 @@ def _propagate(fn, dtype, F, X, OJO, MR, bt, G, dtt, L, u, CG, method):
     B = F.shape[2]
     keep = []
     cg = _cg_ptrs(CG, B, dtype, keep)
-    out = np.zeros_like(F, order="F")
+    out = np.empty_like(F, order="F")  # written whole, the entries outside |m|, |n| <= l as zeros
     args = [_p(F, t), _dims(F), _p(_interleaved(X, cdt), t)]
     if OJO is not None:
         args.append(_p(_interleaved(OJO, cdt), t))
@@ -244,7 +244,7 @@ def pendulum_propagate_reduced32(F, X, MR, bt, G, dtt, L, u, CG, method):
 def pendulum_propagate_reduced_den(F, f, X, mR, bt, G, dtt, L, u, d, w, method):
     """Fnew = pendulum_propagate_reduced_den(F, f, X, mR, bt, G, dtt, L, u, d, w, method)."""
     F = _interleaved(F, np.complex128)
-    out = np.zeros_like(F, order="F")
+    out = np.empty_like(F, order="F")  # written whole, the entries outside |m|, |n| <= l as zeros
     _check(lib().hpup_pendulum_propagate_reduced_den(
         _p(F), _dims(F), _p(np.asfortranarray(f, dtype=np.float64)), _p(_interleaved(X, np.complex128)),
         _p(np.asfortranarray(mR, dtype=np.float64)), _p(np.ascontiguousarray(np.ravel(bt), dtype=np.float64)),
@@ -373,7 +373,7 @@ def gyrobias_propagate(F, X, dt, u, G1, G2):
     """Fnew = gyrobias_propagate(F, X, dt, u, G1, G2) (gyrobias_propagate/kernel.cu:8-120): one
     Euler step of the attitude x gyro-bias model, FP64."""
     F = np.asfortranarray(F, dtype=np.complex128)
-    out = np.zeros_like(F, order="F")
+    out = np.empty_like(F, order="F")  # written whole, the entries outside |m|, |n| <= l as zeros
     _check(lib().hpup_gyrobias_propagate(_p(F), _dims(F), _p(_interleaved(X, np.complex128)), ctypes.c_double(dt),
                                          _p(_interleaved(u, np.complex128)),
                                          _p(np.asfortranarray(G1, dtype=np.float64)),
