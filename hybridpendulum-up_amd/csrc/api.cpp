@@ -299,6 +299,7 @@ template <class T> struct DriftTables {
         for (int i = 0; i < 3; i++) { v.b[i] = (T)s.b[i]; v.gyro[i] = (T)s.gyro[i]; v.c0[i] = (T)s.c0[i]; }
         v.ramp = s.ramp ? 1 : 0;
         v.odd = s.odd ? 1 : 0;
+        v.same12 = s.same12 ? 1 : 0;
         v.smix = smix ? 1 : 0;
         v.adj = s.adj ? 1 : 0;
         v.has_gyro = s.has_gyro ? 1 : 0;

@@ -41,7 +41,8 @@ template <class T> struct DriftDev {
     const cT<T>* grav[3];
     // every kap_p = c0[p] + i (real circulant): the real-circulant path
     int ramp;
-    int odd;  // ... and the real circulants are odd
+    int odd;     // ... and the real circulants are odd
+    int same12;  // ... and those of axes 1 and 2 are equal
     T c0[3];
     // structured mixing coefficients: -i CG_1 real, -i CG_2 imaginary,
     // CG_3 zero, u_1 imaginary, u_2 real (the pendulum models)
@@ -97,6 +98,10 @@ template <class T> bool drift_fold_ok(const DriftDev<T>& D);
 template <class T>
 void launch_drift_fold(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0,
                        void* Fout, const StageCoef<T>& sc, hipStream_t st);
+// the same for the reduced model's FP64 grids of 34 to 62 points per axis
+bool drift_fold64_ok(const DriftDev<double>& D);
+void launch_drift_fold64(const DriftDev<double>& D, const MixDev<double>& MX, const void* Fin, const void* F0, void* Fout,
+                         const StageCoef<double>& sc, hipStream_t st);
 // name of the kernel launch_drift_fused runs for D (grav: density-form gravity)
 template <class T> const char* drift_fused_name(const DriftDev<T>& D, bool grav, bool bf16x3);
 // out = T3 in; scaled: out = T3 [(e3[r] - i b3 kc(k3)) in] (the 3-D adjoint's

@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
 
     // ---- this wave's matrices (plane (p1, p2)), entry [out lr][in 4 s + lq]
     const int p1 = w & 1, p2 = w >> 1;
-    T m1[KS], m2[KS], d1[KS], d2[KS], ws[KS], rr1, rr2;
+    T m1[KS], m2[KS], d1[KS], d2[KS], rr1, rr2;
     {
         auto mats = [&](const cT<T>* kap, int p, T c0, T b, T* m, T* d, T& rr) {
             auto K = [&](int j) { return kap[((j % N) + N) % N].y; };
@@ -122,14 +122,21 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
                 eo *= T(0.25);
                 m[s] = p ? oe : eo;               // K into this plane's parity
                 d[s] = -b * kco * (p ? eo : oe);  // b c (i K): K to the other parity and kc back
-                ws[s] = !in ? T(0) : self ? T(0.25) : T(0.5);  // the axis sum's weights
             }
-            rr = lr <= H ? c0 * (p ? b * kco : T(1)) : T(0);
+            rr = lr <= H ? T(0.5) * c0 * (p ? b * kco : T(1)) : T(0);
         };
         mats(D.kap, p1, D.c0[0], D.b[0], m1, d1, rr1);
         mats(D.kap + N, p2, D.c0[1], D.b[1], m2, d2, rr2);
     }
 
+    // weights of the axis sums: a half for a = 0 (step 0) and a = H (the last
+    // step), one else (zeros lie beyond H)
+    const T wa = lq == 0 || lq == H ? T(0.5) : T(1), wb = lq == (H & 3) ? T(0.5) : T(1);
+    auto add_w = [&](cT<T>& t, int s, cT<T> x) {
+        if (s == 0) t = cscale<T>(x, wa);
+        else if (s < KS - 1) t = cadd<T>(t, x);
+        else t = cmk<T>(fma(wb, x.x, t.x), fma(wb, x.y, t.y));
+    };
     // ---- this thread's elements
     const int HH = H1 * H1, q = tid / HH;
     const bool act = q < XS;
@@ -319,19 +326,16 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
                 ar = MF::fma(m2[s], -v.y, ar);
                 ai = MF::fma(m2[s], v.x, ai);
                 const cT<T> y2 = y2col[4 * s * RS];
-                s2.x = fma(ws[s], y2.x, s2.x);
-                s2.y = fma(ws[s], y2.y, s2.y);
+                add_w(s2, s, y2);
                 if (p1) {
                     const cT<T> y1 = f1row[4 * s];
-                    s1.x = fma(ws[s], y1.x, s1.x);
-                    s1.y = fma(ws[s], y1.y, s1.y);
+                    add_w(s1, s, y1);
                 }
                 if (gyro) {  // T2 F
                     const cT<T> z = f2col[4 * s * RS];
                     gr = MF::fma(m2[s], -z.y, gr);
                     gi = MF::fma(m2[s], z.x, gi);
-                    s3.x = fma(ws[s], x2.x, s3.x);
-                    s3.y = fma(ws[s], x2.y, s3.y);
+                    add_w(s3, s, x2);
                 }
             }
             // p2 odd: times i (b2 kc2 c0 sum F); even: c0 sum V2
@@ -374,8 +378,7 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
                 ai = MF::fma(v.x, m1[s], ai);
                 if (!p1) {  // c0 1 1^T V1
                     const cT<T> y = bw[OV1 + orw + x * 4 * PL + 4 * s];
-                    s1.x = fma(ws[s], y.x, s1.x);
-                    s1.y = fma(ws[s], y.y, s1.y);
+                    add_w(s1, s, y);
                 }
             }
             if (!p1) {
@@ -428,6 +431,323 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
     }
 }
 
+// ------------------------------------------------------ N = 34 .. 62 ----
+//
+// The same folding for the reduced model's larger grids in FP64: planes of up to
+// 32 x 32 points, 2 x 2 tiles of the matrix instruction each.  A workgroup of eight
+// waves holds one slab; wave (plane, row tile) forms both column tiles.  LDS holds
+// two fields of four planes: F and V2, then V1 in F's place, then the result in
+// V2's; V1 and W wait in registers (NQ quartets of elements per thread).  The
+// axes share their matrices, which leaves room for them in LDS: in registers, as in
+// k_drift_fold, they spill 137 registers (B = 30, N = 60: 4.80 ms), axis 1's alone
+// in LDS 59 (3.57 ms), both 19 (2.97 ms; k_drift_fused64 5.38 ms).  N <= 42, one quartet a
+// thread, spills none: 2.8-3.1x, N = 44 .. 62 1.9-2.2x faster than k_drift_fused64 (B =
+// 10).  What bounds it: 17000 matrix cycles of 47000 per slab; one workgroup fits a CU,
+// so the mixing's loads and the products take turns.
+template <int KS, int NQ>
+__global__ __launch_bounds__(512, 2) void k_drift_fold64(DriftDev<double> D, MixDev<double> MX, const cT<double>* Fin,
+                                                         const cT<double>* F0, cT<double>* Fout, StageCoef<double> sc,
+                                                         int nslab) {
+    using T = double;
+    using MF = Mfma<T>;
+    using acc_t = typename MF::acc;
+    constexpr int NC = 4, MB = 2, HP = 4 * KS, RS = HP + 1, PL = HP * RS, OV = 4 * PL;
+    extern __shared__ __align__(16) char smem_fold64[];
+    const int N = D.N, NN = N * N, H = N / 2, H1 = H + 1, HH = H1 * H1;
+    cT<T>* pA = reinterpret_cast<cT<T>*>(smem_fold64);  // [4][HP][RS], zero beyond H1 x H1
+    cT<T>* pB = pA + OV;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, lr = lane & 15, lq = lane >> 4;
+    const int pl = w & 3, rt = w >> 2, p1 = pl & 1, p2 = pl >> 1;
+    for (int i = tid; i < 2 * OV; i += 512) pA[i] = czero<T>();
+
+    // ---- the axes' matrices (the same for both: D.same12) in LDS, [odd -> even,
+    // even -> odd][in][out]
+    T* sM = reinterpret_cast<T*>(pA + 2 * OV);
+    auto entry = [&](const cT<T>* kap, int o, int a, T& oe, T& eo) {
+        const bool in = a <= H && o <= H, self = a == 0 || a == H;
+        auto K = [&](int j) { return kap[((j % N) + N) % N].y; };
+        const T km = in ? K(o - a) : T(0), kp = in ? K(o + a) : T(0);
+        oe = !in || o == 0 || o == H ? T(0) : T(0.25) * (self ? km : km + kp);  // even -> odd
+        eo = !in || self ? T(0) : T(0.25) * (km - kp);                        // odd -> even
+    };
+    for (int i = tid; i < HP * HP; i += 512) entry(D.kap, i % HP, i / HP, sM[HP * HP + i], sM[i]);
+    T rr1[2], k1o[2], rr2, k2o;  // k_o: -b kc of the outputs
+    {
+        const int o2 = 16 * rt + lr;
+        k2o = o2 <= H ? -D.b[1] * D.kc[o2] : T(0);
+        rr2 = o2 <= H ? T(0.5) * D.c0[1] * (p2 ? -k2o : T(1)) : T(0);
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const int o1 = 16 * c + lr;
+            k1o[c] = o1 <= H ? -D.b[0] * D.kc[o1] : T(0);
+            rr1[c] = o1 <= H ? T(0.5) * D.c0[0] * (p1 ? -k1o[c] : T(1)) : T(0);
+        }
+    }
+    const T wa = lq == 0 || lq == H ? T(0.5) : T(1), wb = lq == (H & 3) ? T(0.5) : T(1);
+    auto add_w = [&](cT<T>& t, int s, cT<T> x) {
+        if (s == 0) t = cscale<T>(x, wa);
+        else if (s < KS - 1) t = cadd<T>(t, x);
+        else t = cmk<T>(fma(wb, x.x, t.x), fma(wb, x.y, t.y));
+    };
+    // LDS reads of the products (rows and columns beyond the plane are clamped: not stored)
+    const int row = 16 * rt + lr < HP ? 16 * rt + lr : HP - 1;
+    const int orw = row * RS + lq;
+    const T* sm2 = sM + p2 * HP * HP + lq * HP + row;
+    const T* sd2 = sM + (p2 ^ 1) * HP * HP + lq * HP + row;
+    int ocl[2];
+    const T *sm1[2], *sd1[2];  // K into this plane's parity along axis 1; the other one
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const int col = 16 * c + lr < HP ? 16 * c + lr : HP - 1;
+        ocl[c] = lq * RS + col;
+        sm1[c] = sM + p1 * HP * HP + lq * HP + col;
+        sd1[c] = sM + (p1 ^ 1) * HP * HP + lq * HP + col;
+    }
+    const cT<T>* aw = pA + pl * PL;
+    const cT<T>* a1 = pA + (pl ^ 1) * PL;
+    const cT<T>* a2 = pA + (pl ^ 2) * PL;
+
+    const int nrc = (int)D.nrc, TS = MX.TS;
+    const int nxcd = gridDim.x >= 8 ? 8 : 1;
+    const int per = (int)gridDim.x / nxcd;
+    const int xcd = (int)blockIdx.x % nxcd;
+    const int hi = (int)((int64_t)nslab * (xcd + 1) / nxcd);
+    const kc_ptr<int32_t> ord = as_const<int32_t>(MX.order);
+    __syncthreads();
+    for (int sl = (int)((int64_t)nslab * xcd / nxcd) + (int)blockIdx.x / nxcd; sl < hi; sl += per) {
+        const int r = ord[sl];
+        const int64_t base = (int64_t)r * NN;
+        const kc_ptr<int32_t> srcT = as_const<int32_t>(MX.src) + (int64_t)r * TS;
+        const kc_ptr<T> coefT = as_const<T>((const T*)MX.coef) + 2 * (int64_t)r * TS * NC;
+        // the thread's quartets, their offsets formed anew for each slab (held
+        // through the loop they would cost the registers that V1 and W take)
+        int zo;
+        asm volatile("v_mov_b32 %0, 0" : "=v"(zo));
+        cT<T> W[NQ][4], V1[NQ][4];
+        auto quartet = [&](int q, bool& act, int& pos, unsigned* ob, int& i1, int& i2) {
+            const int e0 = tid + zo + 512 * q;
+            act = e0 < HH;
+            const int e = act ? e0 : 0;
+            i2 = e / H1;
+            i1 = e - i2 * H1;
+            pos = i2 * RS + i1;
+            const int n1 = i1 ? N - i1 : 0, n2 = i2 ? N - i2 : 0;
+            ob[0] = (unsigned)(i2 * N + i1) * (unsigned)sizeof(cT<T>);
+            ob[1] = (unsigned)(i2 * N + n1) * (unsigned)sizeof(cT<T>);
+            ob[2] = (unsigned)(n2 * N + i1) * (unsigned)sizeof(cT<T>);
+            ob[3] = (unsigned)(n2 * N + n1) * (unsigned)sizeof(cT<T>);
+        };
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            bool act;
+            int pos, i1, i2;
+            unsigned ob[4];
+            quartet(q, act, pos, ob, i1, i2);
+            const T kc1 = D.kc[i1], kc2 = D.kc[i2];
+            const T dde = D.G[0] * D.kd[i1] + D.G[3] * D.kd[i2], ddo = -(D.G[1] + D.G[2]) * kc1 * kc2;
+            cT<T> fo[4], V2[4], pv[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) fo[j] = *at_b(Fin + base, ob[j]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) W[q][j] = V1[q][j] = V2[j] = czero<T>();
+            for (int t0 = 0; t0 < TS; t0 += MB) {
+                int src[MB];
+                cT<T> fv[MB][4];
+#pragma unroll
+                for (int u = 0; u < MB; u++) src[u] = t0 + u < TS ? srcT[t0 + u] : -1;
+#pragma unroll
+                for (int u = 0; u < MB; u++) {
+                    const cT<T>* Fs = Fin + (int64_t)(src[u] < 0 ? 0 : (src[u] & 0xffffff)) * NN;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) fv[u][j] = *at_b(Fs, ob[j]);
+                }
+#pragma unroll
+                for (int u = 0; u < MB; u++) {
+                    if (src[u] < 0) continue;
+                    const int fl = src[u] >> 24;
+                    const int64_t cb = (int64_t)(t0 + u) * NC;
+                    if (fl & 1) {
+                        const T a = coefT[2 * cb] * kc1, b = coefT[2 * (cb + 1) + 1] * kc2;
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            const T aj = j & 1 ? -a : a, bj = j & 2 ? -b : b;
+                            W[q][j].x = fma(aj, fv[u][j].x, fma(-bj, fv[u][j].y, W[q][j].x));
+                            W[q][j].y = fma(aj, fv[u][j].y, fma(bj, fv[u][j].x, W[q][j].y));
+                        }
+                    }
+                    if (fl & 2) {
+                        const T ui = coefT[2 * (cb + 2) + 1];
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            V1[q][j].x = fma(-ui, fv[u][j].y, V1[q][j].x);
+                            V1[q][j].y = fma(ui, fv[u][j].x, V1[q][j].y);
+                        }
+                    }
+                    if (fl & 4) {
+                        const T ur = coefT[2 * (cb + 3)];
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            V2[j].x = fma(ur, fv[u][j].x, V2[j].x);
+                            V2[j].y = fma(ur, fv[u][j].y, V2[j].y);
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const T dd = (j == 0 || j == 3) ? dde + ddo : dde - ddo;
+                W[q][j].x = fma(dd, fo[j].x, W[q][j].x);
+                W[q][j].y = fma(dd, fo[j].y, W[q][j].y);
+            }
+            parity4<T>(fo, pv);
+            if (act) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) pA[pos + j * PL] = pv[j];
+            }
+            parity4<T>(V2, pv);
+            if (act) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) pB[pos + j * PL] = pv[j];
+            }
+            __builtin_amdgcn_sched_barrier(0);  // one quartet's registers at a time
+        }
+        __syncthreads();  // 1: F and V2 complete
+
+        // ---- everything but T1 V1
+        acc_t ar[2], ai[2];
+#pragma unroll
+        for (int c = 0; c < 2; c++) ar[c] = ai[c] = MF::zero();
+        {
+            cT<T> s1 = czero<T>();  // axis sums of this lane's a
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                const cT<T> x1 = aw[orw + 4 * s];
+#pragma unroll
+                for (int c = 0; c < 2; c++) {  // b1 c1 (i K): K to the other parity and kc back
+                    const T d = k1o[c] * sd1[c][4 * s * HP];
+                    ar[c] = MF::fma(x1.x, d, ar[c]);
+                    ai[c] = MF::fma(x1.y, d, ai[c]);
+                }
+                if (p1) {
+                    const cT<T> y1 = a1[orw + 4 * s];
+                    add_w(s1, s, y1);
+                }
+            }
+            if (p1) {
+#pragma unroll
+                for (int c = 0; c < 2; c++) {
+                    ar[c] = MF::fma(-s1.y, rr1[c], ar[c]);
+                    ai[c] = MF::fma(s1.x, rr1[c], ai[c]);
+                }
+            }
+        }
+        {
+            const cT<T>* f = aw;
+            const cT<T>* f2 = a2;
+            const cT<T>* y2p = p2 ? f2 : f + OV;  // p2 odd: b2 c2 (c0 1 1^T F); even: c0 1 1^T V2
+            cT<T> s2[2] = {czero<T>(), czero<T>()};
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                const T m = sm2[4 * s * HP], d = k2o * sd2[4 * s * HP];
+#pragma unroll
+                for (int c = 0; c < 2; c++) {
+                    const int o = ocl[c] + 4 * s * RS;
+                    const cT<T> x2 = f[o], v = f2[OV + o], y2 = y2p[o];
+                    ar[c] = MF::fma(d, x2.x, ar[c]);
+                    ai[c] = MF::fma(d, x2.y, ai[c]);
+                    ar[c] = MF::fma(m, -v.y, ar[c]);
+                    ai[c] = MF::fma(m, v.x, ai[c]);
+                    add_w(s2[c], s, y2);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                ar[c] = MF::fma(rr2, p2 ? -s2[c].y : s2[c].x, ar[c]);
+                ai[c] = MF::fma(rr2, p2 ? s2[c].x : s2[c].y, ai[c]);
+            }
+        }
+        __syncthreads();  // 2: F and V2 consumed
+        cT<T> f0v[NQ][4];
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            bool act;
+            int pos, i1, i2;
+            unsigned ob[4];
+            quartet(q, act, pos, ob, i1, i2);
+            cT<T> pv[4];
+            parity4<T>(V1[q], pv);
+            if (act) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) pA[pos + j * PL] = pv[j];
+            }
+            const cT<T>* Fz = (sc.read_f0 ? F0 : Fin) + base;
+            if (!sc.deriv_only) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) f0v[q][j] = ld_once<T>(at_b(Fz, ob[j]));
+            }
+        }
+        __syncthreads();  // 3: V1 complete
+        {
+            cT<T> s1 = czero<T>();
+#pragma unroll
+            for (int s = 0; s < KS; s++) {
+                const cT<T> v = a1[orw + 4 * s];
+#pragma unroll
+                for (int c = 0; c < 2; c++) {
+                    const T m = sm1[c][4 * s * HP];
+                    ar[c] = MF::fma(-v.y, m, ar[c]);
+                    ai[c] = MF::fma(v.x, m, ai[c]);
+                }
+                if (!p1) {  // c0 1 1^T V1
+                    const cT<T> y = aw[orw + 4 * s];
+                    add_w(s1, s, y);
+                }
+            }
+            if (!p1) {
+#pragma unroll
+                for (int c = 0; c < 2; c++) {
+                    ar[c] = MF::fma(s1.x, rr1[c], ar[c]);
+                    ai[c] = MF::fma(s1.y, rr1[c], ai[c]);
+                }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int o2 = 16 * rt + MF::orow(lq, v), o1 = 16 * c + lr;
+                if (o2 < H1 && o1 < H1) pB[pl * PL + o2 * RS + o1] = cmk<T>(ar[c][v], ai[c][v]);
+            }
+        __syncthreads();  // 4: the result planes are complete, V1 consumed
+
+        // ---- dF = unfolded planes + W, epilogue
+#pragma unroll
+        for (int q = 0; q < NQ; q++) {
+            bool act;
+            int pos, i1, i2;
+            unsigned ob[4];
+            quartet(q, act, pos, ob, i1, i2);
+            const bool self1 = i1 == 0 || i1 == H, self2 = i2 == 0 || i2 == H;
+            const bool st[4] = {act, act && !self1, act && !self2, act && !self1 && !self2};
+            cT<T> pv[4], y[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) pv[j] = pB[pos + j * PL];
+            parity4<T>(pv, y);
+            const T h = sc.dt * sc.cd;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {  // every load is consumed before the first store
+                y[j] = cadd<T>(y[j], W[q][j]);
+                y[j] = sc.deriv_only ? cscale<T>(y[j], sc.dt)
+                                     : cmk<T>(fma(h, y[j].x, f0v[q][j].x), fma(h, y[j].y, f0v[q][j].y));
+                asm volatile("" : "+v"(y[j].x), "+v"(y[j].y));
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (st[j]) st_once<T>(at_b(Fout + base, ob[j]), y[j]);
+        }
+    }
+}
+
 // ---------------------------------------------------------- launcher -----
 
 // Sizes.  FP64: 3-D 1.07-1.54x (B = 8), 2-D 1.1-1.4x (B = 20) faster than the kernels
@@ -440,6 +760,33 @@ template <class T> bool drift_fold_ok(const DriftDev<T>& D) {
     if (!D.ramp || !D.odd || !D.smix || D.adj || D.N % 2 || D.N > 30) return false;
     if (sizeof(T) == 4) return D.dim == 3 && D.N >= 18;
     return D.N >= 4 && D.N != 16;
+}
+
+template <int KS, int NQ>
+static void fold64_t(const DriftDev<double>& D, const MixDev<double>& MX, const void* Fin, const void* F0, void* Fout,
+                     const StageCoef<double>& sc, hipStream_t st) {
+    const size_t sh = sizeof(cT<double>) * 2 * 4 * (size_t)(4 * KS * (4 * KS + 1)) + sizeof(double) * 2 * (16 * KS * KS);
+    auto kern = k_drift_fold64<KS, NQ>;
+    allow_lds((const void*)kern, sh);
+    const unsigned grid = persistent_blocks((const void*)kern, D.nrc, 512, sh);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), sh, st, D, MX, (const cT<double>*)Fin, (const cT<double>*)F0,
+                       (cT<double>*)Fout, sc, (int)D.nrc);
+}
+
+bool drift_fold64_ok(const DriftDev<double>& D) {
+    return D.ramp && D.odd && D.same12 && D.smix && !D.adj && D.dim == 2 && D.N % 2 == 0 && D.N >= 34 && D.N <= 62;
+}
+void launch_drift_fold64(const DriftDev<double>& D, const MixDev<double>& MX, const void* Fin, const void* F0, void* Fout,
+                         const StageCoef<double>& sc, hipStream_t st) {
+    HPUP_REQUIRE(drift_fold64_ok(D) && !sc.read_acc && !sc.write_acc, HPUP_ERR_UNSUPPORTED,
+                 "folded drift, N = 34 .. 62: odd real circulants, structured mixing, no stage sums");
+    const bool one = (D.N / 2 + 1) * (D.N / 2 + 1) <= 512;  // N <= 42
+    switch ((D.N / 2 + 4) / 4) {
+    case 5: return fold64_t<5, 1>(D, MX, Fin, F0, Fout, sc, st);
+    case 6: return one ? fold64_t<6, 1>(D, MX, Fin, F0, Fout, sc, st) : fold64_t<6, 2>(D, MX, Fin, F0, Fout, sc, st);
+    case 7: return fold64_t<7, 2>(D, MX, Fin, F0, Fout, sc, st);
+    default: return fold64_t<8, 2>(D, MX, Fin, F0, Fout, sc, st);
+    }
 }
 
 template <class T, int DIM, int KS, int XS>

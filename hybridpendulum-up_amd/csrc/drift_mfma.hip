@@ -1597,6 +1597,9 @@ void launch_drift_fused(const DriftDev<T>& D, const MixDev<T>& MX, const void* F
     if (D.N > 32) {
         HPUP_REQUIRE(!bf16x3, HPUP_ERR_UNSUPPORTED, "3xBF16 drift needs N <= 32");
         HPUP_REQUIRE(!D.adj, HPUP_ERR_UNSUPPORTED, "the adjoint operator needs N <= 32");
+        if constexpr (sizeof(T) == 8) {
+            if (!grav && drift_fold64_ok(D)) return launch_drift_fold64(D, MX, Fin, F0, Fout, sc, st);
+        }
         if (D.ramp && D.smix) {
             if (grav) launch_fused64_t<T, true, true, true>(D, MX, Fin, F0, Fout, ACC, sc, nslab, st);
             else launch_fused64_t<T, true, false, true>(D, MX, Fin, F0, Fout, ACC, sc, nslab, st);
@@ -1675,6 +1678,9 @@ void launch_drift_fused(const DriftDev<T>& D, const MixDev<T>& MX, const void* F
 }
 
 template <class T> const char* drift_fused_name(const DriftDev<T>& D, bool grav, bool bf16x3) {
+    if constexpr (sizeof(T) == 8) {
+        if (D.N > 32 && !grav && drift_fold64_ok(D)) return "k_drift_fold64";
+    }
     if (D.N > 32) return "k_drift_fused64";
     if (!bf16x3 && !grav && drift_fold_ok<T>(D)) return "k_drift_fold";
     if (!bf16x3 && !D.adj && D.ramp && D.smix && !grav && D.N <= kCompactMaxN) return "k_drift_fused_c";

@@ -166,6 +166,7 @@ struct DriftSpec {
     bool ramp = false;
     // ramp, and Im kappa_p is odd on every axis (x real): the parity-folded kernel
     bool odd = false;
+    bool same12 = false;  // odd, and Im kappa_1 = Im kappa_2 (one box for both axes)
     double c0[3] = {0, 0, 0};
     // Clebsch-Gordan gravity terms per compact output r: up to TG terms (src, coef[dim] complex)
     int TG = 0;

@@ -311,6 +311,12 @@ DriftSpec build_drift_spec_from_arrays(int B, int dim, int N, double L, const do
             if (!(std::abs(kap(p, j).imag() + kap(p, (N - j) % N).imag()) <= 1e-3 * tol * mx)) s.odd = false;
     }
     if (!s.ramp) s.odd = false;
+    s.same12 = s.odd && dim >= 2;
+    for (int j = 0; j < N && s.same12; j++) {
+        double mx = 0.0;
+        for (int a = 0; a < N; a++) mx = std::max(mx, std::abs(kap(0, a)));
+        if (!(std::abs(kap(0, j).imag() - kap(1, j).imag()) <= 1e-3 * tol * mx)) s.same12 = false;
+    }
 
     // ---- OJO: separable gyroscopic coefficients
     if (dim == 3 && OJOr) {

@@ -1,6 +1,7 @@
 """The parity-folded drift kernel (odd real circulants on even and odd parts)
 against the oracle at the edges of its range: the smallest and largest grids of
-each tile depth (6 | 10, 14 | 18, 22 | 24, 30), slab groups that do not divide
+each tile depth (6 | 10, 14 | 18, 22 | 24, 30; the reduced model's FP64 kernel for
+34 to 62 points at 34, 38 | 40, 42 | 44, 46 | 48 | 62: one and two quartets a thread), slab groups that do not divide
 the k3 axis (10 = 4 + 4 + 2, 14 = 3 x 4 + 2), grids that keep another kernel
 (16; FP32 2-D and small 3-D grids), full diffusion matrices, inertias with
 and without gyroscopic terms, several slabs per workgroup, and a coordinate whose
@@ -72,6 +73,29 @@ def test_derivative_and_step(dim, N, inertia, precision, tol):
     e = rel_l2(p.download_full(F), y)
     print("  two steps rel err %.2e" % e, flush=True)
     assert e < tol
+
+
+@pytest.mark.parametrize("N", [34, 38, 40, 42, 44, 46, 48, 62])
+def test_derivative_and_step_64(N):
+    test_derivative_and_step(2, N, "", "fp64", 1e-10)
+
+
+@pytest.mark.parametrize("N", [20, 40])
+def test_axes_of_different_ramps(N):
+    """X_2 of a ramp twice as steep: odd real circulants that differ by axis, which
+    the 34 to 62 point kernel's shared matrices must not take."""
+    print("case fold axes", N, flush=True)
+    B, L, dt = 3, 8.0, 0.01
+    Ffull = _full(B, 2, N, L, 60 + N)
+    X, _, MR, u, cells = operators(B, 2, N, L)
+    Xg = X.copy()
+    Xg[..., 1] *= 2.0
+    b = np.array(BT[:2])
+    ref = O.integrate(B, 2, N, Ffull, Xg, None, MR, b, G2, dt, L, u, cells, "RK2")
+    out = hpup.pendulum_propagate_reduced(Ffull, Xg, MR, b, G2, dt, L, u, cells, "RK2")
+    e = rel_l2(out, ref)
+    print("  rel err %.2e" % e, flush=True)
+    assert e < 1e-10
 
 
 @pytest.mark.parametrize("precision,tol", [("fp64", 1e-10), ("fp32", 2e-5)])
