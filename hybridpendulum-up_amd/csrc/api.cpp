@@ -420,6 +420,12 @@ template <class T> struct PlanT : PlanBase {
     void backward(const void* F, void* f, hipStream_t st) override {
         const XformDev<T> X = xform();
         ensure(G, sizeof(cT<T>) * (size_t)g_elems(model.B, nx));
+        if (model.dim == 0) {  // no omega axes
+            launch_beta_inv<T>(X, F, G.p, st);
+            launch_inv_ag<T>(X, G.p, f, st);
+            HPUP_HIP(hipGetLastError());
+            return;
+        }
         ensure(tmp, cbytes());
         if (half_omega(X)) {  // the Hermitian part on half of the rows
             launch_omega_half<T>(X, F, tmp.p, true, st);
