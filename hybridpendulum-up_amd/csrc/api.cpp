@@ -358,6 +358,7 @@ struct PlanBase {
     std::vector<double> xg_host;  // omega coordinates [ix][a]
     DevBuf xg_dev;
     void get_stat(const void* f, hpup_stat& out, double* fx, bool fit, hipStream_t st);
+    bool keep_rounding = false;  // hpup_plan_keep_rounding
     virtual int profile(void* F, int nreps, double* ms, int maxk, hipStream_t st) = 0;
     virtual const char* profile_name(int i) const = 0;
     virtual double profile_bytes(int i) const = 0;
@@ -394,13 +395,19 @@ template <class T> struct PlanT : PlanBase {
     }
     size_t cbytes() const { return sizeof(cT<T>) * (size_t)ncoef; }
 
-    // FP32 grids whose rounding 64-bit figures stand in (XformDev::keep): the
-    // reduced model's with a reset, whose densities get_stat reads, and 3-D grids
-    // of up to 16 points per axis, those of the restitution gradient
+    // FP32 plans in whose rounding 64-bit figures stand: those of the gradient
+    // sweeps (keep_rounding), and the reduced model's with a reset, whose densities
+    // get_stat reads.  They keep the drift kernels and DFTs of XformDev::keep.
+    bool keeps() const { return sizeof(T) == 4 && model.dim >= 2 && (keep_rounding || (model.dim == 2 && reset)); }
     XformDev<T> xform() const {
         XformDev<T> X = xf.view;
-        X.keep = sizeof(T) == 4 && (model.dim == 2 ? (bool)reset : model.dim == 3 && model.N <= 16);
+        X.keep = keeps() ? 1 : 0;
         return X;
+    }
+    DriftDev<T> drift_view() const {
+        DriftDev<T> D = dr.view;
+        D.keep = keeps() ? 1 : 0;
+        return D;
     }
     void forward(const void* f, void* F, hipStream_t st) override { forward_weighted(f, nullptr, 0, F, st); }
     // forward transform of the grid product f(R, x) wR[R * wstride]
@@ -470,7 +477,7 @@ template <class T> struct PlanT : PlanBase {
     // receives an event before and after each kernel (nk + 1 events).
     void stage(const void* Fin, const void* F0, void* Fout, const StageCoef<T>& sc, hipStream_t st,
                hipEvent_t* ev = nullptr) {
-        DriftDev<T> D = dr.view;
+        DriftDev<T> D = drift_view();
         // the fused kernel reads neighbouring rotation rows of Fin while other
         // workgroups write Fout, so the two must not alias (the three-pass
         // path reads Fin only through its own slab and may run in place)
@@ -741,7 +748,7 @@ template <class T> struct PlanT : PlanBase {
         static const char* names[3] = {"k_rotmix", "k_axis_outer", "k_drift_slab"};
         if (fused()) {
             if (i == 0) return "k_axis3_mfma";
-            return i == 1 ? drift_fused_name<T>(dr.view, den, bf16x3) : "";
+            return i == 1 ? drift_fused_name<T>(drift_view(), den, bf16x3) : "";
         }
         return (i >= 0 && i < 3) ? names[i] : "";
     }
@@ -989,6 +996,12 @@ int hpup_plan_axpy_stage(hpup_plan* p, const void* in, const void* F0, double sc
 int hpup_plan_adjoint_stage(hpup_plan* p, const void* ybar, const void* y, double scale, void* ybar_out,
                             void* fbar, int fbar_init, double* grad, void* stream) {
     return guard([&] { p->impl->adjoint_stage(ybar, y, scale, ybar_out, fbar, fbar_init, grad, (hipStream_t)stream); });
+}
+int hpup_plan_keep_rounding(hpup_plan* p) {
+    return guard([&] {
+        HPUP_REQUIRE(p, HPUP_ERR_ARG, "null argument");
+        p->impl->keep_rounding = true;
+    });
 }
 int hpup_plan_step_stages(hpup_plan* p, const void* F, void* const* ys, void* F_next, void* stream) {
     return guard([&] {

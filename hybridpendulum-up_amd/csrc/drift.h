@@ -43,6 +43,7 @@ template <class T> struct DriftDev {
     int ramp;
     int odd;     // ... and the real circulants are odd
     int same12;  // ... and those of axes 1 and 2 are equal
+    int keep;    // FP32: not the folded kernel (see XformDev::keep)
     T c0[3];
     // structured mixing coefficients: -i CG_1 real, -i CG_2 imaginary,
     // CG_3 zero, u_1 imaginary, u_2 real (the pendulum models)
@@ -141,8 +142,8 @@ template <class T> struct XformDev {
     // rows r <= B (angle), k < B (frequency)
     const T* agF;
     const T* agI;
-    // FP32 only: the grid's 64-bit figures (statistics, gradients) are taken from
-    // it, and its transforms keep the direct (alpha, gamma) stages and (k1, k2)
+    // FP32 only: 64-bit figures (statistics, gradients) are taken from the plan's
+    // grids, and its transforms keep the direct (alpha, gamma) stages and (k1, k2)
     // DFTs, in whose rounding those figures stand, with these tables
     int keep;
     const cT<T>* twMB;  // [32][32] e^{i pi (r - (B-1)) t / B} for r < 2B-1, t < 2B, zero elsewhere, then its

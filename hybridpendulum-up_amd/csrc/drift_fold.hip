@@ -29,7 +29,7 @@
 // units 32 %, tag lookups 60 %, HBM 75 % of a copy's rate).  The six gathered
 // source rows cost 0.28 of 1.37 ms, the streams alone 0.83 ms.  Against
 // k_drift_fused / k_drift_fused_c (ms per launch, average of a step's four):
-//   B = 15, N = 30: FP32 1.63 -> 1.37, FP64 3.00 -> 2.48;  B = 30, N = 20, FP32: 5.54 -> 4.04.
+//   B = 15, N = 30: FP32 1.63 -> 1.35, FP64 3.00 -> 2.52;  B = 30, N = 20, FP32: 5.54 -> 3.86.
 // Tried and not kept: the slab in its natural order with 16-byte loads and the
 // folding in LDS (FP64 N = 30: 2.80, FP32 N = 20: 4.63), mixing tables prefetched
 // through LDS (FP32 1.57), three waves per SIMD in FP64 (spills, 3.08).
@@ -190,6 +190,9 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
     };
     if (AHEAD && sl < hi) load_own(rnext, kg);
     while (sl < hi) {
+        // a wave's priority rises through a slab (mixing, products, epilogue), so that
+        // workgroups drift apart in phase instead of queueing for one unit: 2-3 %
+        __builtin_amdgcn_s_setprio(0);
         const int r = rnext;
         // the group's first k3; a last group that would pass N starts earlier and
         // leaves the slabs it shares with the previous group to that one
@@ -303,6 +306,7 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
         }
         if (AHEAD && sl + per < hi) load_own(rnext, kn);
         __syncthreads();  // 1: the planes are complete
+        __builtin_amdgcn_s_setprio(1);
 
         // ---- everything but T1 V1
         acc_t cr[XS], ci[XS];
@@ -393,6 +397,7 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
             }
         }
         __syncthreads();  // 3: the result planes are complete
+        __builtin_amdgcn_s_setprio(2);
 
         // ---- dF = unfolded planes + W, epilogue (as k_drift_fused)
         cT<T> y[4], qv[4];
@@ -750,16 +755,14 @@ __global__ __launch_bounds__(512, 2) void k_drift_fold64(DriftDev<double> D, Mix
 
 // ---------------------------------------------------------- launcher -----
 
-// Sizes.  FP64: 3-D 1.07-1.54x (B = 8), 2-D 1.1-1.4x (B = 20) faster than the kernels
-// that serve the others, but for N = 16, which fills k_drift_fused_c's tile while its
-// planes of nine points do not fill a K step here (3-D 0.82x, 2-D 1.04x).  FP32: 3-D
-// from N = 18 on, 1.10-1.39x.  Smaller 3-D grids and the reduced model keep the other
-// kernels' rounding, in which the 64-bit gradients of an FP32 sweep stand (they
-// would move by 1e-8; N <= 14 would gain 1.04-1.32x, 2-D 0.76-1.38x).
+// Sizes, against the kernels that serve the others (B = 8 in 3-D, B = 20 in 2-D):
+// 3-D 1.04-1.54x faster at N = 4 .. 14 and 18 .. 30, 2-D 1.1-1.4x in FP64 and, from
+// N = 14 on, 1.03-1.38x in FP32.  N = 16 fills k_drift_fused_c's tile while its planes
+// of nine points do not fill a K step here (3-D FP64 0.82x, 2-D FP32 0.90x); small
+// 2-D FP32 slabs leave most of a workgroup idle (0.76-0.89x).
 template <class T> bool drift_fold_ok(const DriftDev<T>& D) {
-    if (!D.ramp || !D.odd || !D.smix || D.adj || D.N % 2 || D.N > 30) return false;
-    if (sizeof(T) == 4) return D.dim == 3 && D.N >= 18;
-    return D.N >= 4 && D.N != 16;
+    if (!D.ramp || !D.odd || !D.smix || D.adj || (sizeof(T) == 4 && D.keep)) return false;
+    return D.N % 2 == 0 && D.N <= 30 && D.N != 16 && D.N >= (D.dim == 2 && sizeof(T) == 4 ? 14 : 4);
 }
 
 template <int KS, int NQ>
@@ -807,19 +810,17 @@ void launch_drift_fold(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fi
                        void* Fout, const StageCoef<T>& sc, hipStream_t st) {
     HPUP_REQUIRE(drift_fold_ok<T>(D) && !sc.read_acc && !sc.write_acc,
                  HPUP_ERR_UNSUPPORTED, "folded drift: odd real circulants, structured mixing, no stage sums");
-    if constexpr (sizeof(T) == 8) {
-        const int KS = (D.N / 2 + 1 + 3) / 4;
-        if (D.dim == 2) {
-            switch (KS) {
-            case 1: return fold_t<T, 2, 1, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
-            case 2: return fold_t<T, 2, 2, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
-            case 3: return fold_t<T, 2, 3, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
-            default: return fold_t<T, 2, 4, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
-            }
+    const int KS = (D.N / 2 + 1 + 3) / 4;
+    if (D.dim == 2) {
+        if constexpr (sizeof(T) == 8) {
+            if (KS == 1) return fold_t<T, 2, 1, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
         }
-        if (KS == 1) return fold_t<T, 3, 1, 4>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 4, 6
-        if (KS == 2) return fold_t<T, 3, 2, 4>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 8 .. 14
+        if (KS <= 2) return fold_t<T, 2, 2, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
+        if (KS == 3) return fold_t<T, 2, 3, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
+        return fold_t<T, 2, 4, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
     }
+    if (KS == 1) return fold_t<T, 3, 1, 4>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 4, 6
+    if (KS == 2) return fold_t<T, 3, 2, 4>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 8 .. 14
     // slabs per workgroup: as many quarter planes as 256 threads hold
     if (D.N <= 20) return fold_t<T, 3, 3, 2>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 18, 20
     if (D.N == 22) return fold_t<T, 3, 3, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);

@@ -84,7 +84,7 @@ EXPORTS = [
     "hpup_plan_adjoint_stage", "hpup_plan_axpy_stage",
     "hpup_plan_set_reset", "hpup_plan_reset_region", "hpup_plan_reset", "hpup_plan_hybrid_step",
     "hpup_plan_reset_adjoint", "hpup_plan_reset_eps_grad", "hpup_plan_adjoint_stage_noalloc",
-    "hpup_plan_step_stages", "hpup_plan_adjoint_step",
+    "hpup_plan_keep_rounding", "hpup_plan_step_stages", "hpup_plan_adjoint_step",
 ]
 
 
@@ -118,6 +118,7 @@ def lib():
                                               ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p,
                                               ctypes.c_void_p]
         L.hpup_plan_adjoint_stage_noalloc.argtypes = L.hpup_plan_adjoint_stage.argtypes
+        L.hpup_plan_keep_rounding.argtypes = [ctypes.c_void_p]
         L.hpup_plan_step_stages.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p),
                                             ctypes.c_void_p, ctypes.c_void_p]
         L.hpup_plan_adjoint_step.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p),
@@ -543,6 +544,12 @@ class Plan:
                                              1 if fbar_init else 0, ctypes.c_void_p(grad.data_ptr()),
                                              self._stream()))
         return out
+
+    def keep_rounding(self):
+        """FP32 plans: the order of sums that a gradient sweep's 64-bit gradients
+        stand on, instead of the faster kernels."""
+        _check(lib().hpup_plan_keep_rounding(self._h))
+        return self
 
     def step_stages(self, F, ys, F_next=None):
         """Forward model plans: ys (s - 1 coefficient tensors) receive the Horner

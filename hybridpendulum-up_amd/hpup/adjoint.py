@@ -46,7 +46,7 @@ class Gradient:
         self.N = N
         self.b = np.array(tuple(b)[:2], dtype=np.float64)
         self.G = np.zeros((2, 2)) if G is None else np.asarray(G, dtype=np.float64).reshape(2, 2).copy()
-        self.fwd = Plan(B, 2, N, **kw)
+        self.fwd = Plan(B, 2, N, **kw).keep_rounding()
         self.adj = Plan(B, 2, N, operator=1, **kw)
 
     def run(self, F0, nsteps, dJ, checkpoint=None):
@@ -202,7 +202,7 @@ class HybridGradient:
         kw = dict(L=L, b=b, G=G, Jt=Jt, dt=dt, method=method, precision=precision)
         self.dt = dt
         self.reset = dict(reset)
-        self.fwd = Plan(B, dim, N, **kw)
+        self.fwd = Plan(B, dim, N, **kw).keep_rounding()
         self.fwd.set_reset(**self.reset)
         self.adj = Plan(B, dim, N, operator=1, **kw)
         self.ta = TransformAdjoint(self.fwd)

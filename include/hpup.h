@@ -292,6 +292,12 @@ int hpup_plan_axpy_stage(hpup_plan* plan, const void* in, const void* F0, double
 int hpup_plan_adjoint_stage(hpup_plan* plan, const void* ybar, const void* y, double scale, void* ybar_out,
                             void* fbar, int fbar_init, double* grad, void* stream);
 
+/* FP32 plans: keeps the drift kernels and DFTs that a gradient sweep's 64-bit
+ * parameter gradients stand on, in the order of their sums, instead of the faster
+ * ones, which would move such figures by about 1e-7 (no counterpart in the
+ * reference; callers: gradient sweeps, before the plan's first use).  Plans of the
+ * reduced model do so by themselves once they have a reset.  FP64 plans: no effect. */
+int hpup_plan_keep_rounding(hpup_plan* plan);
 /* The stage values of one step of a forward model plan (no counterpart in the
  * reference; callers: gradient sweeps that keep them for the reverse pass).
  * With y_0 = F and the Horner stages y_j = F + c_j dt A y_{j-1} (c = 1 Euler;

@@ -3,7 +3,7 @@ against the oracle at the edges of its range: the smallest and largest grids of
 each tile depth (6 | 10, 14 | 18, 22 | 24, 30; the reduced model's FP64 kernel for
 34 to 62 points at 34, 38 | 40, 42 | 44, 46 | 48 | 62: one and two quartets a thread), slab groups that do not divide
 the k3 axis (10 = 4 + 4 + 2, 14 = 3 x 4 + 2), grids that keep another kernel
-(16; FP32 2-D and small 3-D grids), full diffusion matrices, inertias with
+(16; small FP32 2-D grids), full diffusion matrices, inertias with
 and without gyroscopic terms, several slabs per workgroup, and a coordinate whose
 real circulant is not odd, which the folding must not take.
 

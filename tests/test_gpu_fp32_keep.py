@@ -1,8 +1,8 @@
-"""FP32 grids behind 64-bit figures (the reduced model with a reset, 3-D grids of up to
-16 points per axis) keep the direct (alpha, gamma) stages and the Toeplitz
-or direct (k1, k2) DFTs: against the FP64 plan at the edges of those kernels (B =
-16 | 17, the FFT bandlimit 15; N = 32 | 34, 64; the smallest grids), and the same
-plan's transforms before it has a reset, which take the MFMA forms in 2-D.
+"""FP32 plans behind 64-bit figures (the reduced model with a reset, the gradient
+sweeps' plans: Plan.keep_rounding) keep the direct (alpha, gamma) stages and the
+Toeplitz or direct (k1, k2) DFTs: against the FP64 plan at the edges of those
+kernels (B = 16 | 17, the FFT bandlimit 15; N = 32 | 34, 64; the smallest grids), and
+the same plan's transforms before it keeps them, which take the MFMA forms.
 
 Tolerance: relative L2 2e-5, the other FP32 tests' (a transform is about 2 N + 6 B
 products deep, rounding below 300 * 6e-8 = 1.8e-5)."""
@@ -34,6 +34,8 @@ def test_against_fp64(dim, B, N):
         rt = torch.float64 if precision == "fp64" else torch.float32
         F = p.forward(f0.to(rt).cuda())
         b = p.backward(F, p.empty_grid())
+        if dim == 3:
+            p.keep_rounding()
         p.set_reset(**WALL, **(dict(tilt=0.1, jacobian=True) if dim == 3 else {}))
         H, f = F.clone(), p.empty_grid()
         p.hybrid_step(H, f, 1)
