@@ -669,11 +669,16 @@ template <class T> struct PlanT : PlanBase {
         const int ns = horner(c);
         ensure(Ya, cbytes());
         ensure(Yb, cbytes());
+        // every stage leaves its partial sums in a part of gpart of its own; the
+        // last one's launch adds them all to gout, in the stages' order
+        ensure(gpart, sizeof(double) * kGradMaxWG * 5 * 4);
+        GradScales sc{};
         const void* ybar = lam;
-        for (int j = ns - 1; j >= 0; j--) {
+        for (int j = ns - 1, q = 0; j >= 0; j--, q++) {
             const void* y = j == 0 ? F : ys[j - 1];
             void* out = (ybar == Ya.p) ? Yb.p : Ya.p;
-            adjoint_stage(ybar, y, c[j], out, Fbar, j == ns - 1 ? 1 : 0, gout, st, false);
+            sc.s[q] = c[j];
+            adjoint_stage_at(ybar, y, c[j], out, Fbar, q == 0 ? 1 : 0, gout, gpart.as<double>(), q, sc, j == 0 ? ns : 0, st);
             ybar = out;
         }
     }
@@ -685,12 +690,6 @@ template <class T> struct PlanT : PlanBase {
     // (grad_scratch) instead of the plan's buffer, and nothing is allocated
     void adjoint_stage(const void* ybar, const void* y, double scale, void* out, void* fbar, int fbar_init,
                        double* gout, hipStream_t st, bool noalloc) override {
-        HPUP_REQUIRE(has_drift && fused() && dr.view.adj, HPUP_ERR_UNSUPPORTED,
-                     "adjoint_stage needs an adjoint operator plan (operator kind 1, N <= 32)");
-        HPUP_REQUIRE(ybar && y && out && gout, HPUP_ERR_ARG, "null argument");
-        HPUP_REQUIRE(ybar != out && y != out, HPUP_ERR_ARG, "adjoint stage cannot run in place");
-        HPUP_REQUIRE(fbar != ybar && fbar != y && fbar != out, HPUP_ERR_ARG, "fbar must not alias the stage arrays");
-        HPUP_REQUIRE(model.dim == 2, HPUP_ERR_UNSUPPORTED, "parameter gradients: reduced model (dim 2) only");
         double* part;
         if (noalloc) {
             int dev = 0;
@@ -700,13 +699,27 @@ template <class T> struct PlanT : PlanBase {
             ensure(gpart, sizeof(double) * kGradMaxWG * 5);
             part = gpart.as<double>();
         }
+        adjoint_stage_at(ybar, y, scale, out, fbar, fbar_init, gout, part, 0, GradScales{{scale, 0, 0, 0}}, 1, st);
+    }
+    // the same with the partial sums at part + q kGradMaxWG 5; nred > 0: the
+    // first nred stages' sums, weighted by sc, are added to gout after this one
+    void adjoint_stage_at(const void* ybar, const void* y, double scale, void* out, void* fbar, int fbar_init,
+                          double* gout, double* part, int q, const GradScales& sc, int nred, hipStream_t st) {
+        HPUP_REQUIRE(has_drift && fused() && dr.view.adj, HPUP_ERR_UNSUPPORTED,
+                     "adjoint_stage needs an adjoint operator plan (operator kind 1, N <= 32)");
+        HPUP_REQUIRE(ybar && y && out && gout, HPUP_ERR_ARG, "null argument");
+        HPUP_REQUIRE(ybar != out && y != out, HPUP_ERR_ARG, "adjoint stage cannot run in place");
+        HPUP_REQUIRE(fbar != ybar && fbar != y && fbar != out, HPUP_ERR_ARG, "fbar must not alias the stage arrays");
+        HPUP_REQUIRE(model.dim == 2, HPUP_ERR_UNSUPPORTED, "parameter gradients: reduced model (dim 2) only");
         DriftDev<T> D = dr.view;
         D.gy = y;
         D.gacc = fbar;
         D.gacc_init = fbar_init ? 1 : 0;
-        D.gpart = part;
+        D.gpart = part + (int64_t)q * kGradMaxWG * 5;
+        D.gbase = part;
         D.gout = gout;
-        D.gscale = scale;
+        D.gscales = sc;
+        D.gns = nred;
         launch_drift_fused<T>(D, dr.mix, ybar, Z3.p, nullptr, out, ACC.p,
                               StageCoef<T>{(T)scale, 0, 1, 0, 0, 0, 0, 0, 1}, false, st);
         HPUP_HIP(hipGetLastError());

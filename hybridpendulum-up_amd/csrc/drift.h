@@ -20,6 +20,10 @@ void allow_lds(const void* kernel, size_t bytes);
 // LDS size).
 unsigned persistent_blocks(const void* kernel, int64_t nwork, int threads, size_t lds);
 
+struct GradScales {
+    double s[4];
+};
+
 template <class T> struct DriftDev {
     int B, dim, N;
     int64_t nx, nrc;
@@ -54,14 +58,17 @@ template <class T> struct DriftDev {
     // (e3 of the adjoint tables is the conjugate of the forward one)
     const cT<T>* s3;
     // gradient stage (adj only, gpart non-null): forward stage value y, the
-    // sweep's running sum, the workgroups' partial sums (kGradMaxWG x 5), and
-    // out[5] += gscale * sums
+    // sweep's running sum and the workgroups' partial sums (kGradMaxWG x 5)
     const void* gy;
     void* gacc;      // nullable: gacc += the stage output
     int gacc_init;   // gacc = the stage input + the stage output instead (the sweep's first stage)
     double* gpart;
+    // with gns > 0 the launch ends with out[5] += gscales[j] * (sum of the
+    // partials of stage j), j = 0 .. gns - 1, from gbase + j kGradMaxWG 5
+    double* gbase;
     double* gout;
-    double gscale;
+    GradScales gscales;
+    int gns;
 };
 constexpr int kGradMaxWG = 4096;
 constexpr int kMaxDevices = 64;

@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
     T m1[KS], m2[KS], d1[KS], d2[KS], rr1, rr2;
     {
         auto mats = [&](const cT<T>* kap, int p, T c0, T b, T* m, T* d, T& rr) {
-            auto K = [&](int j) { return kap[((j % N) + N) % N].y; };
+            auto K = [&](int j) { return kap[j < 0 ? j + N : j < N ? j : j - N].y; };  // -N < j < 2 N
             const T kco = lr <= H ? D.kc[lr] : T(0);
 #pragma unroll
             for (int s = 0; s < KS; s++) {
@@ -470,7 +470,7 @@ __global__ __launch_bounds__(512, 2) void k_drift_fold64(DriftDev<double> D, Mix
     T* sM = reinterpret_cast<T*>(pA + 2 * OV);
     auto entry = [&](const cT<T>* kap, int o, int a, T& oe, T& eo) {
         const bool in = a <= H && o <= H, self = a == 0 || a == H;
-        auto K = [&](int j) { return kap[((j % N) + N) % N].y; };
+        auto K = [&](int j) { return kap[j < 0 ? j + N : j < N ? j : j - N].y; };  // -N < j < 2 N
         const T km = in ? K(o - a) : T(0), kp = in ? K(o + a) : T(0);
         oe = !in || o == 0 || o == H ? T(0) : T(0.25) * (self ? km : km + kp);  // even -> odd
         eo = !in || self ? T(0) : T(0.25) * (km - kp);                        // odd -> even

@@ -479,6 +479,7 @@ __global__ __launch_bounds__(256, (GRAD ? (sizeof(T) == 4 ? 3 : 2) : FusedWaves<
     int r = sl % nrc;
     int k3 = sl / nrc;
     while (sl < hi) {
+        __builtin_amdgcn_s_setprio(0);
         // zo is 0, produced by an opaque move each iteration: indices derived
         // from it are recomputed per slab instead of being hoisted out of the
         // loop (one register each for every address), which keeps the kernel
@@ -613,6 +614,7 @@ __global__ __launch_bounds__(256, (GRAD ? (sizeof(T) == 4 ? 3 : 2) : FusedWaves<
             Wv[v] = wv;
         }
         __syncthreads();  // plane A complete; the V planes of the previous slab are consumed
+        __builtin_amdgcn_s_setprio(1);
 
         cT<T> P1[4], P2[4];
         if constexpr (ADJ) {
@@ -682,6 +684,7 @@ __global__ __launch_bounds__(256, (GRAD ? (sizeof(T) == 4 ? 3 : 2) : FusedWaves<
             pc_im[k2 * kPad + k1w] = ok[v] ? V2[v].y : T(0);
         }
         __syncthreads();  // V planes complete; plane A is consumed
+        __builtin_amdgcn_s_setprio(2);
         cT<T> Q1[4], Q2[4];
         gm.t1(pb_re, pb_im, Q1, D.c0[0]);
         gm.t2(pc_re, pc_im, Q2, D.c0[1]);
@@ -1115,6 +1118,7 @@ __global__ __launch_bounds__(256, CompactWaves<T>::n) void k_drift_fused_c(Drift
     int r = sl % nrc;
     int k3 = sl / nrc;
     while (sl < hi) {
+        __builtin_amdgcn_s_setprio(0);
         const int64_t base = ((int64_t)r * nz + k3) * NN;
         const cT<T>* Fb = Fin + base;
         const T kc3 = DIM == 3 ? as_const<T>(D.kc)[k3] : T(0), kd3 = DIM == 3 ? as_const<T>(D.kd)[k3] : T(0);
@@ -1222,6 +1226,7 @@ __global__ __launch_bounds__(256, CompactWaves<T>::n) void k_drift_fused_c(Drift
                 pc_im[pos[i]] = V2[i].y;
             }
         __syncthreads();  // 1: A, B, C complete
+        __builtin_amdgcn_s_setprio(1);
 
         // ---- tile: P GEMMs, the gyroscopic P2 term into B, the damping terms into D
         {
@@ -1256,6 +1261,7 @@ __global__ __launch_bounds__(256, CompactWaves<T>::n) void k_drift_fused_c(Drift
             }
         }
         __syncthreads();  // 3: Q in A complete
+        __builtin_amdgcn_s_setprio(2);
 
         // ---- compact: dF = Q + D + S', epilogue (as k_drift_fused)
         cT<T> q[EPL], f0v[EPL], acv[EPL];
@@ -1307,29 +1313,36 @@ __global__ __launch_bounds__(256, CompactWaves<T>::n) void k_drift_fused_c(Drift
     }
 }
 
-// out[i] += scale * sum over the workgroups' partials, one workgroup of
-// kGradRedThreads: thread t sums partials t, t + kGradRedThreads, ... in that
-// order, then a fixed pairwise tree combines the threads, so the result does
-// not depend on timing (the partials are independent loads, all in flight)
+// out[i] += scale_j * (sum over the workgroups' partials of stage j), j = 0 .. ns - 1
+// in turn, for the stages of a reverse step at once: 256 threads per stage.  Thread t
+// sums partials t, t + kGradRedThreads, ... in that order, then a fixed pairwise
+// tree combines the threads, so the result does not depend on timing (the
+// partials are independent loads, all in flight).  One launch a stage took 4.6 us
+// each, 3 % of a sweep at B = 15, N = 30.
 constexpr int kGradRedThreads = 256;
-__global__ __launch_bounds__(kGradRedThreads) void k_grad_reduce(const double* __restrict__ part, int nwg, double scale,
-                                                                 double* __restrict__ out) {
-    __shared__ double red[5][kGradRedThreads];
-    const int t = threadIdx.x;
+__global__ __launch_bounds__(4 * kGradRedThreads) void k_grad_reduce(const double* __restrict__ part, int nwg, GradScales sc,
+                                                                     int ns, double* __restrict__ out) {
+    __shared__ double red[4][5][kGradRedThreads];
+    const int t = threadIdx.x, j = threadIdx.y;
+    const double* p = part + (int64_t)j * kGradMaxWG * 5;
     double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     for (int g = t; g < nwg; g += kGradRedThreads)
 #pragma unroll
-        for (int i = 0; i < 5; i++) s[i] += part[(int64_t)g * 5 + i];
+        for (int i = 0; i < 5; i++) s[i] += p[(int64_t)g * 5 + i];
 #pragma unroll
-    for (int i = 0; i < 5; i++) red[i][t] = s[i];
+    for (int i = 0; i < 5; i++) red[j][i][t] = s[i];
     __syncthreads();
     for (int h = kGradRedThreads / 2; h > 0; h >>= 1) {
         if (t < h)
 #pragma unroll
-            for (int i = 0; i < 5; i++) red[i][t] += red[i][t + h];
+            for (int i = 0; i < 5; i++) red[j][i][t] += red[j][i][t + h];
         __syncthreads();
     }
-    if (t < 5) out[t] += scale * red[t][0];
+    if (j == 0 && t < 5) {
+        double o = out[t];
+        for (int q = 0; q < ns; q++) o = fma(sc.s[q], red[q][t][0], o);
+        out[t] = o;
+    }
 }
 
 // ------------------------------------------------------------ axis 3 ----
@@ -1643,8 +1656,9 @@ void launch_drift_fused(const DriftDev<T>& D, const MixDev<T>& MX, const void* F
                                                                                       nslab, st)
                        : launch_fused_t<T, GemmF<T, true>, 2, false, true, true>(D, MX, Fin, Z3, F0, Fout, ACC, sc,
                                                                                 nslab, st);
-            hipLaunchKernelGGL(k_grad_reduce, dim3(1), dim3(kGradRedThreads), 0, st, (const double*)D.gpart, (int)nwg,
-                               (double)D.gscale, D.gout);
+            if (D.gns > 0)
+                hipLaunchKernelGGL(k_grad_reduce, dim3(1), dim3(kGradRedThreads, D.gns), 0, st, (const double*)D.gbase,
+                                   (int)nwg, D.gscales, D.gns, D.gout);
             return;
         }
         if (D.smix) launch_fused_t<T, GemmF<T, true>, 2, false, true, false, true>(D, MX, Fin, Z3, F0, Fout, ACC, sc, nslab, st);
