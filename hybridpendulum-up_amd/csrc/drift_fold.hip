@@ -756,13 +756,18 @@ __global__ __launch_bounds__(512, 2) void k_drift_fold64(DriftDev<double> D, Mix
 // ---------------------------------------------------------- launcher -----
 
 // Sizes, against the kernels that serve the others (B = 8 in 3-D, B = 20 in 2-D):
-// 3-D 1.04-1.54x faster at N = 4 .. 14 and 18 .. 30, 2-D 1.1-1.4x in FP64 and, from
-// N = 14 on, 1.03-1.38x in FP32.  N = 16 fills k_drift_fused_c's tile while its planes
+// 3-D 1.04-1.58x faster at N = 4 .. 14 and 18 .. 30, 2-D 1.1-1.4x in FP64 and, from
+// N = 18 on, 1.03-1.38x in FP32.  N = 16 fills k_drift_fused_c's tile while its planes
 // of nine points do not fill a K step here (3-D FP64 0.82x, 2-D FP32 0.90x); small
-// 2-D FP32 slabs leave most of a workgroup idle (0.76-0.89x).
+// 2-D FP32 slabs leave most of a workgroup idle (0.76-1.04x up to N = 14).  In 3-D up to
+// N = 14 a workgroup takes four slabs, so few rows leave workgroups without any: below
+// 1.25 rounds of the resident ones it is the slower (FP64 495 groups 0.99x, 660 1.27x;
+// FP32 858 groups 0.87-0.91x, 1144 1.08x, 1365 0.98-1.14x).
 template <class T> bool drift_fold_ok(const DriftDev<T>& D) {
     if (!D.ramp || !D.odd || !D.smix || D.adj || (sizeof(T) == 4 && D.keep)) return false;
-    return D.N % 2 == 0 && D.N <= 30 && D.N != 16 && D.N >= (D.dim == 2 && sizeof(T) == 4 ? 14 : 4);
+    if (D.N % 2 || D.N < 4 || D.N > 30 || D.N == 16) return false;
+    if (D.dim == 2) return sizeof(T) == 8 || D.N >= 18;
+    return D.N > 14 || D.nrc * ((D.N + 3) / 4) >= (sizeof(T) == 8 ? 640 : 1280);
 }
 
 template <int KS, int NQ>
@@ -814,8 +819,8 @@ void launch_drift_fold(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fi
     if (D.dim == 2) {
         if constexpr (sizeof(T) == 8) {
             if (KS == 1) return fold_t<T, 2, 1, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
+            if (KS == 2) return fold_t<T, 2, 2, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
         }
-        if (KS <= 2) return fold_t<T, 2, 2, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
         if (KS == 3) return fold_t<T, 2, 3, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
         return fold_t<T, 2, 4, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
     }
