@@ -106,7 +106,14 @@ template <class T> bool drift_fold_ok(const DriftDev<T>& D);
 template <class T>
 void launch_drift_fold(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0,
                        void* Fout, const StageCoef<T>& sc, hipStream_t st);
-// the same for the reduced model's FP64 grids of 34 to 62 points per axis
+// one wave and one matrix tile per slab, N <= 16: taken where drift_tile_ok (real
+// circulants, structured mixing, forward operator; sizes at its definition), with no
+// grid gravity and no stage sums
+template <class T> bool drift_tile_ok(const DriftDev<T>& D);
+template <class T>
+void launch_drift_tile(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0,
+                       void* Fout, const StageCoef<T>& sc, hipStream_t st);
+// k_drift_fold's form for the reduced model's FP64 grids of 34 to 62 points per axis
 bool drift_fold64_ok(const DriftDev<double>& D);
 void launch_drift_fold64(const DriftDev<double>& D, const MixDev<double>& MX, const void* Fin, const void* F0, void* Fout,
                          const StageCoef<double>& sc, hipStream_t st);

@@ -1,5 +1,6 @@
-// Parity-folded drift kernel for omega grids up to 30 points per axis (the
-// forward operator of the pendulum models: real circulants, structured mixing).
+// Drift kernels for omega grids of up to 30 points per axis, k_drift_fold (18 to 30
+// points, parity-folded) and k_drift_tile (up to 16), and of 34 to 62 points in the
+// reduced model in FP64, k_drift_fold64 (the forward operator of the pendulum models: real circulants, structured mixing).
 //
 // k_drift_fold evaluates the derivative of the (r, k3) slabs it visits with the
 // integrator epilogue, as k_drift_fused does (see drift_mfma.hip for the terms):
@@ -753,21 +754,275 @@ __global__ __launch_bounds__(512, 2) void k_drift_fold64(DriftDev<double> D, Mix
     }
 }
 
+// ------------------------------------------------------------ N <= 16 ----
+//
+// Omega grids of up to 16 points per axis: a slab is one 16 x 16 tile of the matrix
+// instruction, unfolded, and one wave holds it whole, four elements a lane in the
+// accumulators' layout.  The circulant T_p = c0 1 1^T + i K_p is a real 16 x 16 product
+// and an axis sum; results and the mixing stay in registers, F, V2 and then V1 go through
+// LDS to become operands.  A workgroup is one wave, so nothing waits for another wave:
+// with four waves to a slab and three barriers the same work took two to three times as
+// long (k_drift_fused_c; B = 12, N = 16 FP64 485 -> 186 us, FP32 222 -> 108 us; B = 20, 2-D,
+// N = 14 FP64 142 -> 45 us, FP32 64 -> 26 us; k_drift_fold 1.2-1.7 times k_drift_fused_c's
+// rate at N <= 14).  Bound by the gathered rows' latency: two (FP64) and four waves a SIMD.
+template <class T, int DIM>
+__global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> D, MixDev<T> MX, const cT<T>* Fin,
+                                                                    const cT<T>* __restrict__ Z3, const cT<T>* F0,
+                                                                    cT<T>* Fout, StageCoef<T> sc, int nslab) {
+    using MF = Mfma<T>;
+    using acc_t = typename MF::acc;
+    constexpr int NC = DIM + 2, MB = 2, RS = 17;
+    __shared__ cT<T> pF[16 * RS], pV[16 * RS];  // F and then V1; V2
+    const int N = D.N, NN = N * N, nz = DIM == 3 ? N : 1;
+    const int lane = threadIdx.x, lr = lane & 15, lq = lane >> 4;
+    for (int i = lane; i < 16 * RS; i += 64) pF[i] = pV[i] = czero<T>();
+
+    // matrices, entry [out lr][in 4 s + lq]
+    T m1[4], m2[4];
+    const T k1o = lr < N ? D.b[0] * D.kc[lr] : T(0), k2o = lr < N ? D.b[1] * D.kc[lr] : T(0);  // b kc of the outputs
+    const T c1 = lr < N ? D.c0[0] : T(0), c2 = lr < N ? D.c0[1] : T(0);
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const int a = 4 * s + lq, j = lr - a;
+        const bool in = a < N && lr < N;
+        m1[s] = in ? D.kap[j < 0 ? j + N : j].y : T(0);
+        m2[s] = in ? D.kap[N + (j < 0 ? j + N : j)].y : T(0);
+    }
+    // the lane's elements (k2, k1 = lr)
+    unsigned ob[4];
+    bool ok[4];
+    int ps[4];
+    T kc2[4], dd0[4];
+    const T kc1 = lr < N ? D.kc[lr] : T(0);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+        const int k2 = MF::orow(lq, v);
+        ok[v] = lr < N && k2 < N;
+        ob[v] = ok[v] ? (unsigned)(k2 * N + lr) * (unsigned)sizeof(cT<T>) : 0u;
+        ps[v] = k2 * RS + lr;
+        kc2[v] = ok[v] ? D.kc[k2] : T(0);
+        // D(k) = sum_i G_ii kd(k_i) - sum_{i != j} G_ij kc(k_i) kc(k_j)
+        dd0[v] = ok[v] ? D.G[0] * D.kd[lr] + D.G[DIM + 1] * D.kd[k2] - (D.G[1] + D.G[DIM]) * kc1 * kc2[v] : T(0);
+    }
+    const T g22 = DIM == 3 ? D.G[8] : T(0), g02 = DIM == 3 ? D.G[2] + D.G[6] : T(0), g12 = DIM == 3 ? D.G[5] + D.G[7] : T(0);
+    const bool gyro = DIM == 3 && D.has_gyro;
+    const int orw = lr * RS + lq, ocl = lq * RS + lr;
+    __syncthreads();
+
+    const int nrc = (int)D.nrc, TS = MX.TS;
+    const int nxcd = gridDim.x >= 8 ? 8 : 1;
+    const int per = (int)gridDim.x / nxcd;
+    const int xcd = (int)blockIdx.x % nxcd;
+    const int hi = (int)((int64_t)nslab * (xcd + 1) / nxcd);
+    int sl = (int)((int64_t)nslab * xcd / nxcd) + (int)blockIdx.x / nxcd;  // slab sl: row sl % nrc of the walk, k3 = sl / nrc
+    const int dr = per % nrc, dk = per / nrc;
+    int rp = sl % nrc, k3 = sl / nrc;
+    const kc_ptr<int32_t> ord = as_const<int32_t>(MX.order);
+    while (sl < hi) {
+        const int r = ord[rp];
+        const int64_t base = ((int64_t)r * nz + k3) * NN;
+        const T kc3 = DIM == 3 ? as_const<T>(D.kc)[k3] : T(0), kd3 = DIM == 3 ? as_const<T>(D.kd)[k3] : T(0);
+        cT<T> fo[4], Zv[4], W[4], V1[4], V2[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            fo[v] = *at_b(Fin + base, ob[v]);
+            Zv[v] = DIM == 3 ? ld_once<T>(at_b(Z3 + base, ob[v])) : czero<T>();
+        }
+        const kc_ptr<int32_t> srcT = as_const<int32_t>(MX.src) + (int64_t)r * TS;
+        const kc_ptr<T> coefT = as_const<T>((const T*)MX.coef) + 2 * (int64_t)r * TS * NC;
+#pragma unroll
+        for (int v = 0; v < 4; v++) W[v] = V1[v] = V2[v] = czero<T>();
+        for (int t0 = 0; t0 < TS; t0 += MB) {
+            int src[MB];
+            cT<T> fv[MB][4];
+#pragma unroll
+            for (int u = 0; u < MB; u++) src[u] = t0 + u < TS ? srcT[t0 + u] : -1;
+#pragma unroll
+            for (int u = 0; u < MB; u++) {
+                const cT<T>* Fs = Fin + ((int64_t)(src[u] < 0 ? 0 : (src[u] & 0xffffff)) * nz + k3) * NN;
+#pragma unroll
+                for (int v = 0; v < 4; v++) fv[u][v] = *at_b(Fs, ob[v]);
+            }
+#pragma unroll
+            for (int u = 0; u < MB; u++) {
+                if (src[u] < 0) continue;
+                const int fl = src[u] >> 24;
+                const int64_t cb = (int64_t)(t0 + u) * NC;
+                if (fl & 1) {
+                    const T a = coefT[2 * cb] * kc1, g1 = coefT[2 * (cb + 1) + 1];
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const T b = g1 * kc2[v];
+                        W[v].x = fma(a, fv[u][v].x, fma(-b, fv[u][v].y, W[v].x));
+                        W[v].y = fma(a, fv[u][v].y, fma(b, fv[u][v].x, W[v].y));
+                    }
+                }
+                if (fl & 2) {
+                    const T ui = coefT[2 * (cb + DIM) + 1];
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        V1[v].x = fma(-ui, fv[u][v].y, V1[v].x);
+                        V1[v].y = fma(ui, fv[u][v].x, V1[v].y);
+                    }
+                }
+                if (fl & 4) {
+                    const T ur = coefT[2 * (cb + DIM + 1)];
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        V2[v].x = fma(ur, fv[u][v].x, V2[v].x);
+                        V2[v].y = fma(ur, fv[u][v].y, V2[v].y);
+                    }
+                }
+            }
+        }
+        T e3r = T(0), e3i = T(0);
+        if (DIM == 3) {
+            const kc_ptr<T> e3p = as_const<T>((const T*)D.e3) + 2 * (int64_t)r;
+            e3r = e3p[0];
+            e3i = e3p[1] + D.b[2] * kc3;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            T dd = dd0[v];
+            if (DIM == 3) dd += g22 * kd3 - kc3 * (g02 * kc1 + g12 * kc2[v]);
+            W[v].x = fma(dd, fo[v].x, W[v].x);
+            W[v].y = fma(dd, fo[v].y, W[v].y);
+            if (DIM == 3) {
+                if (gyro) {
+                    const T z1 = kc2[v] * D.gyro[1], z2 = kc1 * D.gyro[0];
+                    V1[v].x = fma(z1, Zv[v].y, V1[v].x);
+                    V1[v].y = fma(-z1, Zv[v].x, V1[v].y);
+                    V2[v].x = fma(z2, Zv[v].y, V2[v].x);
+                    V2[v].y = fma(-z2, Zv[v].x, V2[v].y);
+                }
+                W[v].x = fma(e3r, Zv[v].x, fma(-e3i, Zv[v].y, W[v].x));
+                W[v].y = fma(e3r, Zv[v].y, fma(e3i, Zv[v].x, W[v].y));
+            }
+            if (ok[v]) {
+                pF[ps[v]] = fo[v];
+                pV[ps[v]] = V2[v];
+            }
+        }
+        cT<T> f0v[4];
+        if (sc.read_f0) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) f0v[v] = ld_once<T>(at_b(F0 + base, ob[v]));
+        } else {
+#pragma unroll
+            for (int v = 0; v < 4; v++) f0v[v] = fo[v];
+        }
+        __syncthreads();  // (one wave: orders its LDS accesses)
+
+        // ---- everything but T1 V1
+        acc_t ar = MF::zero(), ai = MF::zero(), gr = MF::zero(), gi = MF::zero();
+        {
+            cT<T> s1 = czero<T>(), s2 = czero<T>(), sv = czero<T>();  // axis sums of F along 1 and 2, of V2 along 2
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const cT<T> x1 = pF[orw + 4 * s], x2 = pF[ocl + 4 * s * RS], v = pV[ocl + 4 * s * RS];
+                const T d1 = -k1o * m1[s], d2 = -k2o * m2[s];  // b c (i K)
+                ar = MF::fma(x1.x, d1, ar);
+                ai = MF::fma(x1.y, d1, ai);
+                ar = MF::fma(d2, x2.x, ar);
+                ai = MF::fma(d2, x2.y, ai);
+                ar = MF::fma(m2[s], -v.y, ar);
+                ai = MF::fma(m2[s], v.x, ai);
+                if (gyro) {  // T2 F
+                    gr = MF::fma(m2[s], -x2.y, gr);
+                    gi = MF::fma(m2[s], x2.x, gi);
+                }
+                s1 = cadd<T>(s1, x1);
+                s2 = cadd<T>(s2, x2);
+                sv = cadd<T>(sv, v);
+            }
+            const T f1 = k1o * D.c0[0], f2 = k2o * D.c0[1];
+            ar = MF::fma(-s1.y, f1, ar);
+            ai = MF::fma(s1.x, f1, ai);
+            ar = MF::fma(f2, -s2.y, ar);
+            ai = MF::fma(f2, s2.x, ai);
+            ar = MF::fma(c2, sv.x, ar);
+            ai = MF::fma(c2, sv.y, ai);
+            if (gyro) {
+                gr = MF::fma(c2, s2.x, gr);
+                gi = MF::fma(c2, s2.y, gi);
+                const T g3 = kc3 * D.gyro[2];
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    V1[v].x = fma(g3, gi[v], V1[v].x);
+                    V1[v].y = fma(-g3, gr[v], V1[v].y);
+                }
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (ok[v]) pF[ps[v]] = V1[v];
+        __syncthreads();
+        {
+            cT<T> s1 = czero<T>();
+#pragma unroll
+            for (int s = 0; s < 4; s++) {
+                const cT<T> v = pF[orw + 4 * s];
+                ar = MF::fma(-v.y, m1[s], ar);
+                ai = MF::fma(v.x, m1[s], ai);
+                s1 = cadd<T>(s1, v);
+            }
+            ar = MF::fma(s1.x, c1, ar);
+            ai = MF::fma(s1.y, c1, ai);
+        }
+        const T h = sc.dt * sc.cd;
+        cT<T> y[4];
+#pragma unroll
+        for (int v = 0; v < 4; v++) {  // every load is consumed before the first store
+            const cT<T> q = cmk<T>(ar[v] + W[v].x, ai[v] + W[v].y);
+            y[v] = sc.deriv_only ? cscale<T>(q, sc.dt) : cmk<T>(fma(h, q.x, f0v[v].x), fma(h, q.y, f0v[v].y));
+            asm volatile("" : "+v"(y[v].x), "+v"(y[v].y));
+        }
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            if (ok[v]) st_once<T>(at_b(Fout + base, ob[v]), y[v]);
+        __syncthreads();  // V1 consumed
+        sl += per;
+        rp += dr;
+        k3 += dk;
+        if (rp >= nrc) {
+            rp -= nrc;
+            k3++;
+        }
+    }
+}
+
 // ---------------------------------------------------------- launcher -----
 
-// Sizes, against the kernels that serve the others (B = 8 in 3-D, B = 20 in 2-D):
-// 3-D 1.04-1.58x faster at N = 4 .. 14 and 18 .. 30, 2-D 1.1-1.4x in FP64 and, from
-// N = 18 on, 1.03-1.38x in FP32.  N = 16 fills k_drift_fused_c's tile while its planes
-// of nine points do not fill a K step here (3-D FP64 0.82x, 2-D FP32 0.90x); small
-// 2-D FP32 slabs leave most of a workgroup idle (0.76-1.04x up to N = 14).  In 3-D up to
-// N = 14 a workgroup takes four slabs, so few rows leave workgroups without any: below
-// 1.25 rounds of the resident ones it is the slower (FP64 495 groups 0.99x, 660 1.27x;
-// FP32 858 groups 0.87-0.91x, 1144 1.08x, 1365 0.98-1.14x).
+// N = 18 .. 30 (below, k_drift_tile): 3-D 1.07-1.39x, 2-D 1.2-1.3x in FP64 and 1.03-1.38x in
+// FP32 faster than the kernels that serve the others.
 template <class T> bool drift_fold_ok(const DriftDev<T>& D) {
     if (!D.ramp || !D.odd || !D.smix || D.adj || (sizeof(T) == 4 && D.keep)) return false;
-    if (D.N % 2 || D.N < 4 || D.N > 30 || D.N == 16) return false;
-    if (D.dim == 2) return sizeof(T) == 8 || D.N >= 18;
-    return D.N > 14 || D.nrc * ((D.N + 3) / 4) >= (sizeof(T) == 8 ? 640 : 1280);
+    return D.N % 2 == 0 && D.N >= 18 && D.N <= 30;
+}
+
+template <class T, int DIM>
+static void tile_t(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0, void* Fout,
+                   const StageCoef<T>& sc, hipStream_t st) {
+    const int64_t nslab = D.nrc * (DIM == 3 ? D.N : 1);
+    auto kern = k_drift_tile<T, DIM>;
+    const unsigned grid = persistent_blocks((const void*)kern, nslab, 64, 0);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, st, D, MX, (const cT<T>*)Fin, (const cT<T>*)Z3, (const cT<T>*)F0,
+                       (cT<T>*)Fout, sc, (int)nslab);
+}
+// Every N up to 16: faster at all of them (from one round of the waves on), even where
+// most of the tile is padding (N = 4, B = 20: 1.9x FP32, 2.4x FP64)
+template <class T> bool drift_tile_ok(const DriftDev<T>& D) {
+    if (!D.ramp || !D.smix || D.adj || (sizeof(T) == 4 && D.keep)) return false;
+    return D.N <= 16;
+}
+template <class T>
+void launch_drift_tile(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0,
+                       void* Fout, const StageCoef<T>& sc, hipStream_t st) {
+    HPUP_REQUIRE(drift_tile_ok<T>(D) && !sc.read_acc && !sc.write_acc, HPUP_ERR_UNSUPPORTED,
+                 "one-tile drift: real circulants, structured mixing, N <= 16, no stage sums");
+    if (D.dim == 3) tile_t<T, 3>(D, MX, Fin, Z3, F0, Fout, sc, st);
+    else tile_t<T, 2>(D, MX, Fin, Z3, F0, Fout, sc, st);
 }
 
 template <int KS, int NQ>
@@ -815,23 +1070,21 @@ void launch_drift_fold(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fi
                        void* Fout, const StageCoef<T>& sc, hipStream_t st) {
     HPUP_REQUIRE(drift_fold_ok<T>(D) && !sc.read_acc && !sc.write_acc,
                  HPUP_ERR_UNSUPPORTED, "folded drift: odd real circulants, structured mixing, no stage sums");
-    const int KS = (D.N / 2 + 1 + 3) / 4;
-    if (D.dim == 2) {
-        if constexpr (sizeof(T) == 8) {
-            if (KS == 1) return fold_t<T, 2, 1, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
-            if (KS == 2) return fold_t<T, 2, 2, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
-        }
-        if (KS == 3) return fold_t<T, 2, 3, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
-        return fold_t<T, 2, 4, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
-    }
-    if (KS == 1) return fold_t<T, 3, 1, 4>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 4, 6
-    if (KS == 2) return fold_t<T, 3, 2, 4>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 8 .. 14
+    if (D.dim == 2)
+        return D.N <= 22 ? fold_t<T, 2, 3, 1>(D, MX, Fin, Z3, F0, Fout, sc, st)
+                         : fold_t<T, 2, 4, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
     // slabs per workgroup: as many quarter planes as 256 threads hold
     if (D.N <= 20) return fold_t<T, 3, 3, 2>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 18, 20
     if (D.N == 22) return fold_t<T, 3, 3, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);
     return fold_t<T, 3, 4, 1>(D, MX, Fin, Z3, F0, Fout, sc, st);  // N = 24 .. 30
 }
 
+template bool drift_tile_ok<float>(const DriftDev<float>&);
+template bool drift_tile_ok<double>(const DriftDev<double>&);
+template void launch_drift_tile<float>(const DriftDev<float>&, const MixDev<float>&, const void*, const void*, const void*,
+                                       void*, const StageCoef<float>&, hipStream_t);
+template void launch_drift_tile<double>(const DriftDev<double>&, const MixDev<double>&, const void*, const void*,
+                                        const void*, void*, const StageCoef<double>&, hipStream_t);
 template bool drift_fold_ok<float>(const DriftDev<float>&);
 template bool drift_fold_ok<double>(const DriftDev<double>&);
 template void launch_drift_fold<float>(const DriftDev<float>&, const MixDev<float>&, const void*, const void*, const void*,

@@ -1665,6 +1665,7 @@ void launch_drift_fused(const DriftDev<T>& D, const MixDev<T>& MX, const void* F
         else launch_fused_t<T, GemmF<T, true>, 2, false, true>(D, MX, Fin, Z3, F0, Fout, ACC, sc, nslab, st);
         return;
     }
+    if (!grav && drift_tile_ok<T>(D)) return launch_drift_tile<T>(D, MX, Fin, Z3, F0, Fout, sc, st);
     if (!grav && drift_fold_ok<T>(D)) {
         launch_drift_fold<T>(D, MX, Fin, Z3, F0, Fout, sc, st);
         return;
@@ -1696,6 +1697,7 @@ template <class T> const char* drift_fused_name(const DriftDev<T>& D, bool grav,
         if (D.N > 32 && !grav && drift_fold64_ok(D)) return "k_drift_fold64";
     }
     if (D.N > 32) return "k_drift_fused64";
+    if (!bf16x3 && !grav && drift_tile_ok<T>(D)) return "k_drift_tile";
     if (!bf16x3 && !grav && drift_fold_ok<T>(D)) return "k_drift_fold";
     if (!bf16x3 && !D.adj && D.ramp && D.smix && !grav && D.N <= kCompactMaxN) return "k_drift_fused_c";
     return "k_drift_fused";

@@ -1,11 +1,11 @@
-"""The parity-folded drift kernel (odd real circulants on even and odd parts)
-against the oracle at the edges of its range: the smallest and largest grids of
-each tile depth (6 | 10, 14 | 18, 22 | 24, 30; the reduced model's FP64 kernel for
-34 to 62 points at 34, 38 | 40, 42 | 44, 46 | 48 | 62: one and two quartets a thread), slab groups that do not divide
-the k3 axis (10 = 4 + 4 + 2, 14 = 3 x 4 + 2), grids that keep another kernel
-(16; small FP32 2-D grids; FP32 3-D with 4 points at B = 8), full diffusion matrices, inertias with
-and without gyroscopic terms, several slabs per workgroup, and a coordinate whose
-real circulant is not odd, which the folding must not take.
+"""The parity-folded drift kernels (odd real circulants on even and odd parts) and
+the one-wave kernel of grids up to 16 points, against the oracle at the edges of
+their ranges: the smallest grids, 14 and 16 (a partial and a whole tile), 18, 20, 22 |
+24, 30 (the folded kernel's tile depths and slab groups), the reduced model's FP64
+kernel for 34 to 62 points at 34, 38 | 40, 42 | 44, 46 | 48 | 62 (one and two quartets a
+thread), full diffusion matrices, inertias with and without gyroscopic terms,
+several slabs per workgroup, a coordinate whose real circulant is not odd, which the
+folding must not take, and axes of different circulants.
 
 Tolerances: relative L2 1e-10 (FP64) and 2e-5 (FP32), as the other drift kernels'
 tests: a derivative is sums of at most 6 N + 30 products, so FP32 rounding stays
@@ -31,8 +31,8 @@ def _full(B, dim, N, L, seed):
     return O.fft_forward(B, f, O.wigner_table(B), w, dim, N)
 
 
-CASES = [(2, N, "") for N in (4, 6, 12, 14, 16, 18, 22, 24, 30)] + \
-        [(3, N, "gyro") for N in (4, 6, 8, 10, 14, 16, 18, 20, 22, 24, 30)] + [(3, 10, "iso"), (3, 24, "iso")]
+CASES = [(2, N, "") for N in (2, 4, 6, 12, 14, 16, 18, 22, 24, 30)] + \
+        [(3, N, "gyro") for N in (2, 4, 6, 8, 10, 14, 16, 18, 20, 22, 24, 30)] + [(3, 10, "iso"), (3, 24, "iso")]
 
 
 @pytest.mark.parametrize("dim,N,inertia", CASES)
@@ -42,7 +42,6 @@ def test_derivative_and_step(dim, N, inertia, precision, tol):
     epilogues)."""
     import torch
     print("case fold", dim, N, inertia, precision, flush=True)
-    # 3-D: as few rows as the kernel takes (see drift_fold_ok)
     B, L, dt = (3 if dim == 2 else 2 if N > 14 else 8), 8.0, 0.004
     Jt = JT[inertia] if dim == 3 else None
     G, b = (G3 if dim == 3 else G2), np.array(BT[:dim])
