@@ -765,7 +765,11 @@ __global__ __launch_bounds__(512, 2) void k_drift_fold64(DriftDev<double> D, Mix
 // long (k_drift_fused_c; B = 12, N = 16 FP64 485 -> 186 us, FP32 222 -> 108 us; B = 20, 2-D,
 // N = 14 FP64 142 -> 45 us, FP32 64 -> 26 us; k_drift_fold 1.2-1.7 times k_drift_fused_c's
 // rate at N <= 14).  Bound by the gathered rows' latency: two (FP64) and four waves a SIMD.
-template <class T, int DIM>
+//
+// ADJ: the adjoint operator, on the transposed tables and circulants of k_drift_fused's: the
+// damping joins V1 and V2, and axis 3 comes whole as D.s3.  B = 10, N = 16, FP64, per launch
+// (k_drift_fused before): 299 -> 96 us; the forward operator 281 -> 103 us.
+template <class T, int DIM, bool ADJ>
 __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> D, MixDev<T> MX, const cT<T>* Fin,
                                                                     const cT<T>* __restrict__ Z3, const cT<T>* F0,
                                                                     cT<T>* Fout, StageCoef<T> sc, int nslab) {
@@ -826,12 +830,15 @@ __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> 
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             fo[v] = *at_b(Fin + base, ob[v]);
-            Zv[v] = DIM == 3 ? ld_once<T>(at_b(Z3 + base, ob[v])) : czero<T>();
+            Zv[v] = DIM == 3 && (!ADJ || gyro) ? ld_once<T>(at_b(Z3 + base, ob[v])) : czero<T>();
         }
         const kc_ptr<int32_t> srcT = as_const<int32_t>(MX.src) + (int64_t)r * TS;
         const kc_ptr<T> coefT = as_const<T>((const T*)MX.coef) + 2 * (int64_t)r * TS * NC;
 #pragma unroll
-        for (int v = 0; v < 4; v++) W[v] = V1[v] = V2[v] = czero<T>();
+        for (int v = 0; v < 4; v++) {
+            W[v] = ADJ && DIM == 3 ? ld_once<T>(at_b(D.s3 + base, ob[v])) : czero<T>();
+            V1[v] = V2[v] = czero<T>();
+        }
         for (int t0 = 0; t0 < TS; t0 += MB) {
             int src[MB];
             cT<T> fv[MB][4];
@@ -876,7 +883,7 @@ __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> 
             }
         }
         T e3r = T(0), e3i = T(0);
-        if (DIM == 3) {
+        if (DIM == 3 && !ADJ) {
             const kc_ptr<T> e3p = as_const<T>((const T*)D.e3) + 2 * (int64_t)r;
             e3r = e3p[0];
             e3i = e3p[1] + D.b[2] * kc3;
@@ -887,6 +894,13 @@ __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> 
             if (DIM == 3) dd += g22 * kd3 - kc3 * (g02 * kc1 + g12 * kc2[v]);
             W[v].x = fma(dd, fo[v].x, W[v].x);
             W[v].y = fma(dd, fo[v].y, W[v].y);
+            if (ADJ) {
+                const T a1 = D.b[0] * kc1, a2 = D.b[1] * kc2[v];
+                V1[v].x = fma(a1, fo[v].y, V1[v].x);
+                V1[v].y = fma(-a1, fo[v].x, V1[v].y);
+                V2[v].x = fma(a2, fo[v].y, V2[v].x);
+                V2[v].y = fma(-a2, fo[v].x, V2[v].y);
+            }
             if (DIM == 3) {
                 if (gyro) {
                     const T z1 = kc2[v] * D.gyro[1], z2 = kc1 * D.gyro[0];
@@ -895,8 +909,10 @@ __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> 
                     V2[v].x = fma(z2, Zv[v].y, V2[v].x);
                     V2[v].y = fma(-z2, Zv[v].x, V2[v].y);
                 }
-                W[v].x = fma(e3r, Zv[v].x, fma(-e3i, Zv[v].y, W[v].x));
-                W[v].y = fma(e3r, Zv[v].y, fma(e3i, Zv[v].x, W[v].y));
+                if (!ADJ) {
+                    W[v].x = fma(e3r, Zv[v].x, fma(-e3i, Zv[v].y, W[v].x));
+                    W[v].y = fma(e3r, Zv[v].y, fma(e3i, Zv[v].x, W[v].y));
+                }
             }
             if (ok[v]) {
                 pF[ps[v]] = fo[v];
@@ -921,10 +937,12 @@ __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> 
             for (int s = 0; s < 4; s++) {
                 const cT<T> x1 = pF[orw + 4 * s], x2 = pF[ocl + 4 * s * RS], v = pV[ocl + 4 * s * RS];
                 const T d1 = -k1o * m1[s], d2 = -k2o * m2[s];  // b c (i K)
-                ar = MF::fma(x1.x, d1, ar);
-                ai = MF::fma(x1.y, d1, ai);
-                ar = MF::fma(d2, x2.x, ar);
-                ai = MF::fma(d2, x2.y, ai);
+                if (!ADJ) {
+                    ar = MF::fma(x1.x, d1, ar);
+                    ai = MF::fma(x1.y, d1, ai);
+                    ar = MF::fma(d2, x2.x, ar);
+                    ai = MF::fma(d2, x2.y, ai);
+                }
                 ar = MF::fma(m2[s], -v.y, ar);
                 ai = MF::fma(m2[s], v.x, ai);
                 if (gyro) {  // T2 F
@@ -936,10 +954,12 @@ __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> 
                 sv = cadd<T>(sv, v);
             }
             const T f1 = k1o * D.c0[0], f2 = k2o * D.c0[1];
-            ar = MF::fma(-s1.y, f1, ar);
-            ai = MF::fma(s1.x, f1, ai);
-            ar = MF::fma(f2, -s2.y, ar);
-            ai = MF::fma(f2, s2.x, ai);
+            if (!ADJ) {
+                ar = MF::fma(-s1.y, f1, ar);
+                ai = MF::fma(s1.x, f1, ai);
+                ar = MF::fma(f2, -s2.y, ar);
+                ai = MF::fma(f2, s2.x, ai);
+            }
             ar = MF::fma(c2, sv.x, ar);
             ai = MF::fma(c2, sv.y, ai);
             if (gyro) {
@@ -1001,11 +1021,11 @@ template <class T> bool drift_fold_ok(const DriftDev<T>& D) {
     return D.N % 2 == 0 && D.N >= 18 && D.N <= 30;
 }
 
-template <class T, int DIM>
+template <class T, int DIM, bool ADJ>
 static void tile_t(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0, void* Fout,
                    const StageCoef<T>& sc, hipStream_t st) {
     const int64_t nslab = D.nrc * (DIM == 3 ? D.N : 1);
-    auto kern = k_drift_tile<T, DIM>;
+    auto kern = k_drift_tile<T, DIM, ADJ>;
     const unsigned grid = persistent_blocks((const void*)kern, nslab, 64, 0);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, st, D, MX, (const cT<T>*)Fin, (const cT<T>*)Z3, (const cT<T>*)F0,
                        (cT<T>*)Fout, sc, (int)nslab);
@@ -1013,7 +1033,7 @@ static void tile_t(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, c
 // Every N up to 16: faster at all of them (from one round of the waves on), even where
 // most of the tile is padding (N = 4, B = 20: 1.9x FP32, 2.4x FP64)
 template <class T> bool drift_tile_ok(const DriftDev<T>& D) {
-    if (!D.ramp || !D.smix || D.adj || (sizeof(T) == 4 && D.keep)) return false;
+    if (!D.ramp || !D.smix || D.gpart || (sizeof(T) == 4 && D.keep)) return false;
     return D.N <= 16;
 }
 template <class T>
@@ -1021,8 +1041,10 @@ void launch_drift_tile(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fi
                        void* Fout, const StageCoef<T>& sc, hipStream_t st) {
     HPUP_REQUIRE(drift_tile_ok<T>(D) && !sc.read_acc && !sc.write_acc, HPUP_ERR_UNSUPPORTED,
                  "one-tile drift: real circulants, structured mixing, N <= 16, no stage sums");
-    if (D.dim == 3) tile_t<T, 3>(D, MX, Fin, Z3, F0, Fout, sc, st);
-    else tile_t<T, 2>(D, MX, Fin, Z3, F0, Fout, sc, st);
+    if (D.adj && D.dim == 3) tile_t<T, 3, true>(D, MX, Fin, Z3, F0, Fout, sc, st);
+    else if (D.adj) tile_t<T, 2, true>(D, MX, Fin, Z3, F0, Fout, sc, st);
+    else if (D.dim == 3) tile_t<T, 3, false>(D, MX, Fin, Z3, F0, Fout, sc, st);
+    else tile_t<T, 2, false>(D, MX, Fin, Z3, F0, Fout, sc, st);
 }
 
 template <int KS, int NQ>

@@ -1539,7 +1539,8 @@ template <class K> static unsigned persistent_grid(K kernel, int64_t nslab, int 
 
 // the compact-layout kernel serves omega grids up to kCompactMaxN points per
 // axis (at most two elements per lane: the padding of the MFMA tile is then
-// at least half of it)
+// at least half of it) that k_drift_tile and k_drift_fold leave: FP32 plans
+// that keep their rounding, circulants that are not odd at 18 to 22 points
 #ifndef HPUP_COMPACT_MAXN
 #define HPUP_COMPACT_MAXN 22
 #endif
@@ -1645,6 +1646,7 @@ void launch_drift_fused(const DriftDev<T>& D, const MixDev<T>& MX, const void* F
         if (D.dim == 3) {
             HPUP_REQUIRE(!D.gpart, HPUP_ERR_UNSUPPORTED, "parameter gradients: reduced model (dim 2) only");
             HPUP_REQUIRE(D.s3, HPUP_ERR_ARG, "3-D adjoint stage needs its axis-3 term");
+            if (drift_tile_ok<T>(D)) return launch_drift_tile<T>(D, MX, Fin, Z3, F0, Fout, sc, st);
             if (D.smix) launch_fused_t<T, GemmF<T, true>, 3, false, true, false, true>(D, MX, Fin, Z3, F0, Fout, ACC, sc, nslab, st);
             else launch_fused_t<T, GemmF<T, true>, 3, false, true>(D, MX, Fin, Z3, F0, Fout, ACC, sc, nslab, st);
             return;
@@ -1661,6 +1663,7 @@ void launch_drift_fused(const DriftDev<T>& D, const MixDev<T>& MX, const void* F
                                    (int)nwg, D.gscales, D.gns, D.gout);
             return;
         }
+        if (drift_tile_ok<T>(D)) return launch_drift_tile<T>(D, MX, Fin, Z3, F0, Fout, sc, st);
         if (D.smix) launch_fused_t<T, GemmF<T, true>, 2, false, true, false, true>(D, MX, Fin, Z3, F0, Fout, ACC, sc, nslab, st);
         else launch_fused_t<T, GemmF<T, true>, 2, false, true>(D, MX, Fin, Z3, F0, Fout, ACC, sc, nslab, st);
         return;

@@ -204,7 +204,7 @@ class HybridGradient:
         self.reset = dict(reset)
         self.fwd = Plan(B, dim, N, **kw).keep_rounding()
         self.fwd.set_reset(**self.reset)
-        self.adj = Plan(B, dim, N, operator=1, **kw)
+        self.adj = Plan(B, dim, N, operator=1, **kw).keep_rounding()
         self.ta = TransformAdjoint(self.fwd)
 
     def _grid_before_reset(self, F, Fp=None):

@@ -135,3 +135,33 @@ def test_circulant_not_odd(N):
     e = rel_l2(out, ref)
     print("  rel err %.2e" % e, flush=True)
     assert e < 1e-10
+
+
+@pytest.mark.parametrize("dim,N,inertia", [(2, 2, ""), (2, 10, ""), (2, 14, ""), (2, 16, ""), (3, 2, "gyro"),
+                                           (3, 8, "gyro"), (3, 14, "iso"), (3, 16, "gyro"), (3, 16, "iso")])
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-12), ("fp32", 2e-5)])
+def test_adjoint_one_wave(dim, N, inertia, precision, tol):
+    """<A x, y> = <x, A^H y> for the operator and <P x, y> = <x, P^H y> for two midpoint
+    steps, on grids of the one-wave kernel's adjoint form; relative to |A x| |y|, the
+    bounds of the adjoint operators' own tests."""
+    import torch
+    print("case adjoint one wave", dim, N, inertia, precision, flush=True)
+    kw = {} if dim == 2 else {"Jt": JT[inertia]}
+
+    def plan(op):
+        return hpup.Plan(4, dim, N, 8.0, b=BT if dim == 3 else (BT[0], BT[1], 0.0), G=G3 if dim == 3 else G2, dt=0.004,
+                         method="midpoint", precision=precision, operator=op, **kw)
+
+    A, AH = plan(0), plan(1)
+    g = torch.Generator().manual_seed(10 * N + dim)
+
+    def rand():
+        v = torch.randn(2, A.ncoef, generator=g, dtype=torch.float64)
+        return torch.complex(v[0], v[1]).to(A.cdtype).cuda()
+
+    x, y = rand(), rand()
+    for Ax, AHy in ((A.derivative(x), AH.derivative(y)), (A.step(x.clone(), 2), AH.step(y.clone(), 2))):
+        lhs, rhs = complex(torch.vdot(Ax, y).item()), complex(torch.vdot(x, AHy).item())
+        e = abs(lhs - rhs) / float(Ax.abs().pow(2).sum().sqrt() * y.abs().pow(2).sum().sqrt())
+        print("  %.2e" % e, flush=True)
+        assert e <= tol, (lhs, rhs)
