@@ -764,7 +764,9 @@ __global__ __launch_bounds__(512, 2) void k_drift_fold64(DriftDev<double> D, Mix
 // with four waves to a slab and three barriers the same work took two to three times as
 // long (k_drift_fused_c; B = 12, N = 16 FP64 485 -> 186 us, FP32 222 -> 108 us; B = 20, 2-D,
 // N = 14 FP64 142 -> 45 us, FP32 64 -> 26 us; k_drift_fold 1.2-1.7 times k_drift_fused_c's
-// rate at N <= 14).  Bound by the gathered rows' latency: two (FP64) and four waves a SIMD.
+// rate at N <= 14).  B = 12, N = 16, FP64: its streams take 120 of the 186 us at a copy's rate,
+// the rest is gathered rows and issue at two waves a SIMD (FP32: four).  Two source rows in
+// flight; three measured the same to 4 % slower, six 10-20 % slower in 3-D.
 //
 // ADJ: the adjoint operator, on the transposed tables and circulants of k_drift_fused's: the
 // damping joins V1 and V2, and axis 3 comes whole as D.s3.  B = 10, N = 16, FP64, per launch
