@@ -659,6 +659,13 @@ template <class T> struct PlanT : PlanBase {
             axpy_stage(prev, F, c[ns - 1], Fnext, st);
         }
     }
+    // The reverse stages' partial sums: room for the four stages of a step from
+    // the first call on, whichever it is, so that the buffer never moves (a
+    // captured stage holds its address)
+    double* grad_partials() {
+        ensure(gpart, sizeof(double) * kGradMaxWG * 5 * 4);
+        return gpart.as<double>();
+    }
     // The whole reverse step on an adjoint plan from the forward stage values
     // y_0 = F, y_1..y_{s-1} = ys: ybar_s = lam, ybar_{j-1} = c_j dt A^H ybar_j,
     // Fbar = sum_j ybar_j, gout += the parameter terms of every stage
@@ -671,14 +678,14 @@ template <class T> struct PlanT : PlanBase {
         ensure(Yb, cbytes());
         // every stage leaves its partial sums in a part of gpart of its own; the
         // last one's launch adds them all to gout, in the stages' order
-        ensure(gpart, sizeof(double) * kGradMaxWG * 5 * 4);
+        double* part = grad_partials();
         GradScales sc{};
         const void* ybar = lam;
         for (int j = ns - 1, q = 0; j >= 0; j--, q++) {
             const void* y = j == 0 ? F : ys[j - 1];
             void* out = (ybar == Ya.p) ? Yb.p : Ya.p;
             sc.s[q] = c[j];
-            adjoint_stage_at(ybar, y, c[j], out, Fbar, q == 0 ? 1 : 0, gout, gpart.as<double>(), q, sc, j == 0 ? ns : 0, st);
+            adjoint_stage_at(ybar, y, c[j], out, Fbar, q == 0 ? 1 : 0, gout, part, q, sc, j == 0 ? ns : 0, st);
             ybar = out;
         }
     }
@@ -696,8 +703,7 @@ template <class T> struct PlanT : PlanBase {
             HPUP_HIP(hipGetDevice(&dev));
             part = grad_scratch(dev);
         } else {
-            ensure(gpart, sizeof(double) * kGradMaxWG * 5);
-            part = gpart.as<double>();
+            part = grad_partials();
         }
         adjoint_stage_at(ybar, y, scale, out, fbar, fbar_init, gout, part, 0, GradScales{{scale, 0, 0, 0}}, 1, st);
     }
