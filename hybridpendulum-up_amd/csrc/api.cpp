@@ -171,7 +171,7 @@ template <class T> struct XformTables {
 };
 
 template <class T> struct DriftTables {
-    DevBuf cg_src, cg_coef, u_src, u_coef, e3, kap, kc, kd, M3, mix_src, mix_coef, mix_order;
+    DevBuf cg_src, cg_coef, u_src, u_coef, e3, kap, kc, kd, M3, op, mix_src, mix_coef, mix_order;
     DriftDev<T> view{};
     MixDev<T> mix{};
     bool smix = false;
@@ -302,6 +302,12 @@ template <class T> struct DriftTables {
         v.same12 = s.same12 ? 1 : 0;
         v.smix = smix ? 1 : 0;
         v.adj = s.adj ? 1 : 0;
+        // the sizes of k_drift_fold and (FP64) k_drift_fold64
+        if (smix && s.odd && !s.adj && ((N >= 18 && N <= 30) || (sizeof(T) == 8 && N >= 34 && N <= 62))) {
+            const std::vector<long double> t = operator_tables(s);
+            op = upload(std::vector<T>(t.begin(), t.end()));
+            v.op = op.as<T>();
+        }
         v.has_gyro = s.has_gyro ? 1 : 0;
         v.grav[0] = v.grav[1] = v.grav[2] = nullptr;
         v.s3 = nullptr;

@@ -48,6 +48,8 @@ template <class T> struct DriftDev {
     int odd;     // ... and the real circulants are odd
     int same12;  // ... and those of axes 1 and 2 are equal
     int keep;    // FP32: not the folded kernel (see XformDev::keep)
+    // matrices of the folded kernels (OpTab), null where neither serves the plan
+    const T* op;
     T c0[3];
     // structured mixing coefficients: -i CG_1 real, -i CG_2 imaginary,
     // CG_3 zero, u_1 imaginary, u_2 real (the pendulum models)
@@ -107,8 +109,8 @@ template <class T>
 void launch_drift_fold(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0,
                        void* Fout, const StageCoef<T>& sc, hipStream_t st);
 // one wave and one matrix tile per slab, N <= 16: taken where drift_tile_ok (real
-// circulants, structured mixing, forward operator; sizes at its definition), with no
-// grid gravity and no stage sums
+// circulants, structured mixing, forward and adjoint operator; sizes at its
+// definition), with no grid gravity, no stage sums and no gradient sums
 template <class T> bool drift_tile_ok(const DriftDev<T>& D);
 template <class T>
 void launch_drift_tile(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0,

@@ -24,7 +24,7 @@
 // LDS address is a register plus an immediate, and an axis sum is folded over a
 // lane's own points before one matrix instruction adds it: the unfolded kernels
 // spend most of their vector instructions on table reads, axis sums, lane
-// permutes and addresses.
+// permutes and addresses.  The matrices come from the host (OpTab), rounded once.
 //
 // What bounds it: no single unit (B = 15, N = 30, FP32: matrix pipe 24 %, vector
 // units 32 %, tag lookups 60 %, HBM 75 % of a copy's rate).  The six gathered
@@ -106,28 +106,17 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
     const int p1 = w & 1, p2 = w >> 1;
     T m1[KS], m2[KS], d1[KS], d2[KS], rr1, rr2;
     {
-        auto mats = [&](const cT<T>* kap, int p, T c0, T b, T* m, T* d, T& rr) {
-            auto K = [&](int j) { return kap[j < 0 ? j + N : j < N ? j : j - N].y; };  // -N < j < 2 N
-            const T kco = lr <= H ? D.kc[lr] : T(0);
+        constexpr OpTab ot(30);
 #pragma unroll
-            for (int s = 0; s < KS; s++) {
-                const int a = 4 * s + lq;
-                const bool in = a <= H, self = a == 0 || a == H, oself = lr == 0 || lr == H;
-                T oe = T(0), eo = T(0);  // even -> odd, odd -> even
-                if (in && lr <= H) {
-                    const T km = K(lr - a), kp = K(lr + a);
-                    oe = oself ? T(0) : self ? km : km + kp;
-                    eo = self ? T(0) : km - kp;
-                }
-                oe *= T(0.25);
-                eo *= T(0.25);
-                m[s] = p ? oe : eo;               // K into this plane's parity
-                d[s] = -b * kco * (p ? eo : oe);  // b c (i K): K to the other parity and kc back
-            }
-            rr = lr <= H ? T(0.5) * c0 * (p ? b * kco : T(1)) : T(0);
-        };
-        mats(D.kap, p1, D.c0[0], D.b[0], m1, d1, rr1);
-        mats(D.kap + N, p2, D.c0[1], D.b[1], m2, d2, rr2);
+        for (int s = 0; s < KS; s++) {
+            const int i = lr * ot.S + 4 * s + lq;
+            m1[s] = D.op[ot.mat(0, 0, p1) + i];  // K into this plane's parity
+            m2[s] = D.op[ot.mat(1, 0, p2) + i];
+            d1[s] = D.op[ot.mat(0, 1, p1) + i];  // b c (i K): K to the other parity and kc back
+            d2[s] = D.op[ot.mat(1, 1, p2) + i];
+        }
+        rr1 = D.op[ot.vec(0, p1) + lr];
+        rr2 = D.op[ot.vec(1, p2) + lr];
     }
 
     // weights of the axis sums: a half for a = 0 (step 0) and a = H (the last
@@ -466,27 +455,23 @@ __global__ __launch_bounds__(512, 2) void k_drift_fold64(DriftDev<double> D, Mix
     const int pl = w & 3, rt = w >> 2, p1 = pl & 1, p2 = pl >> 1;
     for (int i = tid; i < 2 * OV; i += 512) pA[i] = czero<T>();
 
-    // ---- the axes' matrices (the same for both: D.same12) in LDS, [odd -> even,
-    // even -> odd][in][out]
+    // ---- the axes' matrices (the same for both: D.same12) in LDS, [parity][in][out]
     T* sM = reinterpret_cast<T*>(pA + 2 * OV);
-    auto entry = [&](const cT<T>* kap, int o, int a, T& oe, T& eo) {
-        const bool in = a <= H && o <= H, self = a == 0 || a == H;
-        auto K = [&](int j) { return kap[j < 0 ? j + N : j < N ? j : j - N].y; };  // -N < j < 2 N
-        const T km = in ? K(o - a) : T(0), kp = in ? K(o + a) : T(0);
-        oe = !in || o == 0 || o == H ? T(0) : T(0.25) * (self ? km : km + kp);  // even -> odd
-        eo = !in || self ? T(0) : T(0.25) * (km - kp);                        // odd -> even
-    };
-    for (int i = tid; i < HP * HP; i += 512) entry(D.kap, i % HP, i / HP, sM[HP * HP + i], sM[i]);
+    constexpr OpTab ot(62);
+    for (int i = tid; i < 2 * HP * HP; i += 512) {
+        const int par = i / (HP * HP), e = i - par * HP * HP, a = e / HP, o = e - a * HP;
+        sM[i] = D.op[ot.mat(0, 0, par) + o * ot.S + a];
+    }
     T rr1[2], k1o[2], rr2, k2o;  // k_o: -b kc of the outputs
     {
         const int o2 = 16 * rt + lr;
-        k2o = o2 <= H ? -D.b[1] * D.kc[o2] : T(0);
-        rr2 = o2 <= H ? T(0.5) * D.c0[1] * (p2 ? -k2o : T(1)) : T(0);
+        k2o = D.op[ot.vec(1, 2) + o2];
+        rr2 = D.op[ot.vec(1, p2) + o2];
 #pragma unroll
         for (int c = 0; c < 2; c++) {
             const int o1 = 16 * c + lr;
-            k1o[c] = o1 <= H ? -D.b[0] * D.kc[o1] : T(0);
-            rr1[c] = o1 <= H ? T(0.5) * D.c0[0] * (p1 ? -k1o[c] : T(1)) : T(0);
+            k1o[c] = D.op[ot.vec(0, 2) + o1];
+            rr1[c] = D.op[ot.vec(0, p1) + o1];
         }
     }
     const T wa = lq == 0 || lq == H ? T(0.5) : T(1), wb = lq == (H & 3) ? T(0.5) : T(1);
@@ -770,7 +755,7 @@ __global__ __launch_bounds__(512, 2) void k_drift_fold64(DriftDev<double> D, Mix
 //
 // ADJ: the adjoint operator, on the transposed tables and circulants of k_drift_fused's: the
 // damping joins V1 and V2, and axis 3 comes whole as D.s3.  B = 10, N = 16, FP64, per launch
-// (k_drift_fused before): 299 -> 96 us; the forward operator 281 -> 103 us.
+// (k_drift_fused before): 299 -> 96 us; the forward operator 281 -> 97 us.
 template <class T, int DIM, bool ADJ>
 __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> D, MixDev<T> MX, const cT<T>* Fin,
                                                                     const cT<T>* __restrict__ Z3, const cT<T>* F0,
@@ -783,9 +768,8 @@ __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> 
     const int lane = threadIdx.x, lr = lane & 15, lq = lane >> 4;
     for (int i = lane; i < 16 * RS; i += 64) pF[i] = pV[i] = czero<T>();
 
-    // matrices, entry [out lr][in 4 s + lq]
+    // matrices K_1, K_2, entry [out lr][in 4 s + lq]
     T m1[4], m2[4];
-    const T k1o = lr < N ? D.b[0] * D.kc[lr] : T(0), k2o = lr < N ? D.b[1] * D.kc[lr] : T(0);  // b kc of the outputs
     const T c1 = lr < N ? D.c0[0] : T(0), c2 = lr < N ? D.c0[1] : T(0);
 #pragma unroll
     for (int s = 0; s < 4; s++) {
@@ -931,47 +915,57 @@ __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> 
         }
         __syncthreads();  // (one wave: orders its LDS accesses)
 
-        // ---- everything but T1 V1
-        acc_t ar = MF::zero(), ai = MF::zero(), gr = MF::zero(), gi = MF::zero();
+        // ---- everything but T1 V1: T2 V2, and T_p F for the damping b_p c_p T_p F, c_p = i kc
+        // (!ADJ), and the gyroscopic term.  Each has accumulators of its own: its terms
+        // alternate in sign, and in one chain every addition would round at the size
+        // of all their partial sums; and kc scales the sum, not the matrix, whose
+        // entries stay rounded once.  Error of the FP32 derivative, 2-D, N = 8 / 14 / 16: 2.3e-7
+        // / 2.7e-7 / 2.8e-7 in one chain, now 2.1e-7 / 2.3e-7 / 2.3e-7 (k_drift_fused_c 1.9e-7 /
+        // 2.1e-7 / 2.3e-7); T2 F serves the gyroscopic term too (B = 10, N = 16, FP64: 100 -> 97
+        // us).  The axis sums added over lanes by shuffles, not by the matrix instruction:
+        // 1.9e-7 / 2.2e-7 / 2.2e-7, but FP32 8-18 % slower.
         {
+            acc_t pr = MF::zero(), pi = MF::zero(), qr = MF::zero(), qi = MF::zero(), ar = MF::zero(), ai = MF::zero();
             cT<T> s1 = czero<T>(), s2 = czero<T>(), sv = czero<T>();  // axis sums of F along 1 and 2, of V2 along 2
 #pragma unroll
             for (int s = 0; s < 4; s++) {
                 const cT<T> x1 = pF[orw + 4 * s], x2 = pF[ocl + 4 * s * RS], v = pV[ocl + 4 * s * RS];
-                const T d1 = -k1o * m1[s], d2 = -k2o * m2[s];  // b c (i K)
                 if (!ADJ) {
-                    ar = MF::fma(x1.x, d1, ar);
-                    ai = MF::fma(x1.y, d1, ai);
-                    ar = MF::fma(d2, x2.x, ar);
-                    ai = MF::fma(d2, x2.y, ai);
+                    pr = MF::fma(-x1.y, m1[s], pr);
+                    pi = MF::fma(x1.x, m1[s], pi);
+                }
+                if (!ADJ || gyro) {
+                    qr = MF::fma(m2[s], -x2.y, qr);
+                    qi = MF::fma(m2[s], x2.x, qi);
                 }
                 ar = MF::fma(m2[s], -v.y, ar);
                 ai = MF::fma(m2[s], v.x, ai);
-                if (gyro) {  // T2 F
-                    gr = MF::fma(m2[s], -x2.y, gr);
-                    gi = MF::fma(m2[s], x2.x, gi);
-                }
                 s1 = cadd<T>(s1, x1);
                 s2 = cadd<T>(s2, x2);
                 sv = cadd<T>(sv, v);
             }
-            const T f1 = k1o * D.c0[0], f2 = k2o * D.c0[1];
             if (!ADJ) {
-                ar = MF::fma(-s1.y, f1, ar);
-                ai = MF::fma(s1.x, f1, ai);
-                ar = MF::fma(f2, -s2.y, ar);
-                ai = MF::fma(f2, s2.x, ai);
+                pr = MF::fma(s1.x, c1, pr);
+                pi = MF::fma(s1.y, c1, pi);
             }
+            qr = MF::fma(c2, s2.x, qr);
+            qi = MF::fma(c2, s2.y, qi);
             ar = MF::fma(c2, sv.x, ar);
             ai = MF::fma(c2, sv.y, ai);
-            if (gyro) {
-                gr = MF::fma(c2, s2.x, gr);
-                gi = MF::fma(c2, s2.y, gi);
-                const T g3 = kc3 * D.gyro[2];
+            const T k1 = D.b[0] * kc1, g3 = gyro ? kc3 * D.gyro[2] : T(0);
 #pragma unroll
-                for (int v = 0; v < 4; v++) {
-                    V1[v].x = fma(g3, gi[v], V1[v].x);
-                    V1[v].y = fma(-g3, gr[v], V1[v].y);
+            for (int v = 0; v < 4; v++) {
+                T wr = ar[v], wi = ai[v];
+                if (!ADJ) {
+                    const T k2 = D.b[1] * kc2[v];
+                    wr = fma(-k1, pi[v], fma(-k2, qi[v], wr));
+                    wi = fma(k1, pr[v], fma(k2, qr[v], wi));
+                }
+                W[v].x += wr;
+                W[v].y += wi;
+                if (gyro) {
+                    V1[v].x = fma(g3, qi[v], V1[v].x);
+                    V1[v].y = fma(-g3, qr[v], V1[v].y);
                 }
             }
         }
@@ -980,6 +974,7 @@ __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> 
         for (int v = 0; v < 4; v++)
             if (ok[v]) pF[ps[v]] = V1[v];
         __syncthreads();
+        acc_t ar = MF::zero(), ai = MF::zero();
         {
             cT<T> s1 = czero<T>();
 #pragma unroll
@@ -1019,7 +1014,7 @@ __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> 
 // N = 18 .. 30 (below, k_drift_tile): 3-D 1.07-1.39x, 2-D 1.2-1.3x in FP64 and 1.03-1.38x in
 // FP32 faster than the kernels that serve the others.
 template <class T> bool drift_fold_ok(const DriftDev<T>& D) {
-    if (!D.ramp || !D.odd || !D.smix || D.adj || (sizeof(T) == 4 && D.keep)) return false;
+    if (!D.ramp || !D.odd || !D.smix || !D.op || D.adj || (sizeof(T) == 4 && D.keep)) return false;
     return D.N % 2 == 0 && D.N >= 18 && D.N <= 30;
 }
 
@@ -1061,7 +1056,7 @@ static void fold64_t(const DriftDev<double>& D, const MixDev<double>& MX, const 
 }
 
 bool drift_fold64_ok(const DriftDev<double>& D) {
-    return D.ramp && D.odd && D.same12 && D.smix && !D.adj && D.dim == 2 && D.N % 2 == 0 && D.N >= 34 && D.N <= 62;
+    return D.ramp && D.odd && D.same12 && D.smix && D.op && !D.adj && D.dim == 2 && D.N % 2 == 0 && D.N >= 34 && D.N <= 62;
 }
 void launch_drift_fold64(const DriftDev<double>& D, const MixDev<double>& MX, const void* Fin, const void* F0, void* Fout,
                          const StageCoef<double>& sc, hipStream_t st) {

@@ -202,6 +202,27 @@ DriftSpec build_drift_spec_from_arrays(int B, int dim, int N, double L, const do
 // Builds the same operator from physical parameters (the drivers' recipe).
 DriftSpec build_drift_spec_from_model(const hpup_model& m);
 
+// Matrices of T_p = c0 + i K_p and of the damping b_p c_p T_p, c_p = i kc, of axes 1 and 2
+// as the folded drift kernels (18 to 62 points, odd K_p) multiply by them on the parts x'
+// of drift_fold.hip, formed in extended precision and rounded once to the plan's type.
+// (Formed on the device from rounded entries, K(k - a) +- K(k + a) and b kc times them carry
+// two to four roundings each: a fixed error of the operator, which grows with the
+// steps.  FP32, entries of the damping operators, N = 18 to 30: 4.5e-8 to 6.3e-8, now 3.0e-8
+// to 3.7e-8, unfolded 3.6e-8 to 5.5e-8.)
+//   mat(axis, 0, par): K into the part of parity par (0 even) from the other one;
+//   mat(axis, 1, par): -b kc K into it from the same one;  a quarter of the sums there,
+//   [out][in], zero beyond N / 2.
+//   vec(axis, 0) = c0 / 2 (into the even part), vec(axis, 1) = b kc c0 / 2 (into the odd
+//   one), vec(axis, 2) = -b kc.
+struct OpTab {
+    int S;  // row length
+    __host__ __device__ constexpr OpTab(int N) : S(N <= 30 ? 16 : 32) {}
+    __host__ __device__ constexpr int mat(int axis, int kind, int par) const { return ((axis * 2 + kind) * 2 + par) * S * S; }
+    __host__ __device__ constexpr int vec(int axis, int i) const { return 8 * S * S + (axis * 3 + i) * S; }
+    __host__ __device__ constexpr int size() const { return vec(2, 0); }
+};
+std::vector<long double> operator_tables(const DriftSpec& s);
+
 // Clebsch-Gordan cell by the reference's tridiagonal null-vector recipe (clebsch_gordan.m).
 void host_clebsch_gordan(int l1, int l2, std::vector<double>& CG);
 

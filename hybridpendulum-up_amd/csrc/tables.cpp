@@ -173,6 +173,37 @@ DriftSpec parameter_spec(const DriftSpec& s, int term) {
     return a;
 }
 
+std::vector<long double> operator_tables(const DriftSpec& s) {
+    using ld = long double;
+    const OpTab ot(s.N);
+    std::vector<ld> t(ot.size(), 0.0L);
+    const int N = s.N, H = N / 2, S = ot.S;
+    for (int p = 0; p < 2; p++) {
+        const ld b = s.b[p], c0 = s.c0[p];
+        auto K = [&](int d) { return (ld)s.kappa[2 * (N * p + ((d % N) + N) % N) + 1]; };
+        auto kc = [&](int k) {
+            return 2.0L * 3.14159265358979323846264338327950288L * (k < H ? k : k == H ? 0 : k - N) / (ld)s.L;
+        };
+        // K odd: its odd part (what is left of rounding in the even one is dropped)
+        auto Ko = [&](int d) { return (K(d) - K(-d)) / 2; };
+        for (int o = 0; o <= H; o++) {
+            for (int a = 0; a <= H; a++) {
+                const bool self = a == 0 || a == H;  // a point that is its own mirror
+                const ld eo = self ? 0.0L : (Ko(o - a) - Ko(o + a)) / 4;  // odd -> even
+                const ld oe = o == 0 || o == H ? 0.0L : (self ? Ko(o - a) : Ko(o - a) + Ko(o + a)) / 4;
+                t[ot.mat(p, 0, 0) + o * S + a] = eo;
+                t[ot.mat(p, 0, 1) + o * S + a] = oe;
+                t[ot.mat(p, 1, 0) + o * S + a] = -b * kc(o) * oe;
+                t[ot.mat(p, 1, 1) + o * S + a] = -b * kc(o) * eo;
+            }
+            t[ot.vec(p, 0) + o] = c0 / 2;
+            t[ot.vec(p, 1) + o] = b * kc(o) * c0 / 2;
+            t[ot.vec(p, 2) + o] = -b * kc(o);
+        }
+    }
+    return t;
+}
+
 void host_clebsch_gordan(int l1, int l2, std::vector<double>& CG) {
     const int dim = (2 * l1 + 1) * (2 * l2 + 1);
     CG.assign((size_t)dim * dim, 0.0);
