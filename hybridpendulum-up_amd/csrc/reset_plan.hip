@@ -405,8 +405,9 @@ __global__ __launch_bounds__(256) void k_sum_partials(const double* __restrict__
 // takes sixty; the contact sign is that of sigma (s . y).  Both forms agree
 // to rounding, so the masks differ at most where s . y (dim 2: or the distance
 // to an edge of the box) is at rounding level: those points, told by a margin
-// of 1e-12 N grid units, take the masks of the chain itself (exact_masks), in
-// its order of operations.  Measured on the rows kernel: B = 30, 20^3, FP32 4.81
+// of 1e-12 N grid units for s . y and of (1 + eps)/eps times that for the pulled-back
+// position, take the masks of the chain itself (exact_masks), in its order of
+// operations.  (Both forms' positions are off by about (1 + eps)/eps N 2^-53.)  Measured on the rows kernel: B = 30, 20^3, FP32 4.81
 // -> 3.64 ms, B = 30, 60^2, FP64 2.02 -> 1.50 ms.  Of the 3.64 ms, staging takes 1.4,
 // stores 1.3 and the arithmetic the rest, in turn (one workgroup per CU holds a
 // group); loading the next group into registers meanwhile made it 5.1 ms (spills).
@@ -443,7 +444,7 @@ template <int DIM>
 __device__ __forceinline__ void pull_at(const RowFast& r, const double* sg, int stride, int k, const ResetConsts& c,
                                         int i0, int i1, int i2, Pull<DIM>& p) {
     const int N = c.N, h = N / 2;
-    const double tol = 1e-12 * N;
+    const double tol = 1e-12 * N, tolu = tol * c.kfac;
     const int id[3] = {i0, i1, i2};
     double dot = r.s[0] * (double)(i0 - h) + r.s[1] * (double)(i1 - h);
     if (DIM == 3) dot += r.s[2] * (double)(i2 - h);
@@ -456,9 +457,9 @@ __device__ __forceinline__ void pull_at(const RowFast& r, const double* sg, int 
 #pragma unroll
     for (int a = 0; a < DIM; a++) {
         const double u = (double)id[a] - q * r.s[a];
-        if (DIM == 2) near = near || fabs(u - lo) < tol || fabs(u - hi) < tol;
+        if (DIM == 2) near = near || fabs(u - lo) < tolu || fabs(u - hi) < tolu;
         p.in_on = p.in_on && u >= lo && u <= hi;
-        p.face = p.face || fabs(u - rint(u)) < tol;
+        p.face = p.face || fabs(u - rint(u)) < tolu;
         // beyond the support only masked points remain
         const double cf = fmin(fmax(floor(u), DIM == 2 ? 0.0 : -1.0), DIM == 2 ? (double)(N - 2) : (double)(N - 1));
         p.c[a] = (int)cf;
