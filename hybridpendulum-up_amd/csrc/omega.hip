@@ -63,8 +63,13 @@ template <class T> __device__ __forceinline__ cT<T> sconj(cT<T> z, bool neg) {
 // Measured per launch: B = 30, 60^2, FP64 6.1 -> 1.02 ms forward, 0.79 ms inverse
 // (direct sums on all rows before; half of the rows now); on half of the rows
 // against Toeplitz products: B = 15, 30^3, FP64 0.80 -> 0.65 ms, FP32 0.32 ->
-// 0.23 ms; B = 30, 20^3, FP32 1.08 -> 0.64 ms.  N = 32 gains least: FP64 76 -> 72 us,
-// FP32 37 -> 39 us (B = 20, 32^2).
+// 0.23 ms; B = 30, 20^3, FP32 1.08 -> 0.64 ms.
+//
+// N = 32, whose 17 points do not fill the tiles, gains no time in FP32 against the Toeplitz
+// products, and keeps this form for its error, half of theirs: B = 20, 2-D, forward /
+// inverse 37 / 34 -> 38 / 36 us, B = 30 121 / 121 -> 122 / 114, B = 8, 3-D 58 / 57 -> 64 / 64; relative
+// error 2.7e-7 / 3.0e-7 -> 1.3e-7 / 2.0e-7 (B = 12, the whole transform).  FP64, B = 20: 75 / 76 ->
+// 75 / 62 us.
 //
 // Slab sl is row sl / nz at k3 = sl % nz (rows from the half list unless hr is
 // null).  In place when in == out: a block's slabs are read whole before any is
@@ -72,15 +77,20 @@ template <class T> __device__ __forceinline__ cT<T> sconj(cT<T> z, bool neg) {
 constexpr int kSlabMaxXC = 16;
 
 // Elements a thread loads before its first use: a block's slabs in one batch
-// (two in FP64 when the mirror slabs are loaded too), one memory round trip
+// (two in FP64 when the mirror slabs are loaded too), one memory round trip.  At the
+// largest N of two classes a second batch holds the rest: N = 22 needs 10 and N = 62 16;
+// with these they are up to 9 % faster and the other sizes of their classes (16 to 20,
+// 56 to 60) 1-4 % slower, by the loads they repeat.
 constexpr int slab_batch(int KS, bool NYQ) {
     return NYQ ? (KS == 5 ? 12 : 16) : KS == 1 ? 3 : KS == 2 ? 7 : KS == 3 ? 8 : KS == 4 ? 15 : KS == 5 ? 6 : KS == 6 ? 9 : KS == 7 ? 12 : 15;
 }
 
 // (FP32 is compiled for 5 waves per SIMD: without the bound the compiler spreads
-// over 100 to 140 registers, 3 or 4 waves, and the slabs wait for their loads)
+// over 100 to 140 registers, 3 or 4 waves, and the slabs wait for their loads.  N = 32,
+// B = 20, 2-D, without the mirror slabs' loads: 38 us at 4 waves, 40 at 5; with them 38
+// and 36)
 template <class T, int KS, int TPW, bool SYM, bool NYQ>
-__global__ __launch_bounds__(256, TPW > 1 ? 1 : sizeof(T) == 8 ? 3 : NYQ ? 4 : 5) void k_slab_dft(const cT<T>* in, cT<T>* out, const T* __restrict__ tab, int N,
+__global__ __launch_bounds__(256, TPW > 1 ? 1 : sizeof(T) == 8 ? 3 : NYQ && !SYM ? 4 : 5) void k_slab_dft(const cT<T>* in, cT<T>* out, const T* __restrict__ tab, int N,
                                                   T scale, T sgn, int nslab, int nz, const int32_t* __restrict__ hr,
                                                   int mirror, int XC) {
     using MF = Mfma<T>;
