@@ -1837,7 +1837,7 @@ void launch_inv_ag(const XformDev<T>& X, const void* G, void* f, hipStream_t st)
         default: return X.B < 32 ? inv_ag_mfma<T, 2, 8>(X, G, f, st) : inv_ag_mfma<T, 3, 8>(X, G, f, st);
         }
     }
-    // gamma chunks of 16 for B > 32
+    // gamma chunks of 16 for B > 32, and for B = 17 .. 32 where the plan keeps its rounding
     constexpr int GC = 16;
     const int ngc = (n2 + GC - 1) / GC;
     const size_t per_x = sizeof(cT<T>) * ((size_t)M * n2);

@@ -546,8 +546,9 @@ class Plan:
         return out
 
     def keep_rounding(self):
-        """FP32 plans: the order of sums that a gradient sweep's 64-bit gradients
-        stand on, instead of the faster kernels."""
+        """FP32 plans: from the next call on, the order of sums that a gradient
+        sweep's 64-bit gradients stand on, instead of the faster kernels (the
+        reduced model's FP32 plans do so by themselves from set_reset on)."""
         _check(lib().hpup_plan_keep_rounding(self._h))
         return self
 

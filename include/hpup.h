@@ -292,11 +292,14 @@ int hpup_plan_axpy_stage(hpup_plan* plan, const void* in, const void* F0, double
 int hpup_plan_adjoint_stage(hpup_plan* plan, const void* ybar, const void* y, double scale, void* ybar_out,
                             void* fbar, int fbar_init, double* grad, void* stream);
 
-/* FP32 plans: keeps the drift kernels and DFTs that a gradient sweep's 64-bit
- * parameter gradients stand on, in the order of their sums, instead of the faster
- * ones, which would move such figures by about 1e-7 (no counterpart in the
- * reference; callers: gradient sweeps, before the plan's first use).  Plans of the
- * reduced model do so by themselves once they have a reset.  FP64 plans: no effect. */
+/* FP32 plans: from the next call on, the drift kernels and DFTs that a gradient
+ * sweep's 64-bit parameter gradients stand on, in the order of their sums, instead
+ * of the faster ones, which would move such figures by about 1e-7 (no counterpart
+ * in the reference; callers: gradient sweeps).  May be called at any time and any
+ * number of times; results before and after differ in FP32 rounding, and it cannot
+ * be undone.  FP32 plans of the reduced model do the same by themselves from
+ * hpup_plan_set_reset on, whose densities get_stat reads in 64 bits.  FP64 plans
+ * (and the drift of HPUP_BF16X3 plans): no effect. */
 int hpup_plan_keep_rounding(hpup_plan* plan);
 /* The stage values of one step of a forward model plan (no counterpart in the
  * reference; callers: gradient sweeps that keep them for the reverse pass).
@@ -402,7 +405,8 @@ typedef struct {
  * getIndRule.cu:50-90, propagate.cu:123-229): the chain
  * getLambda_mex(..., true) -> getOmega_mex(..., 'old') -> getIndRule_mex ->
  * pendulum_reduced_discrete_propagate(false, ...) in one device pass.  dim 3
- * extends it to a full body angular velocity (trilinear interpolation). */
+ * extends it to a full body angular velocity (trilinear interpolation).
+ * FP32, dim 2: the plan keeps its rounding from here on (hpup_plan_keep_rounding). */
 int hpup_plan_set_reset(hpup_plan* plan, const hpup_reset_params* params);
 /* The region's rotation indices (ascending, 0-based as lambda_indR): writes
  * up to max_rows of them into indR (nullable) and returns their number, or a
