@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
     int rnext = sl < hi ? ord[rp] : 0;
     cT<T> fo[4], Zv[4];
     auto load_own = [&](int row, int k3g) {
-        const int64_t bn = ((int64_t)row * nz + (DIM == 3 ? min(k3g * XS, N - XS) : 0)) * NN;
+        const int64_t bn = ((int64_t)row * nz + k3g * XS) * NN;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             fo[j] = *at_b(Fin + bn, ob[j]);
@@ -184,10 +184,7 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
         // workgroups drift apart in phase instead of queueing for one unit: 2-3 %
         __builtin_amdgcn_s_setprio(0);
         const int r = rnext;
-        // the group's first k3; a last group that would pass N starts earlier and
-        // leaves the slabs it shares with the previous group to that one
-        const int k30 = DIM == 3 ? min(kg * XS, N - XS) : 0;
-        const bool own = act && k30 + xs >= kg * XS;
+        const int k30 = kg * XS;  // the group's first k3
         const int64_t base = ((int64_t)r * nz + k30) * NN;
         int rn = rp + dr, kn = kg + dk;
         if (rn >= nrc) {
@@ -399,7 +396,7 @@ __global__ __launch_bounds__(256, fold_waves<T>()) void k_drift_fold(DriftDev<T>
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) qv[j] = cadd<T>(y[j], W[j]);
-        const bool st[4] = {own, own && !self1, own && !self2, own && !self1 && !self2};
+        const bool st[4] = {act, act && !self1, act && !self2, act && !self1 && !self2};
         if (sc.deriv_only) {
 #pragma unroll
             for (int j = 0; j < 4; j++)
@@ -1075,7 +1072,8 @@ template <class T, int DIM, int KS, int XS>
 static void fold_t(const DriftDev<T>& D, const MixDev<T>& MX, const void* Fin, const void* Z3, const void* F0, void* Fout,
                    const StageCoef<T>& sc, hipStream_t st) {
     const size_t sh = sizeof(cT<T>) * 3 * XS * 4 * (size_t)(4 * KS * (4 * KS + 1));
-    const int nkg = DIM == 3 ? (D.N + XS - 1) / XS : 1;
+    HPUP_REQUIRE(DIM == 2 || D.N % XS == 0, HPUP_ERR_UNSUPPORTED, "folded drift: whole slab groups");
+    const int nkg = DIM == 3 ? D.N / XS : 1;
     const int64_t ng = D.nrc * nkg;
     auto kern = k_drift_fold<T, DIM, KS, XS>;
     allow_lds((const void*)kern, sh);
