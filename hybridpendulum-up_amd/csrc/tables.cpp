@@ -332,6 +332,10 @@ DriftSpec build_drift_spec_from_arrays(int B, int dim, int N, double L, const do
     auto kap = [&](int p, int j) { return cd(s.kappa[2 * (N * p + j)], s.kappa[2 * (N * p + j) + 1]); };
     // constant real part on every axis -> the kernels' real-circulant path
     s.ramp = s.odd = true;
+    // what the folded kernels drop, an even part of Im kappa or a difference between
+    // axes, is at most the rounding of the arrays: of FP64 transforms (the models'
+    // and the drivers' leave up to 2.4e-15 of the largest entry), or of FP32 entries
+    const double rnd = tol < 1e-6 ? 1e-5 * tol : 1e-3 * tol;
     for (int p = 0; p < dim; p++) {
         double mx = 0.0, dev = 0.0;
         for (int j = 0; j < N; j++) mx = std::max(mx, std::abs(kap(p, j)));
@@ -339,14 +343,14 @@ DriftSpec build_drift_spec_from_arrays(int B, int dim, int N, double L, const do
         s.c0[p] = kap(p, 0).real();
         if (!(dev <= 1e-3 * tol * mx)) s.ramp = false;
         for (int j = 0; j < N; j++)
-            if (!(std::abs(kap(p, j).imag() + kap(p, (N - j) % N).imag()) <= 1e-3 * tol * mx)) s.odd = false;
+            if (!(std::abs(kap(p, j).imag() + kap(p, (N - j) % N).imag()) <= rnd * mx)) s.odd = false;
     }
     if (!s.ramp) s.odd = false;
     s.same12 = s.odd && dim >= 2;
     for (int j = 0; j < N && s.same12; j++) {
         double mx = 0.0;
         for (int a = 0; a < N; a++) mx = std::max(mx, std::abs(kap(0, a)));
-        if (!(std::abs(kap(0, j).imag() - kap(1, j).imag()) <= 1e-3 * tol * mx)) s.same12 = false;
+        if (!(std::abs(kap(0, j).imag() - kap(1, j).imag()) <= rnd * mx)) s.same12 = false;
     }
 
     // ---- OJO: separable gyroscopic coefficients
