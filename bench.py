@@ -35,8 +35,8 @@ MFMA_PEAK_TFLOPS = {"fp32": 157.3, "fp64": 78.6, "bf16x3": 2500.0 / 6}
 MEASURED_TRAFFIC = {
     ("k_drift_fused", "fp32", "RK4"): 5.085e9,   # profiles/k_drift_fused_B15_N30_RK4.md
     ("k_drift_fused", "fp64", "RK4"): 9.451e9,
-    ("k_drift_fold", "fp32", "RK4"): 4.340e9,    # profiles/kernels_by_workload.md
-    ("k_drift_fold", "fp64", "RK4"): 8.098e9,
+    ("k_drift_fold", "fp32", "RK4"): 4.362e9,    # profiles/kernels_by_workload.md
+    ("k_drift_fold", "fp64", "RK4"): 8.108e9,
 }
 
 

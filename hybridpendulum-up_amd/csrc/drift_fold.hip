@@ -26,11 +26,11 @@
 // spend most of their vector instructions on table reads, axis sums, lane
 // permutes and addresses.  The matrices come from the host (OpTab), rounded once.
 //
-// What bounds it: no single unit (B = 15, N = 30, FP32: matrix pipe 24 %, vector
-// units 32 %, tag lookups 60 %, HBM 75 % of a copy's rate).  The six gathered
-// source rows cost 0.28 of 1.37 ms, the streams alone 0.83 ms.  Against
+// What bounds it: no single unit (B = 15, N = 30, FP32: matrix pipe 27 %, vector
+// units 32 %, tag lookups 61 %, HBM 69 % of a copy's rate, waves waiting half of their
+// time).  The six gathered source rows cost 0.28 of 1.37 ms, the streams alone 0.83 ms.  Against
 // k_drift_fused / k_drift_fused_c (ms per launch, average of a step's four):
-//   B = 15, N = 30: FP32 1.63 -> 1.35, FP64 3.00 -> 2.52;  B = 30, N = 20, FP32: 5.54 -> 3.86.
+//   B = 15, N = 30: FP32 1.63 -> 1.35, FP64 3.00 -> 2.53;  B = 30, N = 20, FP32: 5.54 -> 3.85.
 // Tried and not kept: the slab in its natural order with 16-byte loads and the
 // folding in LDS (FP64 N = 30: 2.80, FP32 N = 20: 4.63), mixing tables prefetched
 // through LDS (FP32 1.57), three waves per SIMD in FP64 (spills, 3.08).
@@ -744,15 +744,15 @@ __global__ __launch_bounds__(512, 2) void k_drift_fold64(DriftDev<double> D, Mix
 // and an axis sum; results and the mixing stay in registers, F, V2 and then V1 go through
 // LDS to become operands.  A workgroup is one wave, so nothing waits for another wave:
 // with four waves to a slab and three barriers the same work took two to three times as
-// long (k_drift_fused_c; B = 12, N = 16 FP64 485 -> 186 us, FP32 222 -> 108 us; B = 20, 2-D,
-// N = 14 FP64 142 -> 45 us, FP32 64 -> 26 us; k_drift_fold 1.2-1.7 times k_drift_fused_c's
-// rate at N <= 14).  B = 12, N = 16, FP64: its streams take 120 of the 186 us at a copy's rate,
+// long (k_drift_fused_c; B = 12, N = 16 FP64 485 -> 177 us, FP32 222 -> 98 us; B = 20, 2-D,
+// N = 14 FP64 142 -> 43 us, FP32 64 -> 24 us; k_drift_fold 1.2-1.7 times k_drift_fused_c's
+// rate at N <= 14).  B = 12, N = 16, FP64: its streams take 120 of the 177 us at a copy's rate,
 // the rest is gathered rows and issue at two waves a SIMD (FP32: four).  Two source rows in
 // flight; three measured the same to 4 % slower, six 10-20 % slower in 3-D.
 //
 // ADJ: the adjoint operator, on the transposed tables and circulants of k_drift_fused's: the
 // damping joins V1 and V2, and axis 3 comes whole as D.s3.  B = 10, N = 16, FP64, per launch
-// (k_drift_fused before): 299 -> 96 us; the forward operator 281 -> 97 us.
+// (k_drift_fused before): 299 -> 95 us; the forward operator 281 -> 96 us.
 template <class T, int DIM, bool ADJ>
 __global__ __launch_bounds__(64, fold_waves<T>()) void k_drift_tile(DriftDev<T> D, MixDev<T> MX, const cT<T>* Fin,
                                                                     const cT<T>* __restrict__ Z3, const cT<T>* F0,
