@@ -47,7 +47,7 @@ template <class T> struct DriftDev {
     int ramp;
     int odd;     // ... and the real circulants are odd
     int same12;  // ... and those of axes 1 and 2 are equal
-    int keep;    // FP32: not the folded kernel (see XformDev::keep)
+    int keep;    // FP32: neither the folded nor the one-tile kernel (see XformDev::keep)
     // matrices of the folded kernels (OpTab), null where neither serves the plan
     const T* op;
     T c0[3];
@@ -94,7 +94,7 @@ template <class T> struct MixDev {
     int TS;
     const int32_t* src;   // nrc*TS, -1 padded
     const cT<T>* coef;    // nrc*TS*(dim+2)
-    const int32_t* order; // the nrc rows in the order the folded kernel walks them
+    const int32_t* order; // the nrc rows in the order the folded and one-tile kernels walk them
 };
 
 // bf16x3: circulants as 3xBF16 split products (FP32 storage only)

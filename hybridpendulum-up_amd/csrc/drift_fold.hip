@@ -1,6 +1,7 @@
-// Drift kernels for omega grids of up to 30 points per axis, k_drift_fold (18 to 30
-// points, parity-folded) and k_drift_tile (up to 16), and of 34 to 62 points in the
-// reduced model in FP64, k_drift_fold64 (the forward operator of the pendulum models: real circulants, structured mixing).
+// Drift kernels of the pendulum models (real circulants, structured mixing):
+//   k_drift_fold: omega grids of 18 to 30 points per axis, parity-folded;
+//   k_drift_tile: up to 16 points, one wave per slab, forward and adjoint operator;
+//   k_drift_fold64: 34 to 62 points, the reduced model in FP64, parity-folded.
 //
 // k_drift_fold evaluates the derivative of the (r, k3) slabs it visits with the
 // integrator epilogue, as k_drift_fused does (see drift_mfma.hip for the terms):
